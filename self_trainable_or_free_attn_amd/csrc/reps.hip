@@ -3,7 +3,7 @@
 //
 //   gram_kernel    partial Gram matrices sum_rows q q^T per (head, row split), bf16 MFMA, fp32; written to the
 //                  workspace and reduced in a fixed order (deterministic, unlike the reference's atomics)
-//   chol_kernel    G = Gram * scale^2 / L + 1e-3 * mean(diag) * I; right-looking Cholesky in LDS with the pivot
+//   chol_kernel    G = Gram * scale^2 / L + 1e-3 * mean(diag) * I; right-looking Cholesky by panels with the pivot
 //                  clamped at trace/D * 1e-12; writes the factor transposed (metric_t[e][d] = Lchol[d][e]), bf16
 //   probe_kernel   64 probe queries: scale * mean of the valid q rows of block round(i * (nb - 1) / 63)
 //   kmeans_kernel  one wave per (block, head): probe softmax weights (MFMA), the token Gram matrix X X^T of
@@ -135,64 +135,117 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(float* __restrict__ gr
   g[0] = s;
 }
 
-constexpr int CHOL_T = 1024;                 // threads of the Cholesky workgroup
-constexpr int CHOL_R = HD * HD / CHOL_T;     // rows of one column per thread
+// Cholesky of one head's 128 x 128 matrix, G = Gram * gscale + ridge, right-looking in panels of 16 columns; one
+// workgroup of four waves per head. Wave w holds rows 32 w .. 32 w + 31 as 32 x 32 MFMA accumulator tiles (the lower
+// triangle). Per panel: the tiles that hold it publish it to LDS; waves 0 and 1 factor it, one row per lane with the
+// 16 x 16 diagonal block held in every wave's lanes, so the sixteen column steps exchange values by v_readlane alone,
+// without a barrier; the factored panel goes back through LDS as the operands of the trailing update on
+// v_mfma_f32_32x32x2_f32 (float32 products and sums). What bounds it is the chain of 128 column steps on a few
+// workgroups (one per head): 0.25 us a column here, where one barrier and a round of LDS broadcasts per column over
+// 1024 threads took 0.61 (12 heads: 78 -> 32 us; a 13 770-token, 12-head layer of two branches 798 -> 709 us).
+constexpr int CHOL_T = 256;
+constexpr int CHOL_P = 16;                   // panel columns
+constexpr int CHOL_S = CHOL_P + 4;           // LDS row stride of the published panel: 16-byte reads without conflicts
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
 
 __global__ __launch_bounds__(CHOL_T) void chol_kernel(const float* __restrict__ gram, bf16_t* __restrict__ metric_t,
                                                       int splits, float gscale) {
-  __shared__ float A[HD][HD + 1];
-  __shared__ float red[CHOL_T / 64];
-  const int h = blockIdx.x, tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) float panel_s[HD * CHOL_S];  // the panel's columns, row-major
+  __shared__ __attribute__((aligned(16))) float fac_s[CHOL_P][HD];     // its factor, column-major, 0 above the diagonal
+  __shared__ float red[2];
+  const int h = blockIdx.x, tid = threadIdx.x, l = tid & 63, hi = l >> 5, lq = l & 31;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   // the split partials were summed into split 0 by gram_reduce_kernel
-  for (int i = tid; i < HD * HD; i += CHOL_T) A[i / HD][i % HD] = gram[(size_t)h * splits * HD * HD + i] * gscale;
-  __syncthreads();
-  float dsum = tid < HD ? A[tid][tid] : 0.0f;
-  dsum = wave_sum(dsum);
-  if ((tid & 63) == 0) red[tid >> 6] = dsum;
+  const float* g = gram + (size_t)h * splits * HD * HD;
+  const float diag = tid < HD ? g[tid * (HD + 1)] * gscale : 0.0f;
+  const float dsum = wave_sum(diag);
+  if (l == 0 && wv < 2) red[wv] = dsum;
+  f32x16 c[4];  // [tile column]: rows 32 wv + 8 (r / 4) + 4 hi + r % 4, column 32 ct + lq
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = 32 * wv + 8 * (r / 4) + 4 * hi + (r % 4);
+      c[ct][r] = ct <= wv ? g[row * HD + 32 * ct + lq] * gscale : 0.0f;
+    }
   __syncthreads();
   const float ridge = 1e-3f * (red[0] + red[1]) / (float)HD;
   __syncthreads();
-  if (tid < HD) A[tid][tid] += ridge;
-  __syncthreads();
-  float tr = tid < HD ? A[tid][tid] : 0.0f;
-  tr = wave_sum(tr);
-  if ((tid & 63) == 0) red[tid >> 6] = tr;
+  const float tr = wave_sum(tid < HD ? diag + ridge : 0.0f);
+  if (l == 0 && wv < 2) red[wv] = tr;
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct)
+    if (ct == wv) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (8 * (r / 4) + 4 * hi + (r % 4) == lq) c[ct][r] += ridge;
+    }
   __syncthreads();
   const float eps = (red[0] + red[1]) / (float)HD * 1e-12f;
   bf16_t* mt = metric_t + (size_t)h * HD * HD;
-  // Register-resident right-looking factorisation: thread (cc = tid % 128, part = tid / 128) holds column cc at
-  // rows 16 part .. 16 part + 15 (1024 threads, so a step's own arithmetic is short against its barrier and LDS
-  // round trip). Step j: the owners of column j publish it into column buffer j % 2 (16-byte LDS writes) with its
-  // rows above j as zeros, one barrier, then every thread reads the pivot column with 16-byte
-  // broadcast reads and subtracts the rank-1 update col * (col[cc] / pivot) from its own entries: the zeros leave
-  // the finished rows alone, and the columns left of j (already published) are never read again, so no entry
-  // needs a mask. (Two buffers: step j+1 writes the other one while step j's readers may still be reading.)
-  const int cc = tid & (HD - 1), rb = CHOL_R * (tid >> 7);
-  float a[CHOL_R];
+
+#pragma unroll  // (rolled, with run-time tile columns: 36 us against 32)
+  for (int p = 0; p < HD / CHOL_P; ++p) {
+    const int c0 = CHOL_P * p;
+    // publish columns c0 .. c0 + 15 of this wave's rows (rows above the panel hold finished values: masked below)
 #pragma unroll
-  for (int i = 0; i < CHOL_R; ++i) a[i] = A[rb + i][cc];
-  __syncthreads();
-  float* colbuf = &A[0][0];  // the matrix now lives in registers; reuse the LDS as two column buffers
-  for (int j = 0; j < HD; ++j) {
-    float* cb = colbuf + (j & 1) * HD;
-    if (cc == j) {
+    for (int ct = 0; ct < 4; ++ct)
+      if (ct == p / 2 && wv >= ct && (lq / CHOL_P) == (p & 1)) {
 #pragma unroll
-      for (int q4 = 0; q4 < CHOL_R / 4; ++q4) {
-        f32x4 c4;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) c4[k] = rb + 4 * q4 + k >= j ? a[4 * q4 + k] : 0.0f;
-        *reinterpret_cast<f32x4*>(cb + rb + 4 * q4) = c4;
+        for (int r = 0; r < 16; ++r)
+          panel_s[(32 * wv + 8 * (r / 4) + 4 * hi + (r % 4)) * CHOL_S + (lq & (CHOL_P - 1))] = c[ct][r];
       }
+    __syncthreads();
+    if (wv < 2) {
+      const int row = tid;
+      float x[CHOL_P], d[CHOL_P];  // this lane's row of the panel; row c0 + lane % 16 of its diagonal block
+      const bool active = 64 * wv + 63 >= c0;  // (wave-uniform) some row of this wave is at or below the panel
+      if (active) {
+#pragma unroll
+        for (int i = 0; i < CHOL_P / 4; ++i) {
+          const f32x4 xv = *reinterpret_cast<const f32x4*>(&panel_s[max(row, c0) * CHOL_S + 4 * i]);
+          const f32x4 dv = *reinterpret_cast<const f32x4*>(&panel_s[(c0 + (l & (CHOL_P - 1))) * CHOL_S + 4 * i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[4 * i + e] = xv[e];
+            d[4 * i + e] = dv[e];
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < CHOL_P; ++j) {
+          // 1 / sqrt(pivot), hardware rsq (1 ulp); the pivot is clamped
+          const float inv = __builtin_amdgcn_rsqf(fmaxf(lane_value(d[j], j), eps));
+          d[j] *= inv;
+          x[j] *= inv;
+#pragma unroll
+          for (int k = j + 1; k < CHOL_P; ++k) {
+            const float lkj = lane_value(d[j], k);
+            d[k] = fmaf(-d[j], lkj, d[k]);
+            x[k] = fmaf(-x[j], lkj, x[k]);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < CHOL_P; ++j) fac_s[j][row] = active && row >= c0 + j ? x[j] : 0.0f;
     }
     __syncthreads();
-    const float inv = __builtin_amdgcn_rsqf(fmaxf(cb[j], eps));  // 1 / sqrt(pivot), hardware rsq (1 ulp)
-    const float sc = cb[cc] * (inv * inv);
-    if (tid < HD) mt[j * HD + tid] = f2bf(cb[tid] * inv);  // metric_t[j][d] = Lchol[d][j] (zero above j)
+    {  // metric_t[j][d] = Lchol[d][j] (zero above j): eight entries per thread
+      const int j = tid >> 4, d8 = (tid & 15) * 8;
+      *reinterpret_cast<bf16x8*>(mt + (c0 + j) * HD + d8) = pack8(&fac_s[j][d8]);
+    }
+    // trailing update of the columns right of the panel (rows above the panel meet zeros)
+    if (c0 + CHOL_P < HD && 32 * wv + 31 >= c0 + CHOL_P) {
 #pragma unroll
-    for (int q4 = 0; q4 < CHOL_R / 4; ++q4) {
-      const f32x4 c4 = *reinterpret_cast<const f32x4*>(cb + rb + 4 * q4);
+      for (int ks = 0; ks < CHOL_P / 2; ++ks) {
+        const float fa = -fac_s[2 * ks + hi][32 * wv + lq];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) a[4 * q4 + k] = fmaf(-c4[k], sc, a[4 * q4 + k]);
+        for (int ct = 0; ct < 4; ++ct)
+          if (32 * ct + 31 >= c0 + CHOL_P && ct <= wv)
+            c[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa, fac_s[2 * ks + hi][32 * ct + lq], c[ct], 0, 0, 0);
+      }
     }
   }
 }
