@@ -94,12 +94,16 @@ __device__ __forceinline__ void select_row_lds(const unsigned short* keys, int N
   }
 }
 
-// grid (cdiv(NB, SR), bh_count), 256 threads, SR = 32 rows per workgroup (NB <= 2048, the keys of a row in
-// registers) or 8 (WIDE, NB <= 8192: the S tile of 32 rows is computed by each of its four workgroups, which keep
-// their 8 rows; the keys are read from LDS in every step). K < 0: scores only.
-template <bool FROM_SCORES, bool WIDE>
+// grid (cdiv(NB, SR), bh_count), 256 threads, SR = 32 or 8 rows per workgroup: at 8 the S tile of 32 rows is computed
+// by each of its four workgroups, which keep their 8 rows. NCH > 0: a row has at most NCH chunks of 64 columns, whose
+// keys sit in NCH registers during the search (NCH = 32: NB <= 2048). NCH = 0: the keys are read from LDS in every
+// step (SR = 8, NB <= 8192). K < 0: scores only.
+// A row costs its wave 16 dependent rounds of NCH compares and ballots, so NCH follows NB (one unrolled search over
+// 32 chunk slots with a test per slot took 51 us at NB = 64 and 98 us at NB = 480, 24 heads) and a wave takes as few
+// rows as the grid allows (rows_launch).
+template <bool FROM_SCORES, int NCH, int SR>
 __global__ __launch_bounds__(256) void rows_select_kernel(RowsArgs a) {
-  constexpr int SR = WIDE ? WIDE_ROWS : ROWS;
+  constexpr bool WIDE = NCH == 0;
   extern __shared__ __attribute__((aligned(16))) unsigned short keys_s[];  // [SR][NBp]
   const int strip = blockIdx.x, bhl = blockIdx.y;
   const int NB = a.NB, NBp = (NB + 63) & ~63;
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(256) void rows_select_kernel(RowsArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int rr = t0 + 8 * (r / 4) + 4 * hi + (r % 4) - r0;  // row within this workgroup's strip
-        if (WIDE && (rr < 0 || rr >= SR)) continue;
+        if (SR < ROWS && (rr < 0 || rr >= SR)) continue;
         const e16_t s = f2e(mul_rn(e2f(f2e(acc[r])), a.scale));
         const bool in = r0 + rr < NB && col < NB;
         keys_s[rr * NBp + col] = in ? (unsigned short)key16(s) : 0;
@@ -156,44 +160,44 @@ __global__ __launch_bounds__(256) void rows_select_kernel(RowsArgs a) {
                      a.selbits + ((size_t)bhl * (size_t)((NB + 31) & ~31) + row) * a.W, a.W);
       continue;
     }
-    unsigned kv[MAX_NB / 64];
+    if constexpr (!WIDE) {
+      unsigned kv[NCH];  // (columns past NB have key 0: they never reach a threshold t >= 1)
 #pragma unroll
-    for (int c = 0; c < MAX_NB / 64; ++c) kv[c] = c < nchunk ? keys_s[rr * NBp + 64 * c + l] : 0u;
-    // T = the largest t with #(key >= t) >= K; keys of padding columns are 0 and never reach t >= 1
-    unsigned T = 0x10000u;
-    if (K > 0) {
-      unsigned lo = 0, hi2 = 0x10000u;
-      while (hi2 - lo > 1) {
-        const unsigned mid = (lo + hi2) >> 1;
-        int cnt = 0;
+      for (int c = 0; c < NCH; ++c) kv[c] = c < nchunk ? keys_s[rr * NBp + 64 * c + l] : 0u;
+      // T = the largest t with #(key >= t) >= K
+      unsigned T = 0x10000u;
+      if (K > 0) {
+        unsigned lo = 0, hi2 = 0x10000u;
+        while (hi2 - lo > 1) {
+          const unsigned mid = (lo + hi2) >> 1;
+          int cnt = 0;
 #pragma unroll
-        for (int c = 0; c < MAX_NB / 64; ++c)
-          if (c < nchunk) cnt += __popcll(__builtin_amdgcn_ballot_w64(kv[c] >= mid));
-        if (cnt >= K) lo = mid; else hi2 = mid;
+          for (int c = 0; c < NCH; ++c) cnt += __popcll(__builtin_amdgcn_ballot_w64(kv[c] >= mid));
+          if (cnt >= K) lo = mid; else hi2 = mid;
+        }
+        T = lo;
       }
-      T = lo;
-    }
-    int above = 0;
+      int above = 0;
 #pragma unroll
-    for (int c = 0; c < MAX_NB / 64; ++c)
-      if (c < nchunk) above += __popcll(__builtin_amdgcn_ballot_w64(kv[c] > T && 64 * c + l < NB));
-    const int take_eq = K - above;  // T-equal entries to take, smallest column first
-    int eq_run = 0, sel_run = 0;
-    int* out = a.q2k_idx + base;
-    unsigned* bits = a.selbits + ((size_t)bhl * (size_t)((NB + 31) & ~31) + row) * a.W;
+      for (int c = 0; c < NCH; ++c) above += __popcll(__builtin_amdgcn_ballot_w64(kv[c] > T && 64 * c + l < NB));
+      const int take_eq = K - above;  // T-equal entries to take, smallest column first
+      int eq_run = 0, sel_run = 0;
+      int* out = a.q2k_idx + base;
+      unsigned* bits = a.selbits + ((size_t)bhl * (size_t)((NB + 31) & ~31) + row) * a.W;
 #pragma unroll
-    for (int c = 0; c < MAX_NB / 64; ++c) {
-      if (c >= nchunk) continue;
-      const int j = 64 * c + l;
-      const bool in = j < NB;
-      const bool eq = in && kv[c] == T;
-      const unsigned long long eqb = __builtin_amdgcn_ballot_w64(eq);
-      const bool sel = in && (kv[c] > T || (eq && eq_run + __popcll(eqb & lanes_below()) < take_eq));
-      const unsigned long long sb = __builtin_amdgcn_ballot_w64(sel);
-      if (sel) out[sel_run + __popcll(sb & lanes_below())] = j;
-      eq_run += __popcll(eqb);
-      sel_run += __popcll(sb);
-      if (l < 2 && 2 * c + l < a.W) bits[2 * c + l] = (unsigned)(sb >> (32 * l));
+      for (int c = 0; c < NCH; ++c) {
+        if (c >= nchunk) continue;
+        const int j = 64 * c + l;
+        const bool in = j < NB;
+        const bool eq = in && kv[c] == T;
+        const unsigned long long eqb = __builtin_amdgcn_ballot_w64(eq);
+        const bool sel = in && (kv[c] > T || (eq && eq_run + __popcll(eqb & lanes_below()) < take_eq));
+        const unsigned long long sb = __builtin_amdgcn_ballot_w64(sel);
+        if (sel) out[sel_run + __popcll(sb & lanes_below())] = j;
+        eq_run += __popcll(eqb);
+        sel_run += __popcll(sb);
+        if (l < 2 && 2 * c + l < a.W) bits[2 * c + l] = (unsigned)(sb >> (32 * l));
+      }
     }
   }
 }
@@ -725,6 +729,33 @@ static int invert(const TopkCarve& c, int* k2q_ptr, int* k2q_idx, int NB, int bh
   return ES_OK;
 }
 
+template <bool FROM_SCORES, int NCH>
+static void rows_launch_n(const RowsArgs& a, int bh_count, bool narrow, hipStream_t stream) {
+  const int SR = narrow || NCH == 0 ? WIDE_ROWS : ROWS;
+  const size_t lds = (size_t)SR * ((a.NB + 63) & ~63) * 2;  // <= 128 KB
+  const dim3 grid((a.NB + SR - 1) / SR, bh_count);
+  if (SR == WIDE_ROWS)
+    hipLaunchKernelGGL((rows_select_kernel<FROM_SCORES, NCH, WIDE_ROWS>), grid, dim3(256), lds, stream, a);
+  else if constexpr (NCH != 0)
+    hipLaunchKernelGGL((rows_select_kernel<FROM_SCORES, NCH, ROWS>), grid, dim3(256), lds, stream, a);
+}
+
+// The search keeps the smallest power of two of chunk registers that holds a row. Strips of 8 rows (a wave searches
+// two rows instead of eight, the S tile is computed four times) while the grid of 32-row strips is under eight
+// workgroups per CU: below that a strip's serial searches are what the launch waits for, above it the repeated
+// products are (routing NB = 480, 24 heads: 98 us in 360 strips of 32 rows, 52 in strips of 8; NB = 64, 2 heads: 51 -> 8 us).
+template <bool FROM_SCORES>
+static void rows_launch(const RowsArgs& a, int bh_count, hipStream_t stream) {
+  const int nchunk = (a.NB + 63) / 64;
+  const bool narrow = (long long)((a.NB + ROWS - 1) / ROWS) * bh_count < 2048;
+  if (nchunk <= 2) rows_launch_n<FROM_SCORES, 2>(a, bh_count, narrow, stream);
+  else if (nchunk <= 4) rows_launch_n<FROM_SCORES, 4>(a, bh_count, narrow, stream);
+  else if (nchunk <= 8) rows_launch_n<FROM_SCORES, 8>(a, bh_count, narrow, stream);
+  else if (nchunk <= 16) rows_launch_n<FROM_SCORES, 16>(a, bh_count, narrow, stream);
+  else if (a.NB <= MAX_NB) rows_launch_n<FROM_SCORES, 32>(a, bh_count, narrow, stream);
+  else rows_launch_n<FROM_SCORES, 0>(a, bh_count, narrow, stream);
+}
+
 static int rows_common(const void* qc, const void* kc, const void* scores_in, void* scores_out, int NB, int NBc_pad,
                        int bh0, int bh_count, int K, int* q2k_ptr, int* q2k_idx, int* k2q_ptr, int* k2q_idx,
                        void* workspace, size_t workspace_bytes, int D, hipStream_t stream, const char* what) {
@@ -740,16 +771,9 @@ static int rows_common(const void* qc, const void* kc, const void* scores_in, vo
   a.bh0 = bh0;
   a.W = (NB + 31) / 32;
   a.scale = 1.0f / sqrtf((float)D);  // D: the logical head dimension (64 or 128)
-  const bool wide = NB > MAX_NB;
-  const int SR = wide ? WIDE_ROWS : ROWS;
-  const size_t lds = (size_t)SR * ((NB + 63) & ~63) * 2;  // <= 128 KB either way
-  const dim3 grid((NB + SR - 1) / SR, bh_count);
   if (K < 0) {  // scores only
     a.K = -1;
-    if (wide)
-      hipLaunchKernelGGL((rows_select_kernel<false, true>), grid, dim3(256), lds, stream, a);
-    else
-      hipLaunchKernelGGL((rows_select_kernel<false, false>), grid, dim3(256), lds, stream, a);
+    rows_launch<false>(a, bh_count, stream);
     return check_launch(what);
   }
   ES_REQUIRE(q2k_ptr && k2q_ptr && workspace, ES_ERR_INVALID, "VSA: null tensor pointer");
@@ -769,14 +793,10 @@ static int rows_common(const void* qc, const void* kc, const void* scores_in, vo
                        NB, W, bh_count);
   hipLaunchKernelGGL(fill_base_kernel, dim3((bh_count + 255) / 256), dim3(256), 0, stream, c.base,
                      (const TopkState*)nullptr, (long long)NB * K, (const int*)nullptr, NB, bh0, bh_count);
-  if (scores_in != nullptr && wide)
-    hipLaunchKernelGGL((rows_select_kernel<true, true>), grid, dim3(256), lds, stream, a);
-  else if (scores_in != nullptr)
-    hipLaunchKernelGGL((rows_select_kernel<true, false>), grid, dim3(256), lds, stream, a);
-  else if (wide)
-    hipLaunchKernelGGL((rows_select_kernel<false, true>), grid, dim3(256), lds, stream, a);
+  if (scores_in != nullptr)
+    rows_launch<true>(a, bh_count, stream);
   else
-    hipLaunchKernelGGL((rows_select_kernel<false, false>), grid, dim3(256), lds, stream, a);
+    rows_launch<false>(a, bh_count, stream);
   invert(c, k2q_ptr, k2q_idx, NB, bh0, bh_count, stream);
   return check_launch(what);
 }

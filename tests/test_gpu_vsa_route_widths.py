@@ -1,0 +1,43 @@
+"""The per-row block selection at the edges of its register layouts (2, 4, 8, 16, 32 chunks of 64 columns) and of its
+strip rule (8 rows per workgroup under 2048 strips of 32, else 32), bit for bit against the oracle. Pooled rows hold
+small integers, so every dot product is exact, scores tie often and the order of ties is tested too."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import vsa_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("NB,heads,K", [(1, 2, 1), (63, 2, 5), (64, 2, 64), (65, 2, 16), (128, 3, 0), (129, 2, 40),
+                                        (256, 2, 17), (257, 2, 100), (512, 1, 60), (513, 1, 60), (1024, 1, 200),
+                                        (1025, 1, 1), (2048, 1, 333),
+                                        (33, 1025, 7), (130, 411, 20), (200, 300, 50), (300, 205, 31)])
+@pytest.mark.parametrize("given", [False, True])
+def test_row_selection_widths(dev, NB, heads, K, given):
+    from self_trainable_or_free_attn_amd.vsa import _C
+    print("rows", NB, heads, K, given, flush=True)
+    g = torch.Generator().manual_seed(NB * 7 + heads)
+    pad = (NB + 63) // 64 * 64
+    qc, kc = (torch.zeros(1, heads, pad, 128) for _ in range(2))
+    for x in (qc, kc):
+        x[:, :, :NB, :16] = torch.randint(-2, 3, (1, heads, NB, 16), generator=g).float()
+    qd, kd = qc.bfloat16().to(dev), kc.bfloat16().to(dev)
+    if given:
+        scores = _C.block_scores(qd, kd, NB)
+        i32 = dict(device=dev, dtype=torch.int32)
+        out = [torch.full((1, heads, NB + 1), -1, **i32), torch.full((heads * NB * K,), -1, **i32)]
+        out += [torch.full((1, heads, NB + 1), -1, **i32), torch.full((heads * NB * K,), -1, **i32)]
+        _C.row_topk_into(scores, K, 0, *out)
+    else:
+        out = _C.route_rows(qd, kd, NB, K)
+    qp, qi, kp, ki = (x.cpu().numpy() for x in out)
+    for h in sorted({0, heads // 2, heads - 1}):
+        s = ref.block_scores(qc[:, h:h + 1, :NB].numpy(), kc[:, h:h + 1, :NB].numpy())
+        mask = ref.row_topk_mask(s, K).reshape(NB, NB)
+        base = h * NB * K
+        assert np.array_equal(qp[0, h], base + np.arange(NB + 1) * K)
+        assert np.array_equal(qi[base:base + NB * K], np.nonzero(mask)[1])
+        assert np.array_equal(kp[0, h], base + np.concatenate([[0], np.cumsum(mask.sum(0))]))
+        assert np.array_equal(ki[base:base + NB * K], np.nonzero(mask.T)[1])
