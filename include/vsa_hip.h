@@ -35,7 +35,7 @@ extern "C" {
 /* ---------------------------------------------------------------- pooling and fusion */
 
 /* Router group means of R tokens (qr / kr / vr, each may be NULL; empty groups are 0) and whole-block means
- * (qc / kc / vc) over the valid tokens of each block. Padding rows of the outputs are not written.
+ * (qc / kc / vc) over the valid tokens of each block. Padding rows of the outputs are written as zeros.
  * Replaces csrc/vsa/vsa2_api.cpp:73-97 pool_fwd (kernel csrc/vsa/router/pool.cu:16-51). */
 int vsa_pool(const void* q, const void* k, const void* v, const int* blk_cnt, void* qr, void* kr, void* vr,
              void* qc, void* kc, void* vc, int BH, int L, int D, int R, hipStream_t stream);
@@ -47,7 +47,8 @@ int vsa_fuse_fwd(const void* of, const void* oc, const void* gate, void* o, cons
                  int D, int NBc_pad, int gate_mode, int gate_act, hipStream_t stream);
 
 /* dO_f = valid ? dO : 0 (dout_f may be NULL), delta_f = rowsum(dO_f * O_f) [BH, L] fp32,
- * dO_c[blk] = sum over valid rows of act(gate) * dO (bf16), delta_c = <dO_c, O_c> [BH, NBc_pad] fp32,
+ * dO_c[blk] = sum over valid rows of act(gate) * dO (bf16), delta_c = <dO_c, O_c> [BH, NBc_pad] fp32 (both 0 on
+ * the rows past NB),
  * dgate = act'(gate) * <dO, O_c> (mode 1, [BH, L]) or act'(gate) * dO * O_c (mode 2), 0 on padding rows.
  * Replaces csrc/vsa/vsa2_api.cpp fuse_bwd (kernel csrc/vsa/fuse.cu:82-166). */
 int vsa_fuse_bwd(const void* dout, const void* of, const void* oc, const void* gate, void* dout_f, float* delta_f,

@@ -114,10 +114,10 @@ def pool_fwd(q, k, v, blk_cnt, R):
     NB = L // BLOCK
     _check(blk_cnt.numel() == NB, "blk_cnt must have L/64 entries")
     G = BLOCK // R
-    qr = torch.zeros(B, H, _ceil64(NB * G), HD, device=q.device, dtype=q.dtype)
-    kr = torch.zeros_like(qr)
-    qc = torch.zeros(B, H, _ceil64(NB), HD, device=q.device, dtype=q.dtype)
-    kc, vc = torch.zeros_like(qc), torch.zeros_like(qc)
+    qr = torch.empty(B, H, _ceil64(NB * G), HD, device=q.device, dtype=q.dtype)
+    kr = torch.empty_like(qr)
+    qc = torch.empty(B, H, _ceil64(NB), HD, device=q.device, dtype=q.dtype)
+    kc, vc = torch.empty_like(qc), torch.empty_like(qc)
     _call("vsa_pool", _wide(q), _wide(k), _wide(v), blk_cnt, qr, kr, None, qc, kc, vc, B * H, L, D, int(R))
     return [_narrow(t, D) for t in (qr, kr, qc, kc, vc)]
 
@@ -148,8 +148,8 @@ def fuse_bwd(dout, of, oc, gate, blk_cnt, gate_act, write_dout_f=True):
     mode = 0 if gate is None else (1 if gate.dim() == 3 else 2)
     dout_f = torch.empty(B, H, L, HD, device=dout.device, dtype=dout.dtype) if write_dout_f else None
     delta_f = torch.empty(B, H, L, device=dout.device, dtype=torch.float32)
-    dout_c = torch.zeros(B, H, oc.shape[2], HD, device=dout.device, dtype=dout.dtype)
-    delta_c = torch.zeros(B, H, oc.shape[2], device=dout.device, dtype=torch.float32)
+    dout_c = torch.empty(B, H, oc.shape[2], HD, device=dout.device, dtype=dout.dtype)
+    delta_c = torch.empty(B, H, oc.shape[2], device=dout.device, dtype=torch.float32)
     gate_w = _wide(gate) if mode == 2 else gate
     dgate = torch.empty_like(gate_w) if gate is not None else None
     _call("vsa_fuse_bwd", _wide(dout), _wide(of), _wide(oc), gate_w, dout_f, delta_f, dout_c,
@@ -458,10 +458,10 @@ def rep_build(k, v, blk_cnt, mid_reps):
     _tokens(v, "v")
     B, H, L, D = k.shape
     NB, RM = L // BLOCK, int(mid_reps)
-    k_mid = torch.zeros(B, H, _ceil64(NB * RM), HD, device=k.device, dtype=k.dtype)
-    v_mid = torch.zeros_like(k_mid)
-    k_tail = torch.zeros(B, H, _ceil64(NB), HD, device=k.device, dtype=k.dtype)
-    v_tail = torch.zeros_like(k_tail)
+    k_mid = torch.empty(B, H, _ceil64(NB * RM), HD, device=k.device, dtype=k.dtype)
+    v_mid = torch.empty_like(k_mid)
+    k_tail = torch.empty(B, H, _ceil64(NB), HD, device=k.device, dtype=k.dtype)
+    v_tail = torch.empty_like(k_tail)
     lc_mid = torch.empty(NB * RM, device=k.device, dtype=torch.float32)
     lc_tail = torch.empty(NB, device=k.device, dtype=torch.float32)
     _call("vsa_rep_build", _wide(k), _wide(v), blk_cnt, k_mid, v_mid, lc_mid, k_tail, v_tail, lc_tail, B * H, L, D,
