@@ -249,10 +249,7 @@ __global__ __launch_bounds__(256, 2) void vsa_fwd_kernel(VsaFwdArgs a) {
 //   KV owner (dK, dV; k2q lists): one workgroup per (kv block, head), 4 waves = 2 key halves x 2 query halves of
 //     each staged query block. S = Q K^T and dP = dO V^T come out with keys on lanes, so P and dS are directly the
 //     B operands of dV^T += dO^T P and dK^T += Q^T dS (dO^T / Q^T through transposed LDS reads). K and V stay in
-//     registers; Q, dO, lse and delta of each listed query block stream through LDS. It runs as two passes, dV
-//     (S, dV) then dK (S, dP, dK): 5 products per pair instead of 4, but each pass holds one 128-register
-//     accumulator set instead of two, so two waves share a SIMD (one pass with both: 5.68 ms at C2, the two
-//     passes 5.14 ms, bit-identical outputs).
+//     registers; Q, dO, lse and delta of each listed query block stream through LDS. 4 products per pair.
 //   Q owner (dQ; q2k lists): the forward's layout. S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T with K^T through
 //     transposed LDS reads. 3 products per pair; dQ is deterministic (no atomics).
 // The two partial accumulators of a workgroup (query halves, or key halves) are summed once at the end in LDS.
@@ -298,23 +295,27 @@ __device__ __forceinline__ bool owner_of(const VsaBwdArgs& a, int& blk, int& bh,
 // lse (natural) -> log2 domain, +inf for rows that must get P = 0
 __device__ __forceinline__ float lse_to_log2(float lse) { return lse == -INFINITY ? INFINITY : lse * LOG2E; }
 
-// The KV-owner backward: one 256-thread workgroup per (kv block, head), two per CU. Wave (role, key half): a dV
-// wave computes S and P of its 32 keys against the chunk's 64 query rows and dV += P^T dO; a dK wave of the same
-// keys computes dP = dO V^T (V in registers), dS from the dV wave's P (handed over as bf16 / fp16 operands through
-// LDS) and dK += dS^T Q. Each query block's Q / dO is staged once for both roles: four products per pair, 32
-// matrix instructions per wave and chunk, and every wave's accumulators hold the full sums of its keys.
+// The KV-owner backward: one 256-thread workgroup per (kv block, head), two per CU. Wave (key half, query half) owns a
+// 32 x 32 tile of every staged query block and runs all four products on it: S = Q K^T and P, dV += P^T dO, dP = dO V^T
+// and dS, dK += dS^T Q, with K and V of its keys in registers; 32 matrix instructions per wave and chunk and one
+// barrier. The two query halves' sums are added once at the end. Both accumulator sets and both operand rows need 192 of
+// the 256 registers that two waves per SIMD leave; what else is loop-invariant (LDS and transfer offsets) is therefore
+// rebuilt from one register each by XOR, and lse and delta go to LDS without passing through registers. What bounds it
+// is each wave's chain of products and exponentials per chunk, as in the forward. Against a dV wave and a dK wave per
+// key half that handed P over through LDS with a second barrier: 4256 -> 3625 us at 480 blocks, 24 heads, top 60
+// (666 -> 800 TFLOP/s), 604 -> 540 at 240 blocks, 12 heads, top 24; at D = 64, 3187 -> 2400.
 template <bool TASKS, int DH>
 __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   constexpr int NKS = DH / 16, NDB = DH / 32;
   __shared__ __attribute__((aligned(16))) char qd_s[2][2][BK * 256];  // [buffer][Q | dO]
   __shared__ __attribute__((aligned(16))) float st_s[2][2][BK];       // [buffer][lse2 (+inf: P = 0) | delta]
-  __shared__ ev8 p_s[2][4][64];  // [key half][query half x (first | second 8 rows of a lane)][lane]: the dV waves' P
+  __shared__ float lse_s[BK];                                         // the next block's lse as stored
   int kb, bh, beg, end, slot;
   if (!owner_of<TASKS>(a, kb, bh, beg, end, slot)) return;
   const int nc = end - beg;
   const int tid = threadIdx.x, l = tid & 63, hi = l >> 5, lq = l & 31;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int role = wv >> 1, kh = wv & 1;  // role 0: dV, 1: dK (wave-uniform)
+  const int qh = wv >> 1, kh = wv & 1;
   const int key = 32 * kh + lq;
   const int kcnt = sload(a.blk_cnt + kb);
   const bool kvalid = key < kcnt;
@@ -323,178 +324,169 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   const unsigned head_bytes = (unsigned)((size_t)a.L * HD * 2);
   const srd_t rq = make_srd(a.q + head * HD, head_bytes);
   const srd_t rd = make_srd(a.dout + head * HD, head_bytes);
-  unsigned ld_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int P = (wv * 4 + i) * 64 + l, R = P >> 4, g = (P & 15) ^ swz(R);
-    ld_off[i] = g < DH / 8 ? (unsigned)R * 256 + (unsigned)(g * 16) : 0x80000000u;
+  // transfer r of a wave moves rows 16 wv + 4 r + l / 16: this lane's source offset is ld_off ^ 16 r plus 1024 r
+  unsigned ld_off;
+  {
+    const int g = (l & 15) ^ ((l >> 4) << 2);
+    ld_off = g < DH / 8 ? (unsigned)(wv * 16 + (l >> 4)) * 256 + (unsigned)(g * 16) : 0x80000000u;
   }
-  ev8 kvreg[8];  // this lane's key row: K (dV wave, for S) or V (dK wave, for dP)
+  ev8 kreg[8], vreg[8];  // this lane's key row
   {
     const size_t off = (head + (size_t)kb * BK + key) * HD + 8 * hi;
-    const e16_t* src = (role ? a.v : a.k) + off;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) kvreg[ks] = *reinterpret_cast<const ev8*>(src + 16 * ks);
+    for (int ks = 0; ks < NKS; ++ks) {
+      kreg[ks] = *reinterpret_cast<const ev8*>(a.k + off + 16 * ks);
+      vreg[ks] = *reinterpret_cast<const ev8*>(a.v + off + 16 * ks);
+    }
   }
-  // stage query block i (Q, dO: 16 rows of each per wave); wave 0 returns lane l's lse2 / delta of row i * 64 + l
-  auto issue = [&](int i, int sb, float& ls, float& dl) {
+  // stage query block i: Q and dO (16 rows of each per wave), and, wave 0, its 64 delta and raw lse values, which
+  // `stats` turns into what the exponent subtracts once the transfers have landed
+  const srd_t rl = make_srd(a.lse + head, (unsigned)a.L * 4u);
+  const srd_t re = make_srd(a.delta + head, (unsigned)a.L * 4u);
+  auto issue = [&](int i, int sb) {
     const unsigned soff = (unsigned)i * (BK * 256);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      dma16(rq, qd_s[sb][0] + wv * 4096 + r * 1024, ld_off[r], soff);
-      dma16(rd, qd_s[sb][1] + wv * 4096 + r * 1024, ld_off[r], soff);
+      dma16(rq, qd_s[sb][0] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + 1024u * r);
+      dma16(rd, qd_s[sb][1] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + 1024u * r);
     }
     if (wv == 0) {
-      const size_t t = head + (size_t)i * BK + l;
-      ls = lse_to_log2(a.lse[t]);
-      dl = a.delta[t];
+      dma4(rl, lse_s, 4u * l, (unsigned)i * (BK * 4));
+      dma4(re, st_s[sb][1], 4u * l, (unsigned)i * (BK * 4));
     }
   };
-  // LDS offsets within a query half (32 rows, 8 KB); the second half adds 8192
-  int aoff[8];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) aoff[ks] = tile_off(lq, 2 * ks + hi);
-  int toff[2][4];
+  auto stats = [&](int sb) {  // wave 0, after dma_wait()
+    st_s[sb][0][l] = lse_to_log2(lse_s[l]);
+  };
+  // LDS offsets of this wave's query half: row reads of k-step ks at aoff ^ 32 ks, transposed reads of channel block
+  // db at toff ^ 64 db (exact: the swizzle is an XOR of the 16-byte chunk), so two registers hold what would be
+  // sixteen; the kernel fits its two accumulator sets and both operand rows in 256 registers that way
+  int aoff = qh * 8192 + tile_off(lq, hi);
+  int toff0, toff1;
   {
     const int g1 = (l >> 4) & 1, sub = (l & 1) * 8, rowA = 4 * hi + ((l & 15) >> 2);
-#pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      toff[0][db] = tile_off(rowA, 4 * db + 2 * g1 + ((l & 3) >> 1)) + sub;
-      toff[1][db] = tile_off(rowA + 8, 4 * db + 2 * g1 + ((l & 3) >> 1)) + sub;
-    }
+    toff0 = qh * 8192 + tile_off(rowA, 2 * g1 + ((l & 3) >> 1)) + sub;
+    toff1 = qh * 8192 + tile_off(rowA + 8, 2 * g1 + ((l & 3) >> 1)) + sub;
   }
-  f32x16 acc[4];  // dV (role 0) or dK (role 1) of this lane's key
+  f32x16 acc_v[4], acc_k[4];  // this lane's key: dV and dK over this query half
 #pragma unroll
-  for (int db = 0; db < 4; ++db) acc[db] = f32x16{};
+  for (int db = 0; db < 4; ++db) acc_v[db] = acc_k[db] = f32x16{};
 
-  float ls = 0.0f, dl = 0.0f;
   int inext = nc > 1 ? sload(a.col_idx + beg + 1) : 0;
   if (nc > 0) {
-    issue(sload(a.col_idx + beg), 0, ls, dl);
+    issue(sload(a.col_idx + beg), 0);
     dma_wait();
-    if (wv == 0) {
-      st_s[0][0][l] = ls;
-      st_s[0][1][l] = dl;
-    }
+    if (wv == 0) stats(0);
   }
   dma_wait();
   __syncthreads();
   // masked key columns: every row's lse2 becomes +inf for this lane, so P = 2^(s - inf) = 0 without a branch
   const float kmask = kvalid ? 0.0f : INFINITY;
-  ev8* pex = p_s[kh][0];
   for (int j = 0; j < nc; ++j) {
     const int sb = j & 1;
     int inn = 0;
     if (j + 1 < nc) {
-      issue(inext, sb ^ 1, ls, dl);
+      issue(inext, sb ^ 1);
       if (j + 2 < nc) inn = sload(a.col_idx + beg + j + 2);
     }
+    asm volatile("" : "+v"(aoff), "+v"(toff0), "+v"(toff1), "+v"(ld_off));  // (keeps the offsets from being hoisted)
     const char* qt = qd_s[sb][0];
     const char* dt = qd_s[sb][1];
-    f32x16 dp[2];  // dK wave: dP of each query half
-    if (role == 0) {
+    auto product = [&](const char* xt, const ev8& xa, const ev8& xb, f32x16 (&acc)[4]) {  // acc += xt^T [xa | xb]
 #pragma unroll
-      for (int qh = 0; qh < 2; ++qh) {
-        f32x16 s = {};
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) s = emfma(elds16(qt, qh * 8192 + aoff[ks]), kvreg[ks], s);
-        float p[16];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 l4 = *reinterpret_cast<const f32x4*>(&st_s[sb][0][32 * qh + 8 * g + 4 * hi]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) p[4 * g + e] = exp2f_fast(fmaf(s[4 * g + e], a.scale_log2, -(l4[e] + kmask)));
-        }
-        const ev8 pa = epack8(&p[0]), pb = epack8(&p[8]);
-        pex[(2 * qh) * 64 + l] = pa;
-        pex[(2 * qh + 1) * 64 + l] = pb;
-        // dV += P^T dO (needs nothing from the dK wave, so it runs before the hand-over barrier)
-        const char* xt = dt + qh * 8192;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          acc[db] = emfma(ecat_tr(lds_read_tr(xt, toff[0][db]), lds_read_tr(xt, toff[1][db])), pa, acc[db]);
-          acc[db] = emfma(ecat_tr(lds_read_tr(xt + 4096, toff[0][db]), lds_read_tr(xt + 4096, toff[1][db])), pb, acc[db]);
-        }
+      for (int db = 0; db < NDB; ++db) {
+        const int t0 = toff0 ^ (64 * db), t1 = toff1 ^ (64 * db);
+        acc[db] = emfma(ecat_tr(lds_read_tr(xt, t0), lds_read_tr(xt, t1)), xa, acc[db]);
+        acc[db] = emfma(ecat_tr(lds_read_tr(xt + 4096, t0), lds_read_tr(xt + 4096, t1)), xb, acc[db]);
       }
-    } else {
+    };
+    f32x16 s = {}, dp = {};
 #pragma unroll
-      for (int qh = 0; qh < 2; ++qh) {
-        dp[qh] = f32x16{};
+    for (int ks = 0; ks < NKS; ++ks) s = emfma(elds16(qt, aoff ^ (32 * ks)), kreg[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) dp[qh] = emfma(elds16(dt, qh * 8192 + aoff[ks]), kvreg[ks], dp[qh]);
-      }
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 l4 = *reinterpret_cast<const f32x4*>(&st_s[sb][0][32 * qh + 8 * g + 4 * hi]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * g + e] = exp2f_fast(fmaf(s[4 * g + e], a.scale_log2, -(l4[e] + kmask)));
     }
-    __syncthreads();  // P is in LDS
-    if (role == 1) {  // dS = P (dP - delta) / sqrt(D), dK += dS^T Q
+    {
+      float p[16];
 #pragma unroll
-      for (int qh = 0; qh < 2; ++qh) {
-        const ev8 pa = pex[(2 * qh) * 64 + l], pb = pex[(2 * qh + 1) * 64 + l];
-        float ds[16];
+      for (int r = 0; r < 16; ++r) p[r] = s[r];
+      product(dt, epack8(&p[0]), epack8(&p[8]), acc_v);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (dP after dV: raised above it, its operands do not fit the registers)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&st_s[sb][1][32 * qh + 8 * g + 4 * hi]);
+    for (int ks = 0; ks < NKS; ++ks) dp = emfma(elds16(dt, aoff ^ (32 * ks)), vreg[ks], dp);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * g + e;
-            const float pv = r < 8 ? (float)pa[r] : (float)pb[r - 8];
-            ds[r] = pv * (dp[qh][r] - d4[e]) * a.scale;
-          }
-        }
-        const ev8 sa = epack8(&ds[0]), sb8 = epack8(&ds[8]);
-        const char* xt = qt + qh * 8192;
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 d4 = *reinterpret_cast<const f32x4*>(&st_s[sb][1][32 * qh + 8 * g + 4 * hi]);
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          acc[db] = emfma(ecat_tr(lds_read_tr(xt, toff[0][db]), lds_read_tr(xt, toff[1][db])), sa, acc[db]);
-          acc[db] = emfma(ecat_tr(lds_read_tr(xt + 4096, toff[0][db]), lds_read_tr(xt + 4096, toff[1][db])), sb8, acc[db]);
-        }
-      }
+      for (int e = 0; e < 4; ++e) s[4 * g + e] = s[4 * g + e] * (dp[4 * g + e] - d4[e]) * a.scale;
+    }
+    {
+      float ds[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ds[r] = s[r];
+      product(qt, epack8(&ds[0]), epack8(&ds[8]), acc_k);
     }
     dma_wait();
-    if (j + 1 < nc && wv == 0) {
-      st_s[sb ^ 1][0][l] = ls;
-      st_s[sb ^ 1][1][l] = dl;
-    }
+    if (j + 1 < nc && wv == 0) stats(sb ^ 1);
     __syncthreads();
     inext = inn;
   }
 
+  // the second query half hands its sums over through the staging buffers: [key half][dV | dK][register][lane]
+  float* xch = reinterpret_cast<float*>(&qd_s[0][0][0]) + kh * (128 * 64);
+  if (qh == 1) {
 #pragma unroll
-  for (int db = NDB; db < 4; ++db) acc[db] = f32x16{};  // columns past D: zero
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        xch[(db * 16 + r) * 64 + l] = acc_v[db][r];
+        xch[(64 + db * 16 + r) * 64 + l] = acc_k[db][r];
+      }
+  }
+  __syncthreads();
+  if (qh == 1) return;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc_v[db][r] += xch[(db * 16 + r) * 64 + l];
+      acc_k[db][r] += xch[(64 + db * 16 + r) * 64 + l];
+    }
   const size_t tok = head + (size_t)kb * BK + key;
-  if (TASKS && slot >= 0) {
-    float* pa_out = (role == 0 ? a.part_b : a.part_a) + ((size_t)slot * BK + key) * HD;
+  // valid keys: dK and dV + add / cnt; padding keys: 0; split chunks: fp32 partials without the add
+  const float inv = kvalid ? 1.0f / (float)kcnt : 0.0f;
+  const float keep = kvalid ? 1.0f : 0.0f;
+  auto store = [&](const f32x16 (&acc)[4], const float* add, float* part, float* out32, e16_t* out16) {
+    const float* adp = add + ((size_t)bh * a.add_nb + kb) * HD;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<float4*>(pa_out + 32 * db + 8 * i + 4 * hi) =
-            make_float4(acc[db][4 * i], acc[db][4 * i + 1], acc[db][4 * i + 2], acc[db][4 * i + 3]);
-    return;
-  }
-  // valid keys: dK or dV + add / cnt; padding keys: 0
-  const float inv = kvalid ? 1.0f / (float)kcnt : 0.0f;
-  const float keep = kvalid ? 1.0f : 0.0f;
-  const float* add = role == 0 ? a.add_b : a.add_a;
-  const float* adp = add + ((size_t)bh * a.add_nb + kb) * HD;
-  float* out32 = role == 0 ? a.out_b32 : a.out_a32;
-  e16_t* out16 = role == 0 ? a.out_b : a.out_a;
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = 32 * db + 8 * i + 4 * hi;
-      f32x4 x4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x4[e] = acc[db][4 * i + e] * keep;
-      if (add != nullptr) x4 += *reinterpret_cast<const f32x4*>(adp + c) * inv;
-      if (out32 != nullptr) {
-        *reinterpret_cast<f32x4*>(out32 + tok * HD + c) = x4;
-      } else {
-        ushort4 o4;
-        o4.x = f2e(x4[0]); o4.y = f2e(x4[1]); o4.z = f2e(x4[2]); o4.w = f2e(x4[3]);
-        *reinterpret_cast<ushort4*>(out16 + tok * HD + c) = o4;
+      for (int i = 0; i < 4; ++i) {
+        const int c = 32 * db + 8 * i + 4 * hi;
+        f32x4 x4 = {};
+        if (db < NDB)  // (columns past D: zero)
+          x4 = f32x4{acc[db][4 * i], acc[db][4 * i + 1], acc[db][4 * i + 2], acc[db][4 * i + 3]};
+        if (TASKS && slot >= 0) {
+          *reinterpret_cast<f32x4*>(part + ((size_t)slot * BK + key) * HD + c) = x4;
+          continue;
+        }
+        x4 *= keep;
+        if (add != nullptr) x4 += *reinterpret_cast<const f32x4*>(adp + c) * inv;
+        if (out32 != nullptr) {
+          *reinterpret_cast<f32x4*>(out32 + tok * HD + c) = x4;
+        } else {
+          ushort4 o4;
+          o4.x = f2e(x4[0]); o4.y = f2e(x4[1]); o4.z = f2e(x4[2]); o4.w = f2e(x4[3]);
+          *reinterpret_cast<ushort4*>(out16 + tok * HD + c) = o4;
+        }
       }
-    }
+  };
+  store(acc_k, a.add_a, a.part_a, a.out_a32, a.out_a);
+  store(acc_v, a.add_b, a.part_b, a.out_b32, a.out_b);
 }
 
 
