@@ -14,7 +14,10 @@
  *                                    D = 64 caller zero-fills columns 64..127 (they add exact zeros to every dot
  *                                    product and come out zero); D sets the softmax scale 1 / sqrt(D). The fine
  *                                    attention entry points (vsa_attn_*) run a D = 64 kernel variant that reads
- *                                    and computes on the first 64 columns only
+ *                                    and computes on the first 64 columns only. D | VSA_PACKED_ROWS: every row
+ *                                    (tokens, pooled rows, fp32 gradients and partials) is D columns wide instead;
+ *                                    taken by the pooling, fusion, fine attention, router and split-KV entry
+ *                                    points, not by the three-tier ones (vsa_rep_*, vsa_row_dot)
  *   blk_cnt                          [NB] int32, valid tokens per block (1..64)
  *   router pools qr, kr, vr          [BH, Lr_pad, 128] bf16, Lr_pad = ceil64(NB * 64 / R)
  *   block means qc, kc, vc           [BH, NBc_pad, 128] bf16, NBc_pad = ceil64(NB)
@@ -27,6 +30,9 @@
 #define VSA_HIP_H
 
 #include "echosparse_hip.h"
+
+/* flag of the D argument: rows stored D columns wide (see D above) */
+#define VSA_PACKED_ROWS 0x10000
 
 #ifdef __cplusplus
 extern "C" {

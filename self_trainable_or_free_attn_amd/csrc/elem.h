@@ -9,6 +9,7 @@
 //   epack8, esum8 floats -> one MFMA operand; the fp32 sum of an operand's 8 values (v_dot2 against 1.0)
 //   elds16, ecat_tr  LDS row read / two transposed half-reads as one operand
 #pragma once
+#include "../../include/vsa_hip.h"
 #include "common.h"
 
 namespace es {
@@ -74,4 +75,19 @@ __device__ __forceinline__ ev8 ecat_tr(s16x4 a, s16x4 b) {
   return r;
 }
 
+// The D argument of the VSA entry points: the logical head dim (64 or 128) and, with VSA_PACKED_ROWS, rows stored D
+// columns wide instead of 128. ld: columns of a stored row.
+struct HeadDim {
+  int d, ld;
+};
+static inline bool head_dim(int D, HeadDim& h) {
+  const int flags = D & ~0xffff;
+  h.d = D & 0xffff;
+  h.ld = flags == VSA_PACKED_ROWS ? h.d : HD;
+  return (h.d == 64 || h.d == HD) && (flags == 0 || flags == VSA_PACKED_ROWS);
+}
+
 }  // namespace es
+
+#define VSA_REQUIRE_DIM(D, h) \
+  ES_REQUIRE(es::head_dim(D, h), ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)")

@@ -39,6 +39,7 @@ struct VsaFwdArgs {
   float *part_o, *part_lse;
   int* queues;  // the eight row-block queue counters of this launch (queues.h)
   int L, NB, BH, per_xcd, fixed;
+  int ld;       // columns of a stored row
   float scale;  // log2(e) / sqrt(D)
 };
 
@@ -78,18 +79,19 @@ __global__ __launch_bounds__(256, 2) void vsa_fwd_kernel(VsaFwdArgs a) {
   const bool qvalid = qrow < qcnt;
   const size_t head = (size_t)bh * a.L;
 
-  const unsigned head_bytes = (unsigned)((size_t)a.L * HD * 2);
-  const srd_t rk = make_srd(a.k + head * HD, head_bytes);
-  const srd_t rv = make_srd(a.v + head * HD, head_bytes);
+  const int ld = DH == HD ? HD : a.ld;  // columns of a stored row
+  const unsigned head_bytes = (unsigned)((size_t)a.L * ld * 2);
+  const srd_t rk = make_srd(a.k + head * ld, head_bytes);
+  const srd_t rv = make_srd(a.v + head * ld, head_bytes);
   // this lane's four load rows R = 16 wv + 4 i + l / 16 of a chunk and its swizzled 16-byte chunk in them
   unsigned ld_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int P = (wv * 4 + i) * 64 + l, R = P >> 4, g = (P & 15) ^ swz(R);
-    ld_off[i] = g < DH / 8 ? (unsigned)R * 256 + (unsigned)(g * 16) : 0x80000000u;
+    ld_off[i] = g < DH / 8 ? (unsigned)(R * ld * 2) + (unsigned)(g * 16) : 0x80000000u;
   }
   auto issue = [&](int b, int sb) {
-    const unsigned soff = (unsigned)b * (BK * 256);
+    const unsigned soff = (unsigned)(b * BK * ld * 2);
     char* kd = kv_s[sb][0] + wv * 4096;
     char* vd = kv_s[sb][1] + wv * 4096;
 #pragma unroll
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void vsa_fwd_kernel(VsaFwdArgs a) {
 
   ev8 qreg[8];
   {
-    const e16_t* qp = a.q + (head + (size_t)qb * BK + qrow) * HD;
+    const e16_t* qp = a.q + (head + (size_t)qb * BK + qrow) * ld;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qreg[ks] = *reinterpret_cast<const ev8*>(qp + 16 * ks + 8 * hi);
   }
@@ -207,11 +209,12 @@ __global__ __launch_bounds__(256, 2) void vsa_fwd_kernel(VsaFwdArgs a) {
   const size_t tok = head + (size_t)qb * BK + qrow;
   const float lse2 = live ? M + log2f(lt) : -INFINITY;
   if (!TASKS || slot < 0) {
-    e16_t* orow = a.out + tok * HD;
+    e16_t* orow = a.out + tok * ld;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        if (DH < HD && 32 * db >= ld) break;
         ushort4 v4;
         v4 = ushort4{0, 0, 0, 0};
         if (db < NDB) {
@@ -224,11 +227,12 @@ __global__ __launch_bounds__(256, 2) void vsa_fwd_kernel(VsaFwdArgs a) {
       }
     if (hi == 0) a.lse[tok] = live ? lse2 * LN2 : -INFINITY;
   } else {
-    float* prow = a.part_o + ((size_t)slot * BK + qrow) * HD;
+    float* prow = a.part_o + ((size_t)slot * BK + qrow) * ld;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        if (DH < HD && 32 * db >= ld) break;
         float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
         if (db < NDB) {
           v4.x = (a0 * o[db][4 * i + 0] + a1 * xo[(db * 16 + 4 * i + 0) * 64 + l]) * inv;
@@ -266,6 +270,7 @@ struct VsaBwdArgs {
   float *part_a, *part_b;      // split partials [slot, 64, D]
   int* queues;                 // the eight row-block queue counters of this launch (queues.h)
   int L, NB, BH, per_xcd, fixed;
+  int ld;                      // columns of a stored row
   float scale_log2, scale;
 };
 
@@ -321,18 +326,19 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   const bool kvalid = key < kcnt;
   const size_t head = (size_t)bh * a.L;
 
-  const unsigned head_bytes = (unsigned)((size_t)a.L * HD * 2);
-  const srd_t rq = make_srd(a.q + head * HD, head_bytes);
-  const srd_t rd = make_srd(a.dout + head * HD, head_bytes);
-  // transfer r of a wave moves rows 16 wv + 4 r + l / 16: this lane's source offset is ld_off ^ 16 r plus 1024 r
+  const int ld = DH == HD ? HD : a.ld;  // columns of a stored row
+  const unsigned head_bytes = (unsigned)((size_t)a.L * ld * 2);
+  const srd_t rq = make_srd(a.q + head * ld, head_bytes);
+  const srd_t rd = make_srd(a.dout + head * ld, head_bytes);
+  // transfer r of a wave moves rows 16 wv + 4 r + l / 16: this lane's source offset is ld_off ^ 16 r plus 4 r rows
   unsigned ld_off;
   {
     const int g = (l & 15) ^ ((l >> 4) << 2);
-    ld_off = g < DH / 8 ? (unsigned)(wv * 16 + (l >> 4)) * 256 + (unsigned)(g * 16) : 0x80000000u;
+    ld_off = g < DH / 8 ? (unsigned)((wv * 16 + (l >> 4)) * ld * 2) + (unsigned)(g * 16) : 0x80000000u;
   }
   ev8 kreg[8], vreg[8];  // this lane's key row
   {
-    const size_t off = (head + (size_t)kb * BK + key) * HD + 8 * hi;
+    const size_t off = (head + (size_t)kb * BK + key) * ld + 8 * hi;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       kreg[ks] = *reinterpret_cast<const ev8*>(a.k + off + 16 * ks);
@@ -344,11 +350,11 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   const srd_t rl = make_srd(a.lse + head, (unsigned)a.L * 4u);
   const srd_t re = make_srd(a.delta + head, (unsigned)a.L * 4u);
   auto issue = [&](int i, int sb) {
-    const unsigned soff = (unsigned)i * (BK * 256);
+    const unsigned soff = (unsigned)(i * BK * ld * 2);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      dma16(rq, qd_s[sb][0] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + 1024u * r);
-      dma16(rd, qd_s[sb][1] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + 1024u * r);
+      dma16(rq, qd_s[sb][0] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + (unsigned)(8 * r * ld));
+      dma16(rd, qd_s[sb][1] + wv * 4096 + r * 1024, ld_off ^ (16u * r), soff + (unsigned)(8 * r * ld));
     }
     if (wv == 0) {
       dma4(rl, lse_s, 4u * l, (unsigned)i * (BK * 4));
@@ -461,27 +467,28 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   const float inv = kvalid ? 1.0f / (float)kcnt : 0.0f;
   const float keep = kvalid ? 1.0f : 0.0f;
   auto store = [&](const f32x16 (&acc)[4], const float* add, float* part, float* out32, e16_t* out16) {
-    const float* adp = add + ((size_t)bh * a.add_nb + kb) * HD;
+    const float* adp = add + ((size_t)bh * a.add_nb + kb) * ld;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        if (DH < HD && 32 * db >= ld) break;
         const int c = 32 * db + 8 * i + 4 * hi;
         f32x4 x4 = {};
         if (db < NDB)  // (columns past D: zero)
           x4 = f32x4{acc[db][4 * i], acc[db][4 * i + 1], acc[db][4 * i + 2], acc[db][4 * i + 3]};
         if (TASKS && slot >= 0) {
-          *reinterpret_cast<f32x4*>(part + ((size_t)slot * BK + key) * HD + c) = x4;
+          *reinterpret_cast<f32x4*>(part + ((size_t)slot * BK + key) * ld + c) = x4;
           continue;
         }
         x4 *= keep;
         if (add != nullptr) x4 += *reinterpret_cast<const f32x4*>(adp + c) * inv;
         if (out32 != nullptr) {
-          *reinterpret_cast<f32x4*>(out32 + tok * HD + c) = x4;
+          *reinterpret_cast<f32x4*>(out32 + tok * ld + c) = x4;
         } else {
           ushort4 o4;
           o4.x = f2e(x4[0]); o4.y = f2e(x4[1]); o4.z = f2e(x4[2]); o4.w = f2e(x4[3]);
-          *reinterpret_cast<ushort4*>(out16 + tok * HD + c) = o4;
+          *reinterpret_cast<ushort4*>(out16 + tok * ld + c) = o4;
         }
       }
   };
@@ -506,26 +513,27 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_q_kernel(VsaBwdArgs a) {
   const size_t head = (size_t)bh * a.L;
   const size_t tok = head + (size_t)qb * BK + qrow;
 
+  const int ld = DH == HD ? HD : a.ld;  // columns of a stored row
   ev8 qreg[8], dreg[8];
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) {
-    qreg[ks] = *reinterpret_cast<const ev8*>(a.q + tok * HD + 16 * ks + 8 * hi);
-    dreg[ks] = *reinterpret_cast<const ev8*>(a.dout + tok * HD + 16 * ks + 8 * hi);
+    qreg[ks] = *reinterpret_cast<const ev8*>(a.q + tok * ld + 16 * ks + 8 * hi);
+    dreg[ks] = *reinterpret_cast<const ev8*>(a.dout + tok * ld + 16 * ks + 8 * hi);
   }
   const float ls = qvalid ? lse_to_log2(a.lse[tok]) : INFINITY;
   const float dl = a.delta[tok];
 
-  const unsigned head_bytes = (unsigned)((size_t)a.L * HD * 2);
-  const srd_t rk = make_srd(a.k + head * HD, head_bytes);
-  const srd_t rv = make_srd(a.v + head * HD, head_bytes);
+  const unsigned head_bytes = (unsigned)((size_t)a.L * ld * 2);
+  const srd_t rk = make_srd(a.k + head * ld, head_bytes);
+  const srd_t rv = make_srd(a.v + head * ld, head_bytes);
   unsigned ld_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int P = (wv * 4 + i) * 64 + l, R = P >> 4, g = (P & 15) ^ swz(R);
-    ld_off[i] = g < DH / 8 ? (unsigned)R * 256 + (unsigned)(g * 16) : 0x80000000u;
+    ld_off[i] = g < DH / 8 ? (unsigned)(R * ld * 2) + (unsigned)(g * 16) : 0x80000000u;
   }
   auto issue = [&](int b, int sb) {
-    const unsigned soff = (unsigned)b * (BK * 256);
+    const unsigned soff = (unsigned)(b * BK * ld * 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dma16(rk, kv_s[sb][0] + wv * 4096 + i * 1024, ld_off[i], soff);
@@ -605,34 +613,37 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_q_kernel(VsaBwdArgs a) {
 #pragma unroll
   for (int db = NDB; db < 4; ++db) dq[db] = f32x16{};  // columns past D: zero
   if (TASKS && slot >= 0) {
-    float* pq = a.part_a + ((size_t)slot * BK + qrow) * HD;
+    float* pq = a.part_a + ((size_t)slot * BK + qrow) * ld;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        if (DH < HD && 32 * db >= ld) break;
         *reinterpret_cast<float4*>(pq + 32 * db + 8 * i + 4 * hi) =
             make_float4(dq[db][4 * i], dq[db][4 * i + 1], dq[db][4 * i + 2], dq[db][4 * i + 3]);
+      }
     return;
   }
   const float inv = qvalid ? 1.0f / (float)qcnt : 0.0f;
   const float keep = qvalid ? 1.0f : 0.0f;
-  const float* adq = a.add_a + ((size_t)bh * a.add_nb + qb) * HD;
+  const float* adq = a.add_a + ((size_t)bh * a.add_nb + qb) * ld;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      if (DH < HD && 32 * db >= ld) break;
       const int c = 32 * db + 8 * i + 4 * hi;
       f32x4 x;
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] = dq[db][4 * i + e] * keep;
       if (a.out_a32 != nullptr) {  // dq_acc += dQ (padding rows keep their value)
-        f32x4* dst = reinterpret_cast<f32x4*>(a.out_a32 + tok * HD + c);
+        f32x4* dst = reinterpret_cast<f32x4*>(a.out_a32 + tok * ld + c);
         *dst = *dst + x;
       } else {
         if (a.add_a != nullptr) x += *reinterpret_cast<const f32x4*>(adq + c) * inv;
         ushort4 q4;
         q4.x = f2e(x[0]); q4.y = f2e(x[1]); q4.z = f2e(x[2]); q4.w = f2e(x[3]);
-        *reinterpret_cast<ushort4*>(a.out_a + tok * HD + c) = q4;
+        *reinterpret_cast<ushort4*>(a.out_a + tok * ld + c) = q4;
       }
     }
 }
@@ -646,7 +657,8 @@ using namespace es;
 static int vsa_check_qkv(const void* q, const void* k, const void* v, int BH, int L, int D) {
   ES_REQUIRE(q && k && v, ES_ERR_INVALID, "VSA: null q / k / v");
   ES_REQUIRE(BH > 0 && L > 0 && L % BK == 0, ES_ERR_INVALID, "VSA: tokens must be [BH, L = NB * 64, D]");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE((size_t)L * HD * 2 < (1ull << 31), ES_ERR_UNSUPPORTED, "VSA: one head's tokens exceed 2 GiB");
   return ES_OK;
 }
@@ -660,7 +672,10 @@ static VsaFwdArgs fwd_args(const void* q, const void* k, const void* v, const in
   a.L = L;
   a.NB = L / BK;
   a.BH = BH;
-  a.scale = LOG2E / sqrtf((float)D);  // D: the logical head dimension (64 or 128)
+  HeadDim h;
+  head_dim(D, h);
+  a.ld = h.ld;
+  a.scale = LOG2E / sqrtf((float)h.d);
   return a;
 }
 
@@ -679,7 +694,7 @@ extern "C" int ES_VSA_API(vsa_attn_fwd)(const void* q, const void* k, const void
   ES_REQUIRE(balanced_launch(BH, a.per_xcd, stream, qs), ES_ERR_LAUNCH, "VSA: row-block queues unavailable");
   a.queues = qs.counters;
   a.fixed = qs.fixed;
-  if (D == 64) hipLaunchKernelGGL((vsa_fwd_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_fwd_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_fwd_kernel<false, 128>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_fwd");
 }
@@ -701,7 +716,7 @@ extern "C" int ES_VSA_API(vsa_attn_fwd_tasks)(const void* q, const void* k, cons
   a.lse = lse;
   a.part_o = part_o;
   a.part_lse = part_lse;
-  if (D == 64) hipLaunchKernelGGL((vsa_fwd_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_fwd_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_fwd_kernel<true, 128>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_fwd_tasks");
 }
@@ -721,8 +736,11 @@ static VsaBwdArgs bwd_args(const void* q, const void* k, const void* v, const vo
   a.NB = L / BK;
   a.BH = BH;
   a.per_xcd = (a.NB + 7) / 8;
-  a.scale = 1.0f / sqrtf((float)D);
-  a.scale_log2 = LOG2E / sqrtf((float)D);
+  HeadDim h;
+  head_dim(D, h);
+  a.ld = h.ld;
+  a.scale = 1.0f / sqrtf((float)h.d);
+  a.scale_log2 = LOG2E / sqrtf((float)h.d);
   return a;
 }
 
@@ -752,7 +770,7 @@ extern "C" int ES_VSA_API(vsa_attn_bwd_kv)(const void* q, const void* k, const v
   ES_REQUIRE(balanced_launch(BH, a.per_xcd, stream, qs), ES_ERR_LAUNCH, "VSA: row-block queues unavailable");
   a.queues = qs.counters;
   a.fixed = qs.fixed;
-  if (D == 64) hipLaunchKernelGGL((vsa_bwd_kv_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_bwd_kv_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_bwd_kv_kernel<false, 128>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_bwd_kv");
 }
@@ -777,7 +795,7 @@ extern "C" int ES_VSA_API(vsa_attn_bwd_kv_tasks)(const void* q, const void* k, c
   a.out_b = (e16_t*)dv;
   a.part_a = part_dk;
   a.part_b = part_dv;
-  if (D == 64) hipLaunchKernelGGL((vsa_bwd_kv_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_bwd_kv_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_bwd_kv_kernel<true, 128>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_bwd_kv_tasks");
 }
@@ -801,7 +819,7 @@ extern "C" int ES_VSA_API(vsa_attn_bwd_q)(const void* q, const void* k, const vo
   ES_REQUIRE(balanced_launch(BH, a.per_xcd, stream, qs), ES_ERR_LAUNCH, "VSA: row-block queues unavailable");
   a.queues = qs.counters;
   a.fixed = qs.fixed;
-  if (D == 64) hipLaunchKernelGGL((vsa_bwd_q_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_bwd_q_kernel<false, 64>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_bwd_q_kernel<false, 128>), dim3((unsigned)qs.grid), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_bwd_q");
 }
@@ -822,7 +840,7 @@ extern "C" int ES_VSA_API(vsa_attn_bwd_q_tasks)(const void* q, const void* k, co
   a.add_nb = add_nb;
   a.out_a = (e16_t*)dq;
   a.part_a = part_dq;
-  if (D == 64) hipLaunchKernelGGL((vsa_bwd_q_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
+  if ((D & 0xffff) == 64) hipLaunchKernelGGL((vsa_bwd_q_kernel<true, 64>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((vsa_bwd_q_kernel<true, 128>), dim3((unsigned)max_tasks), dim3(256), 0, stream, a);
   return check_launch("vsa_attn_bwd_q_tasks");
 }

@@ -57,6 +57,7 @@ struct PoolArgs {
   e16_t* blk[3];        // qc, kc, vc
   const int* blk_cnt;
   int NB, L, R, Lr_pad, NBc_pad;
+  int ld;  // columns of a stored row
 };
 
 constexpr int POOL_BLOCKS = 4;  // 64-token blocks per workgroup
@@ -72,19 +73,20 @@ __global__ __launch_bounds__(192) void pool_kernel(PoolArgs a) {
   const int sub = threadIdx.x / 48, t = threadIdx.x % 48;
   const int blk = blockIdx.x * POOL_BLOCKS + sub;
   const int which = t / 16, c8 = (t % 16) * 8;
-  if (a.src[which] == nullptr) return;  // a null source: that tensor is not pooled
+  const int ld = a.ld;
+  if (a.src[which] == nullptr || c8 >= ld) return;  // a null source: that tensor is not pooled
   const size_t bh = blockIdx.y;
   e16_t* grp = a.grp[which];
   if (blk >= a.NB) {
     const uint4 z = {0u, 0u, 0u, 0u};
-    if (blk < a.NBc_pad) *reinterpret_cast<uint4*>(a.blk[which] + (bh * a.NBc_pad + blk) * HD + c8) = z;
+    if (blk < a.NBc_pad) *reinterpret_cast<uint4*>(a.blk[which] + (bh * a.NBc_pad + blk) * ld + c8) = z;
     if (grp != nullptr)
       for (int r = blk * G; r < min((blk + 1) * G, a.Lr_pad); ++r)
-        *reinterpret_cast<uint4*>(grp + (bh * a.Lr_pad + r) * HD + c8) = z;
+        *reinterpret_cast<uint4*>(grp + (bh * a.Lr_pad + r) * ld + c8) = z;
     return;
   }
   const int n = a.blk_cnt[blk];
-  const e16_t* src = a.src[which] + (bh * a.L + (size_t)blk * BK) * HD + c8;
+  const e16_t* src = a.src[which] + (bh * a.L + (size_t)blk * BK) * ld + c8;
   float tot[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(192) void pool_kernel(PoolArgs a) {
     uint4 u[BATCH];
 #pragma unroll
     for (int i = 0; i < BATCH; ++i)
-      u[i] = r0 + i < n ? *reinterpret_cast<const uint4*>(src + (size_t)(r0 + i) * HD) : uint4{0u, 0u, 0u, 0u};
+      u[i] = r0 + i < n ? *reinterpret_cast<const uint4*>(src + (size_t)(r0 + i) * ld) : uint4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
       float x[8];
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(192) void pool_kernel(PoolArgs a) {
           float m[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) m[e] = mul_rn(s[e], inv);
-          st8(grp + (bh * a.Lr_pad + (size_t)blk * G + g) * HD + c8, m);
+          st8(grp + (bh * a.Lr_pad + (size_t)blk * G + g) * ld + c8, m);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(192) void pool_kernel(PoolArgs a) {
   const float inv = 1.f / (float)n;
 #pragma unroll
   for (int e = 0; e < 8; ++e) tot[e] = mul_rn(tot[e], inv);
-  st8(a.blk[which] + (bh * a.NBc_pad + blk) * HD + c8, tot);
+  st8(a.blk[which] + (bh * a.NBc_pad + blk) * ld + c8, tot);
 }
 
 static void launch_pool(const PoolArgs& a, int BH, hipStream_t stream) {
@@ -141,31 +143,33 @@ struct FuseArgs {
   float *delta_f, *delta_c;
   const int* blk_cnt;
   int NB, L, NBc_pad, gate_mode, gate_act;
+  int ld;  // columns of a stored row
 };
 
 // grid (cdiv(NB, 4), BH), 256 threads: one wave per 64-token block
 __global__ __launch_bounds__(256) void fuse_fwd_kernel(FuseArgs a) {
   const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (blk >= a.NB) return;
-  const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8;
+  const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8, ld = a.ld;
+  if (c8 >= ld) return;
   const size_t bh = blockIdx.y;
   const int n = a.blk_cnt[blk];
   float c[8];
-  ld8(a.oc + (bh * a.NBc_pad + blk) * HD + c8, c);
+  ld8(a.oc + (bh * a.NBc_pad + blk) * ld + c8, c);
   const size_t tok0 = bh * a.L + (size_t)blk * BK;
 #pragma unroll 4
   for (int r = s; r < BK; r += 4) {
     const size_t tok = tok0 + r;
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (r < n) {
-      ld8(a.of + tok * HD + c8, x);
+      ld8(a.of + tok * ld + c8, x);
       if (a.gate_mode == 1) {
         const float g = gact(e2f(a.gate[tok]), a.gate_act);
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] += g * c[e];
       } else if (a.gate_mode == 2) {
         float g[8];
-        ld8(a.gate + tok * HD + c8, g);
+        ld8(a.gate + tok * ld + c8, g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] += gact(g[e], a.gate_act) * c[e];
       } else {
@@ -173,35 +177,36 @@ __global__ __launch_bounds__(256) void fuse_fwd_kernel(FuseArgs a) {
         for (int e = 0; e < 8; ++e) x[e] += c[e];
       }
     }
-    st8(a.o + tok * HD + c8, x);
+    st8(a.o + tok * ld + c8, x);
   }
 }
 
 __global__ __launch_bounds__(256) void fuse_bwd_kernel(FuseArgs a) {
   const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (blk >= a.NBc_pad) return;
-  const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8;
+  const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8, ld = a.ld;
+  const bool col = c8 < ld;  // (lanes past a stored row hold zeros and store nothing)
   const size_t bh = blockIdx.y;
-  const size_t crow = (bh * a.NBc_pad + blk) * HD;
+  const size_t crow = (bh * a.NBc_pad + blk) * ld;
   if (blk >= a.NB) {  // padding rows of the coarse tensors
-    if (s == 0) *reinterpret_cast<uint4*>(a.dout_c + crow + c8) = uint4{0u, 0u, 0u, 0u};
+    if (s == 0 && col) *reinterpret_cast<uint4*>(a.dout_c + crow + c8) = uint4{0u, 0u, 0u, 0u};
     if (l == 0) a.delta_c[bh * a.NBc_pad + blk] = 0.f;
     return;
   }
   const int n = a.blk_cnt[blk];
-  float c[8], dc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  ld8(a.oc + crow + c8, c);
+  float c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (col) ld8(a.oc + crow + c8, c);
   const size_t tok0 = bh * a.L + (size_t)blk * BK;
 #pragma unroll 4
   for (int r = s; r < BK; r += 4) {
     const size_t tok = tok0 + r;
     const bool valid = r < n;
     float d[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (valid) {
-      ld8(a.dout + tok * HD + c8, d);
-      ld8(a.of + tok * HD + c8, f);
+    if (valid && col) {
+      ld8(a.dout + tok * ld + c8, d);
+      ld8(a.of + tok * ld + c8, f);
     }
-    if (a.dout_f != nullptr) st8(a.dout_f + tok * HD + c8, d);
+    if (a.dout_f != nullptr && col) st8(a.dout_f + tok * ld + c8, d);
     float dot_f = 0.f, dot_c = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) dot_f += d[e] * f[e];
@@ -215,14 +220,14 @@ __global__ __launch_bounds__(256) void fuse_bwd_kernel(FuseArgs a) {
       dot_c *= gdact(g, a.gate_act);
     } else if (a.gate_mode == 2) {
       float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dg[8];
-      if (valid) ld8(a.gate + tok * HD + c8, g);
+      if (valid && col) ld8(a.gate + tok * ld + c8, g);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float ge = valid ? gact(g[e], a.gate_act) : 0.f;
         dg[e] = valid ? gdact(ge, a.gate_act) * d[e] * c[e] : 0.f;
         dc[e] += ge * d[e];
       }
-      st8(a.dgate + tok * HD + c8, dg);
+      if (col) st8(a.dgate + tok * ld + c8, dg);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) dc[e] += d[e];
@@ -242,7 +247,7 @@ __global__ __launch_bounds__(256) void fuse_bwd_kernel(FuseArgs a) {
   }
   float part = 0.f;
   if (s == 0) {
-    st8(a.dout_c + crow + c8, dc);
+    if (col) st8(a.dout_c + crow + c8, dc);
 #pragma unroll
     for (int e = 0; e < 8; ++e) part += e2f(f2e(dc[e])) * c[e];
   }
@@ -254,16 +259,17 @@ __global__ __launch_bounds__(256) void fuse_bwd_kernel(FuseArgs a) {
 // [BH, add_nb, D] (optional)
 __global__ __launch_bounds__(256) void finalize_kernel(const float* __restrict__ acc, const float* __restrict__ add,
                                                        e16_t* __restrict__ out, const int* __restrict__ blk_cnt,
-                                                       int NB, int L, int add_nb) {
+                                                       int NB, int L, int add_nb, int ld) {
   const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (blk >= NB) return;
   const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8;
+  if (c8 >= ld) return;
   const size_t bh = blockIdx.y;
   const int n = blk_cnt[blk];
   float ad[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (add != nullptr) {
     const float inv = 1.f / (float)n;
-    const float4* p = reinterpret_cast<const float4*>(add + (bh * add_nb + blk) * HD + c8);
+    const float4* p = reinterpret_cast<const float4*>(add + (bh * add_nb + blk) * ld + c8);
     const float4 u = p[0], w = p[1];
     ad[0] = u.x * inv; ad[1] = u.y * inv; ad[2] = u.z * inv; ad[3] = u.w * inv;
     ad[4] = w.x * inv; ad[5] = w.y * inv; ad[6] = w.z * inv; ad[7] = w.w * inv;
@@ -275,14 +281,14 @@ __global__ __launch_bounds__(256) void finalize_kernel(const float* __restrict__
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (r < n) {
       if (acc != nullptr) {
-        const float4* p = reinterpret_cast<const float4*>(acc + tok * HD + c8);
+        const float4* p = reinterpret_cast<const float4*>(acc + tok * ld + c8);
         const float4 u = p[0], w = p[1];
         x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w; x[4] = w.x; x[5] = w.y; x[6] = w.z; x[7] = w.w;
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] += ad[e];
     }
-    st8(out + tok * HD + c8, x);
+    st8(out + tok * ld + c8, x);
   }
 }
 
@@ -304,37 +310,39 @@ __global__ void rep_counts_kernel(const int* __restrict__ blk_cnt, float* __rest
 
 using namespace es;
 
-static int check_tokens(int BH, int L, int D) {
+static int check_tokens(int BH, int L, int D, HeadDim& h) {
   ES_REQUIRE(BH > 0 && BH <= 65535 && L > 0 && L % BK == 0, ES_ERR_INVALID,
              "VSA: tokens must be [BH <= 65535, L = NB * 64, D]");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  VSA_REQUIRE_DIM(D, h);
   return ES_OK;
 }
 
 extern "C" int ES_VSA_API(vsa_pool)(const void* q, const void* k, const void* v, const int* blk_cnt, void* qr, void* kr, void* vr,
                         void* qc, void* kc, void* vc, int BH, int L, int D, int R, hipStream_t stream) {
-  if (int st = check_tokens(BH, L, D)) return st;
+  HeadDim h;
+  if (int st = check_tokens(BH, L, D, h)) return st;
   ES_REQUIRE(q && k && v && blk_cnt && qc && kc && vc, ES_ERR_INVALID, "VSA: null tensor pointer");
   ES_REQUIRE(R == 4 || R == 8 || R == 16 || R == 32, ES_ERR_INVALID, "VSA2: router pool size R must be 4, 8, 16 or 32");
   const int NB = L / BK, G = BK / R;
   PoolArgs a{{(const e16_t*)q, (const e16_t*)k, (const e16_t*)v},
              {(e16_t*)qr, (e16_t*)kr, (e16_t*)vr},
              {(e16_t*)qc, (e16_t*)kc, (e16_t*)vc},
-             blk_cnt, NB, L, R, (NB * G + 63) / 64 * 64, (NB + 63) / 64 * 64};
+             blk_cnt, NB, L, R, (NB * G + 63) / 64 * 64, (NB + 63) / 64 * 64, h.ld};
   launch_pool(a, BH, stream);
   return check_launch("vsa_pool");
 }
 
 extern "C" int ES_VSA_API(vsa_fuse_fwd)(const void* of, const void* oc, const void* gate, void* o, const int* blk_cnt, int BH,
                             int L, int D, int NBc_pad, int gate_mode, int gate_act, hipStream_t stream) {
-  if (int st = check_tokens(BH, L, D)) return st;
+  HeadDim h;
+  if (int st = check_tokens(BH, L, D, h)) return st;
   ES_REQUIRE(of && oc && o && blk_cnt && (gate_mode == 0 || gate), ES_ERR_INVALID, "VSA: null tensor pointer");
   ES_REQUIRE(gate_mode >= 0 && gate_mode <= 2 && (gate_act == 0 || gate_act == 1), ES_ERR_INVALID,
              "VSA: gate_mode must be 0 (none), 1 (per token) or 2 (elementwise), gate_act 0 (tanh) or 1 (identity)");
   const int NB = L / BK;
   ES_REQUIRE(NBc_pad >= NB, ES_ERR_INVALID, "VSA: coarse output has fewer rows than blocks");
   FuseArgs a{nullptr, (const e16_t*)of, (const e16_t*)oc, (const e16_t*)gate, (e16_t*)o, nullptr, nullptr, nullptr,
-             nullptr, nullptr, blk_cnt, NB, L, NBc_pad, gate_mode, gate_act};
+             nullptr, nullptr, blk_cnt, NB, L, NBc_pad, gate_mode, gate_act, h.ld};
   hipLaunchKernelGGL(fuse_fwd_kernel, dim3((NB + 3) / 4, BH), dim3(256), 0, stream, a);
   return check_launch("vsa_fuse_fwd");
 }
@@ -342,7 +350,8 @@ extern "C" int ES_VSA_API(vsa_fuse_fwd)(const void* of, const void* oc, const vo
 extern "C" int ES_VSA_API(vsa_fuse_bwd)(const void* dout, const void* of, const void* oc, const void* gate, void* dout_f,
                             float* delta_f, void* dout_c, float* delta_c, void* dgate, const int* blk_cnt, int BH,
                             int L, int D, int NBc_pad, int gate_mode, int gate_act, hipStream_t stream) {
-  if (int st = check_tokens(BH, L, D)) return st;
+  HeadDim h;
+  if (int st = check_tokens(BH, L, D, h)) return st;
   ES_REQUIRE(dout && of && oc && delta_f && dout_c && delta_c && blk_cnt, ES_ERR_INVALID, "VSA: null tensor pointer");
   ES_REQUIRE(gate_mode >= 0 && gate_mode <= 2 && (gate_act == 0 || gate_act == 1), ES_ERR_INVALID,
              "VSA: gate_mode must be 0 (none), 1 (per token) or 2 (elementwise), gate_act 0 (tanh) or 1 (identity)");
@@ -350,26 +359,29 @@ extern "C" int ES_VSA_API(vsa_fuse_bwd)(const void* dout, const void* of, const 
   const int NB = L / BK;
   ES_REQUIRE(NBc_pad >= NB, ES_ERR_INVALID, "VSA: coarse output has fewer rows than blocks");
   FuseArgs a{(const e16_t*)dout, (const e16_t*)of, (const e16_t*)oc, (const e16_t*)gate, nullptr, (e16_t*)dout_f,
-             (e16_t*)dout_c, (e16_t*)dgate, delta_f, delta_c, blk_cnt, NB, L, NBc_pad, gate_mode, gate_act};
+             (e16_t*)dout_c, (e16_t*)dgate, delta_f, delta_c, blk_cnt, NB, L, NBc_pad, gate_mode, gate_act, h.ld};
   hipLaunchKernelGGL(fuse_bwd_kernel, dim3((NBc_pad + 3) / 4, BH), dim3(256), 0, stream, a);
   return check_launch("vsa_fuse_bwd");
 }
 
 extern "C" int ES_VSA_API(vsa_finalize)(const float* acc, const float* add, int add_nb, void* out, const int* blk_cnt, int BH,
                             int L, int D, hipStream_t stream) {
-  if (int st = check_tokens(BH, L, D)) return st;
+  HeadDim h;
+  if (int st = check_tokens(BH, L, D, h)) return st;
   ES_REQUIRE(out && blk_cnt, ES_ERR_INVALID, "VSA: null tensor pointer");
   const int NB = L / BK;
   ES_REQUIRE(add == nullptr || add_nb >= NB, ES_ERR_INVALID, "VSA: finalize add has fewer rows than blocks");
   hipLaunchKernelGGL(finalize_kernel, dim3((NB + 3) / 4, BH), dim3(256), 0, stream, acc, add, (e16_t*)out, blk_cnt,
-                     NB, L, add_nb);
+                     NB, L, add_nb, h.ld);
   return check_launch("vsa_finalize");
 }
 
 extern "C" int ES_VSA_API(vsa_rep_build)(const void* k, const void* v, const int* blk_cnt, void* k_mid, void* v_mid,
                              float* lc_mid, void* k_tail, void* v_tail, float* lc_tail, int BH, int L, int D, int RM,
                              hipStream_t stream) {
-  if (int st = check_tokens(BH, L, D)) return st;
+  HeadDim h;
+  if (int st = check_tokens(BH, L, D, h)) return st;
+  ES_REQUIRE(D == h.d, ES_ERR_UNSUPPORTED, "VSA2-rep: rows must be stored with 128 columns");
   ES_REQUIRE(k && v && blk_cnt && k_mid && v_mid && lc_mid && k_tail && v_tail && lc_tail, ES_ERR_INVALID,
              "VSA2-rep: null tensor pointer");
   ES_REQUIRE(RM == 1 || RM == 2 || RM == 4 || RM == 8 || RM == 16, ES_ERR_INVALID,
@@ -379,7 +391,7 @@ extern "C" int ES_VSA_API(vsa_rep_build)(const void* k, const void* v, const int
   PoolArgs a{{nullptr, (const e16_t*)k, (const e16_t*)v},
              {nullptr, (e16_t*)k_mid, (e16_t*)v_mid},
              {nullptr, (e16_t*)k_tail, (e16_t*)v_tail},
-             blk_cnt, NB, L, R, (NB * RM + 63) / 64 * 64, (NB + 63) / 64 * 64};
+             blk_cnt, NB, L, R, (NB * RM + 63) / 64 * 64, (NB + 63) / 64 * 64, HD};
   launch_pool(a, BH, stream);
   hipLaunchKernelGGL(rep_counts_kernel, dim3((NB * RM + 255) / 256), dim3(256), 0, stream, blk_cnt, lc_mid, lc_tail,
                      NB, RM);

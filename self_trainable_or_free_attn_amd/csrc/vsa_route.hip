@@ -55,6 +55,7 @@ struct RowsArgs {
   int *q2k_ptr, *q2k_idx;
   unsigned* selbits;          // [bh_count, ceil32(NB), W]
   int NB, NBc_pad, bh0, K, W;
+  int ld;  // columns of a stored row
   float scale;
 };
 
@@ -121,15 +122,17 @@ __global__ __launch_bounds__(256) void rows_select_kernel(RowsArgs a) {
     }
   } else {
     // S strip: A = qc rows t0 .. t0 + 31 (registers), B = kc rows of each 32-column tile (L2)
+    const int ld = a.ld, nks = ld / 16;  // (wave-uniform)
     ev8 qa[8];
-    const e16_t* qp = a.qc + (bh * a.NBc_pad + t0 + lq) * HD + 8 * hi;
+    const e16_t* qp = a.qc + (bh * a.NBc_pad + t0 + lq) * ld + 8 * hi;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qa[ks] = *reinterpret_cast<const ev8*>(qp + 16 * ks);
+    for (int ks = 0; ks < 8; ++ks) qa[ks] = ks < nks ? *reinterpret_cast<const ev8*>(qp + 16 * ks) : ev8{};
     for (int ct = wv; ct < NBp / 32; ct += 4) {
-      const e16_t* kp = a.kc + (bh * a.NBc_pad + ct * 32 + lq) * HD + 8 * hi;
+      const e16_t* kp = a.kc + (bh * a.NBc_pad + ct * 32 + lq) * ld + 8 * hi;
       f32x16 acc = {};
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) acc = emfma(qa[ks], *reinterpret_cast<const ev8*>(kp + 16 * ks), acc);
+      for (int ks = 0; ks < 8; ++ks)
+        if (ks < nks) acc = emfma(qa[ks], *reinterpret_cast<const ev8*>(kp + 16 * ks), acc);
       const int col = ct * 32 + lq;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -531,6 +534,7 @@ struct PspArgs {
   float* lse2;            // [BH, Lr_pad]
   float* scores;          // [bh_count, NB, NB]
   int NB, R, Lr, Lr_pad, bh0, row_norm;
+  int ld;  // columns of a stored row
   float scale_log2;
 };
 
@@ -553,24 +557,26 @@ __global__ __launch_bounds__(256) void psp_kernel(PspArgs a) {
   const int rg = wv & 1, kh = wv >> 1;
   const int qrow = qt * 64 + 32 * rg + lq;
   const bool qvalid = group_valid(a, qrow);
-  const e16_t* kbase = a.kr + bh * a.Lr_pad * HD;
-  const srd_t rk = make_srd(kbase, (unsigned)((size_t)a.Lr_pad * HD * 2));
+  const int ld = a.ld;
+  const e16_t* kbase = a.kr + bh * a.Lr_pad * ld;
+  const srd_t rk = make_srd(kbase, (unsigned)((size_t)a.Lr_pad * ld * 2));
   unsigned ld_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int P = (wv * 4 + i) * 64 + l, R = P >> 4;
-    ld_off[i] = (unsigned)R * 256 + (unsigned)(((P & 15) ^ swz(R)) * 16);
+    const int g = (P & 15) ^ swz(R);  // (chunks past a stored row land as zeros)
+    ld_off[i] = g * 8 < ld ? (unsigned)(R * ld * 2 + g * 16) : 0x80000000u;
   }
   auto issue = [&](int c, int sb) -> float {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(rk, k_s[sb] + wv * 4096 + i * 1024, ld_off[i], (unsigned)c * (BK * 256));
+    for (int i = 0; i < 4; ++i) dma16(rk, k_s[sb] + wv * 4096 + i * 1024, ld_off[i], (unsigned)(c * BK * ld * 2));
     return group_valid(a, c * 64 + l) ? 0.0f : -INFINITY;
   };
   ev8 qreg[8];
   {
-    const e16_t* qp = a.qr + (bh * a.Lr_pad + qrow) * HD + 8 * hi;
+    const e16_t* qp = a.qr + (bh * a.Lr_pad + qrow) * ld + 8 * hi;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qreg[ks] = *reinterpret_cast<const ev8*>(qp + 16 * ks);
+    for (int ks = 0; ks < 8; ++ks) qreg[ks] = 16 * ks < ld ? *reinterpret_cast<const ev8*>(qp + 16 * ks) : ev8{};
   }
   int koff[8];
 #pragma unroll
@@ -770,7 +776,10 @@ static int rows_common(const void* qc, const void* kc, const void* scores_in, vo
   a.NBc_pad = NBc_pad;
   a.bh0 = bh0;
   a.W = (NB + 31) / 32;
-  a.scale = 1.0f / sqrtf((float)D);  // D: the logical head dimension (64 or 128)
+  HeadDim h;
+  head_dim(D, h);
+  a.ld = h.ld;
+  a.scale = 1.0f / sqrtf((float)h.d);
   if (K < 0) {  // scores only
     a.K = -1;
     rows_launch<false>(a, bh_count, stream);
@@ -804,7 +813,8 @@ static int rows_common(const void* qc, const void* kc, const void* scores_in, vo
 extern "C" int ES_VSA_API(vsa_block_scores)(const void* qc, const void* kc, void* scores, int NB, int NBc_pad, int bh0,
                                 int bh_count, int D, hipStream_t stream) {
   ES_REQUIRE(qc && kc && scores, ES_ERR_INVALID, "VSA: null tensor pointer");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE(NBc_pad == (NB + 63) / 64 * 64, ES_ERR_INVALID, "qc must hold ceil(nb/64)*64 pooled rows");
   return rows_common(qc, kc, nullptr, scores, NB, NBc_pad, bh0, bh_count, -1, nullptr, nullptr, nullptr, nullptr,
                      nullptr, 0, D, stream, "vsa_block_scores");
@@ -814,7 +824,8 @@ extern "C" int ES_VSA_API(vsa_route_rows)(const void* qc, const void* kc, int NB
                               int D, int* q2k_ptr, int* q2k_idx, int* k2q_ptr, int* k2q_idx, void* workspace,
                               size_t workspace_bytes, hipStream_t stream) {
   ES_REQUIRE(qc && kc, ES_ERR_INVALID, "VSA: null tensor pointer");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE(NBc_pad == (NB + 63) / 64 * 64, ES_ERR_INVALID, "qc must hold ceil(nb/64)*64 pooled rows");
   ES_REQUIRE(K >= 0 && K <= NB, ES_ERR_INVALID, "VSA: K must be in [0, NB]");
   return rows_common(qc, kc, nullptr, nullptr, NB, NBc_pad, bh0, bh_count, K, q2k_ptr, q2k_idx, k2q_ptr, k2q_idx,
@@ -882,7 +893,8 @@ static void launch_psp(const PspArgs& a, bool scores, int bh_count, hipStream_t 
 static int psp(const void* qr, const void* kr, const int* blk_cnt, float* lse2, float* scores, int NB, int R,
                int row_norm, int bh0, int bh_count, int D, bool do_scores, hipStream_t stream, const char* what) {
   ES_REQUIRE(qr && kr && blk_cnt && lse2 && (!do_scores || scores), ES_ERR_INVALID, "VSA: null tensor pointer");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE(R == 4 || R == 8 || R == 16 || R == 32, ES_ERR_INVALID, "VSA2: router pool size R must be 4, 8, 16 or 32");
   ES_REQUIRE(row_norm == 0 || row_norm == 1, ES_ERR_INVALID, "VSA2: row_norm must be 0 (valid_groups) or 1 (paper)");
   ES_REQUIRE(NB >= 1 && bh0 >= 0 && bh_count >= 1 && bh_count <= 65535, ES_ERR_INVALID, "VSA: bad (b,h) range");
@@ -899,7 +911,8 @@ static int psp(const void* qr, const void* kr, const int* blk_cnt, float* lse2, 
   a.Lr_pad = (NB * G + 63) / 64 * 64;
   a.bh0 = bh0;
   a.row_norm = row_norm;
-  a.scale_log2 = LOG2E / sqrtf((float)D);
+  a.ld = h.ld;
+  a.scale_log2 = LOG2E / sqrtf((float)h.d);
   ES_REQUIRE((size_t)a.Lr_pad * HD * 2 < (1ull << 31), ES_ERR_UNSUPPORTED, "VSA2: pooled rows exceed 2 GiB");
   switch (G) {
     case 2: launch_psp<2>(a, do_scores, bh_count, stream); break;

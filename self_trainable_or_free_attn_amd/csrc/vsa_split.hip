@@ -140,11 +140,12 @@ __global__ __launch_bounds__(256) void merge_fwd_kernel(const float* __restrict_
                                                         const float* __restrict__ part_lse,
                                                         const int4* __restrict__ merges, const int* __restrict__ info,
                                                         const int* __restrict__ blk_cnt, e16_t* __restrict__ o,
-                                                        float* __restrict__ lse, int L, int NB, int mask_rows) {
+                                                        float* __restrict__ lse, int L, int NB, int ld, int mask_rows) {
   if ((int)blockIdx.x >= info[1]) return;
   const int4 mg = merges[blockIdx.x];
   const int bh = mg.x / NB, qb = mg.x - bh * NB, slot0 = mg.y, c = mg.z;
   const int row = threadIdx.x >> 2, c0 = (threadIdx.x & 3) * 32;
+  if (c0 >= ld) return;  // (rows of ld columns)
   const size_t tok = (size_t)bh * L + (size_t)qb * BK + row;
   float acc[32];
 #pragma unroll
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(256) void merge_fwd_kernel(const float* __restrict_
       float sum = 0.0f;
       for (int j = 0; j < c; ++j) {
         const float w = exp2f(part_lse[(size_t)(slot0 + j) * BK + row] - mx);
-        const f32x4* src = reinterpret_cast<const f32x4*>(part_o + ((size_t)(slot0 + j) * BK + row) * HD + c0);
+        const f32x4* src = reinterpret_cast<const f32x4*>(part_o + ((size_t)(slot0 + j) * BK + row) * ld + c0);
         sum += w;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(256) void merge_fwd_kernel(const float* __restrict_
       out_lse = (mx + log2f(sum)) * 0.6931471805599453f;
     }
   }
-  uint4* dst = reinterpret_cast<uint4*>(o + tok * HD + c0);
+  uint4* dst = reinterpret_cast<uint4*>(o + tok * ld + c0);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     uint4 u;
@@ -189,11 +190,12 @@ __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict_
                                                         const int* __restrict__ info, const float* __restrict__ add,
                                                         int add_nb, const int* __restrict__ blk_cnt,
                                                         e16_t* __restrict__ out, float* __restrict__ out_f32, int L,
-                                                        int NB) {
+                                                        int NB, int ld) {
   if ((int)blockIdx.x >= info[1]) return;
   const int4 mg = merges[blockIdx.x];
   const int bh = mg.x / NB, blk = mg.x - bh * NB, slot0 = mg.y, c = mg.z;
   const int row = threadIdx.x >> 2, c0 = (threadIdx.x & 3) * 32;
+  if (c0 >= ld) return;  // (rows of ld columns)
   const size_t tok = (size_t)bh * L + (size_t)blk * BK + row;
   const int cnt = blk_cnt[blk];
   float acc[32];
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict_
   for (int e = 0; e < 32; ++e) acc[e] = 0.0f;
   if (row < cnt) {
     for (int j = 0; j < c; ++j) {
-      const f32x4* src = reinterpret_cast<const f32x4*>(part + ((size_t)(slot0 + j) * BK + row) * HD + c0);
+      const f32x4* src = reinterpret_cast<const f32x4*>(part + ((size_t)(slot0 + j) * BK + row) * ld + c0);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const f32x4 x = src[q];
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict_
     }
     if (add != nullptr) {
       const float inv = 1.0f / (float)cnt;
-      const f32x4* ad = reinterpret_cast<const f32x4*>(add + ((size_t)bh * add_nb + blk) * HD + c0);
+      const f32x4* ad = reinterpret_cast<const f32x4*>(add + ((size_t)bh * add_nb + blk) * ld + c0);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const f32x4 x = ad[q];
@@ -221,11 +223,11 @@ __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict_
     }
   }
   if (out_f32 != nullptr) {
-    f32x4* dst = reinterpret_cast<f32x4*>(out_f32 + tok * HD + c0);
+    f32x4* dst = reinterpret_cast<f32x4*>(out_f32 + tok * ld + c0);
 #pragma unroll
     for (int q = 0; q < 8; ++q) dst[q] = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
   } else {
-    uint4* dst = reinterpret_cast<uint4*>(out + tok * HD + c0);
+    uint4* dst = reinterpret_cast<uint4*>(out + tok * ld + c0);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       uint4 u;
@@ -275,23 +277,25 @@ extern "C" int vsa_split_plan(const int* ptr, int BH, int NB, int chunk, int max
 extern "C" int ES_VSA_API(vsa_split_merge_fwd)(const float* part_o, const float* part_lse, const int* merges, const int* info,
                                    int max_merges, const int* blk_cnt, void* o, float* lse, int BH, int L, int D,
                                    int mask_rows, hipStream_t stream) {
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE(BH >= 1 && L > 0 && L % BK == 0, ES_ERR_INVALID, "o must be [B,H,L,D]");
   if (max_merges <= 0) return ES_OK;
   ES_REQUIRE(part_o && part_lse && merges && info && blk_cnt && o && lse, ES_ERR_INVALID, "VSA2: null tensor pointer");
   hipLaunchKernelGGL(merge_fwd_kernel, dim3(max_merges), dim3(256), 0, stream, part_o, part_lse, (const int4*)merges,
-                     info, blk_cnt, (e16_t*)o, lse, L, L / BK, mask_rows);
+                     info, blk_cnt, (e16_t*)o, lse, L, L / BK, h.ld, mask_rows);
   return check_launch("vsa_split_merge_fwd");
 }
 
 extern "C" int ES_VSA_API(vsa_split_merge_sum)(const float* part, const int* merges, const int* info, int max_merges,
                                    const float* add, int add_nb, const int* blk_cnt, void* out, float* out_f32, int BH,
                                    int L, int D, hipStream_t stream) {
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
   ES_REQUIRE(BH >= 1 && L > 0 && L % BK == 0, ES_ERR_INVALID, "out must be [B,H,L,D]");
   if (max_merges <= 0) return ES_OK;
   ES_REQUIRE(part && merges && info && blk_cnt && (out || out_f32), ES_ERR_INVALID, "VSA2: null tensor pointer");
   hipLaunchKernelGGL(merge_sum_kernel, dim3(max_merges), dim3(256), 0, stream, part, (const int4*)merges, info, add,
-                     add_nb, blk_cnt, (e16_t*)out, out_f32, L, L / BK);
+                     add_nb, blk_cnt, (e16_t*)out, out_f32, L, L / BK, h.ld);
   return check_launch("vsa_split_merge_sum");
 }

@@ -18,7 +18,8 @@ import torch.nn.functional as F
 from .. import _lib
 
 BLOCK = 64
-HD = 128                # columns of every token row handed to the C ABI
+HD = 128                # the widest token row; the three-tier entry points store every row this wide
+VSA_PACKED_ROWS = 0x10000   # flag of the entry points' D: rows are stored D columns wide (include/vsa_hip.h)
 _FWD_VARIANT = [0]
 
 
@@ -56,9 +57,10 @@ def _f32(x, name):
 
 
 def _wide(x):
-    """x with its last dim zero-padded to 128 columns (x itself when already 128 wide, or None). The C ABI stores
-    every row with 128 columns and takes the logical head dim D (64 or 128) separately: zero columns add exact zeros
-    to every dot product, and every output column past D comes out zero, so narrowing back loses nothing."""
+    """x with its last dim zero-padded to 128 columns (x itself when already 128 wide, or None). The three-tier entry
+    points store every row with 128 columns and take the logical head dim D (64 or 128) separately: zero columns add
+    exact zeros to every dot product, and every output column past D comes out zero, so narrowing back loses
+    nothing. (The others take D = 64 rows as they are stored: `_rows`.)"""
     if x is None or x.shape[-1] == HD:
         return x
     return F.pad(x, (0, HD - x.shape[-1])).contiguous()
@@ -66,6 +68,37 @@ def _wide(x):
 
 def _narrow(x, D):
     return x if x is None or D == HD else x[..., :D].contiguous()
+
+
+def _dim(D):
+    """The D argument of the entry points that take rows stored D columns wide."""
+    return D if D == HD else D | VSA_PACKED_ROWS
+
+
+def _rows(x, D):
+    """x as rows stored D columns wide (None stays None). At D = 64 a tensor in any layout is taken: one that is not
+    contiguous or not 16-byte aligned is copied first. A width other than D is narrowed, or zero-padded at D = 128."""
+    if x is None:
+        return None
+    if D == HD:
+        return _wide(x)
+    if x.shape[-1] != D:
+        x = x[..., :D]
+    plain = type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling()
+    at = x.data_ptr() if plain else x.storage_offset() * x.element_size()
+    return x if x.is_contiguous() and at % 16 == 0 else x.clone(memory_format=torch.contiguous_format)
+
+
+class _InRows:
+    """`_rows` of an in-place argument; put() writes a copy's columns back (zeros past D)."""
+
+    def __init__(self, x, D):
+        self.x, self.w = x, _rows(x, D)
+
+    def put(self):
+        if self.w is not self.x:
+            w = self.x.shape[-1]
+            self.x.copy_(self.w[..., :w] if w <= self.w.shape[-1] else _wide(self.w))
 
 
 class _InPlace:
@@ -114,12 +147,13 @@ def pool_fwd(q, k, v, blk_cnt, R):
     NB = L // BLOCK
     _check(blk_cnt.numel() == NB, "blk_cnt must have L/64 entries")
     G = BLOCK // R
-    qr = torch.empty(B, H, _ceil64(NB * G), HD, device=q.device, dtype=q.dtype)
+    qr = torch.empty(B, H, _ceil64(NB * G), D, device=q.device, dtype=q.dtype)
     kr = torch.empty_like(qr)
-    qc = torch.empty(B, H, _ceil64(NB), HD, device=q.device, dtype=q.dtype)
+    qc = torch.empty(B, H, _ceil64(NB), D, device=q.device, dtype=q.dtype)
     kc, vc = torch.empty_like(qc), torch.empty_like(qc)
-    _call("vsa_pool", _wide(q), _wide(k), _wide(v), blk_cnt, qr, kr, None, qc, kc, vc, B * H, L, D, int(R))
-    return [_narrow(t, D) for t in (qr, kr, qc, kc, vc)]
+    _call("vsa_pool", _rows(q, D), _rows(k, D), _rows(v, D), blk_cnt, qr, kr, None, qc, kc, vc, B * H, L, _dim(D),
+          int(R))
+    return [qr, kr, qc, kc, vc]
 
 
 def fuse_fwd(of, oc, gate, blk_cnt, gate_act):
@@ -135,10 +169,11 @@ def fuse_fwd(of, oc, gate, blk_cnt, gate_act):
             mode = 2
         else:
             raise RuntimeError("gate must be [B, H, L] or [B, H, L, D]")
-    o = torch.empty(B, H, L, HD, device=of.device, dtype=of.dtype)
-    _call("vsa_fuse_fwd", _wide(of), _wide(oc), _wide(gate) if mode == 2 else gate, o, blk_cnt, B * H, L, D,
+    o = torch.empty(B, H, L, D, device=of.device, dtype=of.dtype)
+    _call("vsa_fuse_fwd", _rows(of, D), _rows(oc, D), _rows(gate, D) if mode == 2 else gate, o, blk_cnt, B * H, L,
+              _dim(D),
               oc.shape[2], mode, int(gate_act))
-    return _narrow(o, D)
+    return o
 
 
 def fuse_bwd(dout, of, oc, gate, blk_cnt, gate_act, write_dout_f=True):
@@ -146,24 +181,24 @@ def fuse_bwd(dout, of, oc, gate, blk_cnt, gate_act, write_dout_f=True):
     _tokens(dout, "dout")
     B, H, L, D = dout.shape
     mode = 0 if gate is None else (1 if gate.dim() == 3 else 2)
-    dout_f = torch.empty(B, H, L, HD, device=dout.device, dtype=dout.dtype) if write_dout_f else None
+    dout_f = torch.empty(B, H, L, D, device=dout.device, dtype=dout.dtype) if write_dout_f else None
     delta_f = torch.empty(B, H, L, device=dout.device, dtype=torch.float32)
-    dout_c = torch.empty(B, H, oc.shape[2], HD, device=dout.device, dtype=dout.dtype)
+    dout_c = torch.empty(B, H, oc.shape[2], D, device=dout.device, dtype=dout.dtype)
     delta_c = torch.empty(B, H, oc.shape[2], device=dout.device, dtype=torch.float32)
-    gate_w = _wide(gate) if mode == 2 else gate
+    gate_w = _rows(gate, D) if mode == 2 else gate
     dgate = torch.empty_like(gate_w) if gate is not None else None
-    _call("vsa_fuse_bwd", _wide(dout), _wide(of), _wide(oc), gate_w, dout_f, delta_f, dout_c,
-              delta_c, dgate, blk_cnt, B * H, L, D, oc.shape[2], mode, int(gate_act))
-    return _narrow(dout_f, D), delta_f, _narrow(dout_c, D), delta_c, _narrow(dgate, D) if mode == 2 else dgate
+    _call("vsa_fuse_bwd", _rows(dout, D), _rows(of, D), _rows(oc, D), gate_w, dout_f, delta_f, dout_c,
+              delta_c, dgate, blk_cnt, B * H, L, _dim(D), oc.shape[2], mode, int(gate_act))
+    return dout_f, delta_f, dout_c, delta_c, dgate
 
 
 def finalize(acc, add, blk_cnt, like):
     """valid ? acc + add[blk] / cnt : 0 in like's dtype (reference fuse.cu:9)."""
     B, H, L, D = like.shape
-    out = torch.empty(B, H, L, HD, dtype=like.dtype, device=blk_cnt.device)
+    out = torch.empty(B, H, L, D, dtype=like.dtype, device=blk_cnt.device)
     add_nb = add.shape[2] if add is not None else 0
-    _call("vsa_finalize", _wide(acc), _wide(add), add_nb, out, blk_cnt, B * H, L, D)
-    return _narrow(out, D)
+    _call("vsa_finalize", _rows(acc, D), _rows(add, D), add_nb, out, blk_cnt, B * H, L, _dim(D))
+    return out
 
 
 # ------------------------------------------------------------------ routers
@@ -185,8 +220,9 @@ def block_scores(qc, kc, nb, bh0=0, bh_count=0):
         bh_count = BH - bh0
     _check(bh0 >= 0 and bh_count <= 65535 and bh0 + bh_count <= BH, "bad (b,h) range")
     scores = torch.empty(bh_count, nb, nb, device=qc.device, dtype=qc.dtype)
-    _call("vsa_block_scores", _wide(qc), _wide(kc), scores, int(nb), qc.shape[2], int(bh0), int(bh_count),
-              qc.shape[3])
+    D = qc.shape[3]
+    _call("vsa_block_scores", _rows(qc, D), _rows(kc, D), scores, int(nb), qc.shape[2], int(bh0), int(bh_count),
+              _dim(D))
     return scores
 
 
@@ -220,10 +256,11 @@ def route_rows(qc, kc, nb, topk, max_score_bytes=2 << 30):
     out = _csr(B, H, NB, BH * NB * K, qc.device)
     chunk = min(BH, 65535)
     ws = _workspace(chunk, NB, qc.device)
-    D, qc, kc = qc.shape[3], _wide(qc), _wide(kc)
+    D = qc.shape[3]
+    qc, kc = _rows(qc, D), _rows(kc, D)
     for bh0 in range(0, BH, chunk):
         cnt = min(chunk, BH - bh0)
-        _call("vsa_route_rows", qc, kc, NB, qc.shape[2], bh0, cnt, K, D, *out, ws, ws.numel())
+        _call("vsa_route_rows", qc, kc, NB, qc.shape[2], bh0, cnt, K, _dim(D), *out, ws, ws.numel())
     return list(out)
 
 
@@ -231,7 +268,7 @@ def router_lse(qr, kr, blk_cnt, R):
     """lse2 [B, H, Lr_pad] of every pooled query row (reference vsa2_api.cpp:122-135)."""
     B, H, Lr_pad, D = qr.shape
     lse2 = torch.empty(B, H, Lr_pad, device=qr.device, dtype=torch.float32)
-    _call("vsa_router_lse", _wide(qr), _wide(kr), blk_cnt, lse2, blk_cnt.numel(), int(R), B * H, D)
+    _call("vsa_router_lse", _rows(qr, D), _rows(kr, D), blk_cnt, lse2, blk_cnt.numel(), int(R), B * H, _dim(D))
     return lse2
 
 
@@ -242,7 +279,8 @@ def router_scores(qr, kr, lse2, blk_cnt, R, row_norm, bh0=0, bh_count=0):
     if bh_count <= 0:
         bh_count = B * H - bh0
     scores = torch.empty(bh_count, NB, NB, device=qr.device, dtype=torch.float32)
-    _call("vsa_router_scores", _wide(qr), _wide(kr), lse2, blk_cnt, scores, NB, int(R), int(row_norm), int(bh0), int(bh_count), D)
+    _call("vsa_router_scores", _rows(qr, D), _rows(kr, D), lse2, blk_cnt, scores, NB, int(R), int(row_norm),
+          int(bh0), int(bh_count), _dim(D))
     return scores
 
 
@@ -268,14 +306,15 @@ def route(qr, kr, blk_cnt, R, budget, row_norm, max_score_bytes=2 << 30):
     _check(BH * keff < 2 ** 31, "VSA2: total selected blocks exceed int32 CSR range")
     out = _csr(B, H, NB, BH * keff, qr.device)
     lse2 = router_lse(qr, kr, blk_cnt, R)
-    D, qr, kr = qr.shape[3], _wide(qr), _wide(kr)
+    D = qr.shape[3]
+    qr, kr = _rows(qr, D), _rows(kr, D)
     chunk = int(max(1, min(BH, int(max_score_bytes) // max(nn * 4, 1), 65535)))
     ws = _workspace(chunk, NB, qr.device)
     scores = torch.empty(chunk, NB, NB, device=qr.device, dtype=torch.float32)
     for bh0 in range(0, BH, chunk):
         cnt = min(chunk, BH - bh0)
         s = scores[:cnt]
-        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, D)
+        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, _dim(D))
         _call("vsa_global_topk", s, NB, bh0, cnt, int(budget), *out, None, ws, ws.numel())
     return list(out)
 
@@ -310,10 +349,10 @@ def attn_fwd(q, k, v, row_ptr, col_idx, blk_cnt, use_tk=False):
     _i32(col_idx, "col_idx")
     B, H, L, D = q.shape
     _check(row_ptr.numel() == B * H * (L // BLOCK + 1), "metadata shape mismatch")
-    o = torch.empty(B, H, L, HD, device=q.device, dtype=q.dtype)
+    o = torch.empty(B, H, L, D, device=q.device, dtype=q.dtype)
     lse = torch.empty(B, H, L, device=q.device, dtype=torch.float32)
-    _call("vsa_attn_fwd", _wide(q), _wide(k), _wide(v), row_ptr, col_idx, blk_cnt, o, lse, B * H, L, D)
-    return _narrow(o, D), lse
+    _call("vsa_attn_fwd", _rows(q, D), _rows(k, D), _rows(v, D), row_ptr, col_idx, blk_cnt, o, lse, B * H, L, _dim(D))
+    return o, lse
 
 
 def attn_bwd(q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, dq_acc=None, add_dk=None, add_dv=None,
@@ -324,28 +363,28 @@ def attn_bwd(q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, dq_acc=None, 
     if dq_acc is not None:
         _check(dq_acc.dtype == torch.float32 and dq_acc.shape == q.shape, "dq_acc must be fp32 like q")
     f = dict(device=q.device, dtype=torch.float32) if out_fp32 else dict(device=q.device, dtype=q.dtype)
-    dk, dv = torch.empty(B, H, L, HD, **f), torch.empty(B, H, L, HD, **f)
+    dk, dv = torch.empty(B, H, L, D, **f), torch.empty(B, H, L, D, **f)
     add_nb = add_dk.shape[2] if add_dk is not None else (add_dv.shape[2] if add_dv is not None else 0)
-    q, k, v, dout = _wide(q), _wide(k), _wide(v), _wide(dout)
-    _call("vsa_attn_bwd_kv", q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, _wide(add_dk), _wide(add_dv),
-              add_nb, dk, dv, 1 if out_fp32 else 0, B * H, L, D)
+    q, k, v, dout = _rows(q, D), _rows(k, D), _rows(v, D), _rows(dout, D)
+    _call("vsa_attn_bwd_kv", q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, _rows(add_dk, D), _rows(add_dv, D),
+              add_nb, dk, dv, 1 if out_fp32 else 0, B * H, L, _dim(D))
     if dq_acc is not None:
         q2k_ptr, q2k_idx = csr_transpose(row_ptr, col_idx)
-        acc = _InPlace(dq_acc)
+        acc = _InRows(dq_acc, D)
         _call("vsa_attn_bwd_q", q, k, v, dout, lse, delta, q2k_ptr, q2k_idx, blk_cnt, None, 0, None, acc.w,
-                  B * H, L, D)
+                  B * H, L, _dim(D))
         acc.put()
-    return _narrow(dk, D), _narrow(dv, D)
+    return dk, dv
 
 
 def attn_bwd_q(q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, add_dq=None):
     """dQ over the q2k CSR without atomics, + add_dq / cnt (reference vsa2_api.cpp:419-457)."""
     _attn_args(q, k, v, blk_cnt)
     B, H, L, D = q.shape
-    dq = torch.empty(B, H, L, HD, device=q.device, dtype=q.dtype)
-    _call("vsa_attn_bwd_q", _wide(q), _wide(k), _wide(v), _wide(dout), lse, delta, row_ptr, col_idx, blk_cnt,
-              _wide(add_dq), add_dq.shape[2] if add_dq is not None else 0, dq, None, B * H, L, D)
-    return _narrow(dq, D)
+    dq = torch.empty(B, H, L, D, device=q.device, dtype=q.dtype)
+    _call("vsa_attn_bwd_q", _rows(q, D), _rows(k, D), _rows(v, D), _rows(dout, D), lse, delta, row_ptr, col_idx,
+              blk_cnt, _rows(add_dq, D), add_dq.shape[2] if add_dq is not None else 0, dq, None, B * H, L, _dim(D))
+    return dq
 
 
 # ------------------------------------------------------------------ split-KV
@@ -373,13 +412,13 @@ def attn_fwd_tasks(q, k, v, col_idx, blk_cnt, tasks, info, part_o, part_lse):
     _attn_args(q, k, v, blk_cnt)
     B, H, L, D = q.shape
     _check(part_lse.numel() == part_o.numel() // D, "part_lse must be [slots, 64]")
-    o = torch.empty(B, H, L, HD, device=q.device, dtype=q.dtype)
+    o = torch.empty(B, H, L, D, device=q.device, dtype=q.dtype)
     lse = torch.empty(B, H, L, device=q.device, dtype=torch.float32)
-    po = _InPlace(part_o if part_o.numel() else None)
-    _call("vsa_attn_fwd_tasks", _wide(q), _wide(k), _wide(v), col_idx, blk_cnt, tasks, info, tasks.shape[0], o,
-              lse, po.w, part_lse if part_lse.numel() else None, B * H, L, D)
+    po = _InRows(part_o if part_o.numel() else None, D)
+    _call("vsa_attn_fwd_tasks", _rows(q, D), _rows(k, D), _rows(v, D), col_idx, blk_cnt, tasks, info, tasks.shape[0], o,
+              lse, po.w, part_lse if part_lse.numel() else None, B * H, L, _dim(D))
     po.put()
-    return _narrow(o, D), lse
+    return o, lse
 
 
 def split_merge_fwd(part_o, part_lse, merges, info, blk_cnt, o, lse, mask_rows=True):
@@ -387,9 +426,9 @@ def split_merge_fwd(part_o, part_lse, merges, info, blk_cnt, o, lse, mask_rows=T
     if part_o.numel() == 0:
         return
     B, H, L, D = o.shape
-    ow = _InPlace(o)
-    _call("vsa_split_merge_fwd", _wide(part_o), part_lse, merges, info, merges.shape[0], blk_cnt, ow.w, lse,
-              B * H, L, D, 1 if mask_rows else 0)
+    ow = _InRows(o, D)
+    _call("vsa_split_merge_fwd", _rows(part_o, D), part_lse, merges, info, merges.shape[0], blk_cnt, ow.w, lse,
+              B * H, L, _dim(D), 1 if mask_rows else 0)
     ow.put()
 
 
@@ -399,10 +438,10 @@ def split_merge_sum(part, merges, info, add, blk_cnt, out):
         return
     B, H, L, D = out.shape
     f32 = out.dtype == torch.float32
-    ow = _InPlace(out)
-    _call("vsa_split_merge_sum", _wide(part), merges, info, merges.shape[0], _wide(add),
+    ow = _InRows(out, D)
+    _call("vsa_split_merge_sum", _rows(part, D), merges, info, merges.shape[0], _rows(add, D),
               add.shape[2] if add is not None else 0, blk_cnt, None if f32 else ow.w, ow.w if f32 else None,
-              B * H, L, D)
+              B * H, L, _dim(D))
     ow.put()
 
 
@@ -414,27 +453,28 @@ def attn_bwd_tasks(q, k, v, dout, lse, delta, col_idx, blk_cnt, tasks, info, dq_
     _check(dq_acc is None, "attn_bwd_tasks: dQ comes from attn_bwd_q_tasks on this build (no atomics)")
     _attn_args(q, k, v, blk_cnt)
     B, H, L, D = q.shape
-    dk = torch.empty(B, H, L, HD, device=q.device, dtype=q.dtype)
+    dk = torch.empty(B, H, L, D, device=q.device, dtype=q.dtype)
     dv = torch.empty_like(dk)
     add_nb = add_dk.shape[2] if add_dk is not None else (add_dv.shape[2] if add_dv is not None else 0)
-    pk, pv = _InPlace(part_dk if part_dk.numel() else None), _InPlace(part_dv if part_dv.numel() else None)
-    _call("vsa_attn_bwd_kv_tasks", _wide(q), _wide(k), _wide(v), _wide(dout), lse, delta, col_idx, blk_cnt, tasks,
-              info, tasks.shape[0], _wide(add_dk), _wide(add_dv), add_nb, dk, dv, pk.w, pv.w, B * H, L, D)
+    pk, pv = _InRows(part_dk if part_dk.numel() else None, D), _InRows(part_dv if part_dv.numel() else None, D)
+    _call("vsa_attn_bwd_kv_tasks", _rows(q, D), _rows(k, D), _rows(v, D), _rows(dout, D), lse, delta, col_idx, blk_cnt,
+              tasks, info, tasks.shape[0], _rows(add_dk, D), _rows(add_dv, D), add_nb, dk, dv, pk.w, pv.w, B * H, L, _dim(D))
     pk.put()
     pv.put()
-    return _narrow(dk, D), _narrow(dv, D)
+    return dk, dv
 
 
 def attn_bwd_q_tasks(q, k, v, dout, lse, delta, col_idx, blk_cnt, tasks, info, add_dq, part_dq):
     """dQ of direct q2k tasks; split chunks fill part_dq (reference vsa2_api.cpp:687-730)."""
     _attn_args(q, k, v, blk_cnt)
     B, H, L, D = q.shape
-    dq = torch.empty(B, H, L, HD, device=q.device, dtype=q.dtype)
-    pq = _InPlace(part_dq if part_dq.numel() else None)
-    _call("vsa_attn_bwd_q_tasks", _wide(q), _wide(k), _wide(v), _wide(dout), lse, delta, col_idx, blk_cnt, tasks,
-              info, tasks.shape[0], _wide(add_dq), add_dq.shape[2] if add_dq is not None else 0, dq, pq.w, B * H, L, D)
+    dq = torch.empty(B, H, L, D, device=q.device, dtype=q.dtype)
+    pq = _InRows(part_dq if part_dq.numel() else None, D)
+    _call("vsa_attn_bwd_q_tasks", _rows(q, D), _rows(k, D), _rows(v, D), _rows(dout, D), lse, delta, col_idx, blk_cnt,
+              tasks, info, tasks.shape[0], _rows(add_dq, D), add_dq.shape[2] if add_dq is not None else 0, dq, pq.w,
+              B * H, L, _dim(D))
     pq.put()
-    return _narrow(dq, D)
+    return dq
 
 
 def attn_bwd_q_acc(q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, dq_acc):
@@ -442,9 +482,9 @@ def attn_bwd_q_acc(q, k, v, dout, lse, delta, row_ptr, col_idx, blk_cnt, dq_acc)
     _attn_args(q, k, v, blk_cnt)
     _f32(dq_acc, "dq_acc")
     B, H, L, D = q.shape
-    acc = _InPlace(dq_acc)
-    _call("vsa_attn_bwd_q", _wide(q), _wide(k), _wide(v), _wide(dout), lse, delta, row_ptr, col_idx, blk_cnt, None,
-              0, None, acc.w, B * H, L, D)
+    acc = _InRows(dq_acc, D)
+    _call("vsa_attn_bwd_q", _rows(q, D), _rows(k, D), _rows(v, D), _rows(dout, D), lse, delta, row_ptr, col_idx,
+              blk_cnt, None, 0, None, acc.w, B * H, L, _dim(D))
     acc.put()
     return dq_acc
 
@@ -511,13 +551,14 @@ def route_tier_rows(qr, kr, blk_cnt, R, ka, kab, row_norm, max_score_bytes=2 << 
     bits_a = torch.zeros(B, H, NB, W, **i32)
     bits_ab = torch.zeros(B, H, NB, W, **i32)
     lse2 = router_lse(qr, kr, blk_cnt, R)
-    D, qr, kr = qr.shape[3], _wide(qr), _wide(kr)
+    D = qr.shape[3]
+    qr, kr = _rows(qr, D), _rows(kr, D)
     chunk = int(max(1, min(BH, int(max_score_bytes) // max(NB * NB * 4, 1), 65535)))
     scores = torch.empty(chunk, NB, NB, device=dev, dtype=torch.float32)
     for bh0 in range(0, BH, chunk):
         cnt = min(chunk, BH - bh0)
         s = scores[:cnt]
-        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, D)
+        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, _dim(D))
         _call("vsa_row_tiers", s, NB, bh0, cnt, ka, kab, a_ptr, a_idx, ab_ptr, ab_idx, bits_a, bits_ab)
     k2q_ptr, k2q_idx = csr_transpose(a_ptr, a_idx)
     b_ptr = torch.zeros(B, H, NB + 1, **i32)
@@ -545,14 +586,15 @@ def route_tiers(qr, kr, blk_cnt, R, budget_a, budget_ab, row_norm, max_score_byt
     bits_a = torch.zeros(B, H, NB, W, **i32)
     bits_ab = torch.zeros(B, H, NB, W, **i32)
     lse2 = router_lse(qr, kr, blk_cnt, R)
-    D, qr, kr = qr.shape[3], _wide(qr), _wide(kr)
+    D = qr.shape[3]
+    qr, kr = _rows(qr, D), _rows(kr, D)
     chunk = int(max(1, min(BH, int(max_score_bytes) // max(nn * 4, 1), 65535)))
     ws = _workspace(chunk, NB, dev)
     scores = torch.empty(chunk, NB, NB, device=dev, dtype=torch.float32)
     for bh0 in range(0, BH, chunk):
         cnt = min(chunk, BH - bh0)
         s = scores[:cnt]
-        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, D)
+        _call("vsa_router_scores", qr, kr, lse2, blk_cnt, s, NB, int(R), int(row_norm), bh0, cnt, _dim(D))
         if kab != ka:
             _call("vsa_global_topk", s, NB, bh0, cnt, kab, *ab_out, bits_ab, ws, ws.numel())
         _call("vsa_global_topk", s, NB, bh0, cnt, ka, *a_out, bits_a, ws, ws.numel())
