@@ -160,6 +160,11 @@ int vsa_global_topk(const float* scores, int NB, int bh0, int bh_count, long lon
 int vsa_csr_transpose(const int* ptr, const int* idx, int NB, int bh0, int bh_count, int* out_ptr, int* out_idx,
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* Dense lists over the T = ceil(NB / 64) 64-row tiles of a pooled sequence of NB rows: cnt [T] rows of each tile, ptr
+ * [BH, T + 1], idx [BH * T * T], every tile listing all T (the coarse branch's selection, which is its own transpose;
+ * the reference builds it with torch calls, echosparse/vsa/ops.py:436-446). */
+int vsa_dense_lists(int NB, int BH, int* cnt, int* ptr, int* idx, hipStream_t stream);
+
 /* ---------------------------------------------------------------- split-KV */
 
 /* Device-side task plan of a CSR list ptr [BH, NB + 1]: tasks [BH * NB + max_slots, 4], merges

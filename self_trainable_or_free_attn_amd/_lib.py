@@ -60,6 +60,7 @@ SIGNATURES = {
     "vsa_router_scores": [P, P, P, P, P, I, I, I, I, I, I],
     "vsa_global_topk": [P, I, I, I, LL, P, P, P, P, P, P, Z],
     "vsa_csr_transpose": [P, P, I, I, I, P, P, P, Z],
+    "vsa_dense_lists": [I, I, P, P, P],
     "vsa_split_plan": [P, I, I, I, I, I, DB, DB, I, I, P, P, P],
     "vsa_split_merge_fwd": [P, P, P, P, I, P, P, P, I, I, I, I],
     "vsa_split_merge_sum": [P, P, P, I, P, I, P, P, P, I, I, I],

@@ -350,6 +350,15 @@ static void op_vsa_csr_transpose(const c10::optional<at::Tensor>& ptr, const c10
 }
 static void meta_vsa_csr_transpose(const c10::optional<at::Tensor>& ptr, const c10::optional<at::Tensor>& idx, int64_t NB, int64_t bh0, int64_t bh_count, const c10::optional<at::Tensor>& out_ptr, const c10::optional<at::Tensor>& out_idx, const c10::optional<at::Tensor>& workspace, int64_t workspace_bytes) {}
 
+static void op_vsa_dense_lists(int64_t NB, int64_t BH, const c10::optional<at::Tensor>& cnt, const c10::optional<at::Tensor>& ptr, const c10::optional<at::Tensor>& idx) {
+  const Call es_op_call("vsa_dense_lists", {&cnt, &ptr, &idx});
+  c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
+  const hipStream_t es_op_stream =
+      es_op_call.dev ? c10::hip::getCurrentHIPStream(es_op_call.dev->index()).stream() : nullptr;
+  es_op_check("vsa_dense_lists", vsa_dense_lists(static_cast<int>(es_op_int("vsa_dense_lists", "NB", NB, ES_INT)), static_cast<int>(es_op_int("vsa_dense_lists", "BH", BH, ES_INT)), static_cast<int*>(es_op_data("vsa_dense_lists", "cnt", cnt, ES_I32)), static_cast<int*>(es_op_data("vsa_dense_lists", "ptr", ptr, ES_I32)), static_cast<int*>(es_op_data("vsa_dense_lists", "idx", idx, ES_I32)), es_op_stream));
+}
+static void meta_vsa_dense_lists(int64_t NB, int64_t BH, const c10::optional<at::Tensor>& cnt, const c10::optional<at::Tensor>& ptr, const c10::optional<at::Tensor>& idx) {}
+
 static void op_vsa_split_plan(const c10::optional<at::Tensor>& ptr, int64_t BH, int64_t NB, int64_t chunk, int64_t max_slots, int64_t min_len, double rel_mean, double tail_frac, int64_t resident, int64_t budget, const c10::optional<at::Tensor>& tasks, const c10::optional<at::Tensor>& merges, const c10::optional<at::Tensor>& info) {
   const Call es_op_call("vsa_split_plan", {&ptr, &tasks, &merges, &info});
   c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
@@ -706,6 +715,7 @@ TORCH_LIBRARY(echosparse_gfx950, m) {
   m.def("vsa_router_scores(Tensor? qr, Tensor? kr, Tensor? lse2, Tensor? blk_cnt, Tensor(a!)? scores, int NB, int R, int row_norm, int bh0, int bh_count, int D) -> ()");
   m.def("vsa_global_topk(Tensor? scores, int NB, int bh0, int bh_count, int budget, Tensor(a!)? q2k_ptr, Tensor(b!)? q2k_idx, Tensor(c!)? k2q_ptr, Tensor(d!)? k2q_idx, Tensor(e!)? bits_out, Tensor(f!)? workspace, int workspace_bytes) -> ()");
   m.def("vsa_csr_transpose(Tensor? ptr, Tensor? idx, int NB, int bh0, int bh_count, Tensor(a!)? out_ptr, Tensor(b!)? out_idx, Tensor(c!)? workspace, int workspace_bytes) -> ()");
+  m.def("vsa_dense_lists(int NB, int BH, Tensor(a!)? cnt, Tensor(b!)? ptr, Tensor(c!)? idx) -> ()");
   m.def("vsa_split_plan(Tensor? ptr, int BH, int NB, int chunk, int max_slots, int min_len, float rel_mean, float tail_frac, int resident, int budget, Tensor(a!)? tasks, Tensor(b!)? merges, Tensor(c!)? info) -> ()");
   m.def("vsa_split_merge_fwd(Tensor? part_o, Tensor? part_lse, Tensor? merges, Tensor? info, int max_merges, Tensor? blk_cnt, Tensor(a!)? o, Tensor(b!)? lse, int BH, int L, int D, int mask_rows) -> ()");
   m.def("vsa_split_merge_sum(Tensor? part, Tensor? merges, Tensor? info, int max_merges, Tensor? add, int add_nb, Tensor? blk_cnt, Tensor(a!)? out, Tensor(b!)? out_f32, int BH, int L, int D) -> ()");
@@ -775,6 +785,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CUDA, m) {
   m.impl("vsa_router_scores", TORCH_FN(op_vsa_router_scores));
   m.impl("vsa_global_topk", TORCH_FN(op_vsa_global_topk));
   m.impl("vsa_csr_transpose", TORCH_FN(op_vsa_csr_transpose));
+  m.impl("vsa_dense_lists", TORCH_FN(op_vsa_dense_lists));
   m.impl("vsa_split_plan", TORCH_FN(op_vsa_split_plan));
   m.impl("vsa_split_merge_fwd", TORCH_FN(op_vsa_split_merge_fwd));
   m.impl("vsa_split_merge_sum", TORCH_FN(op_vsa_split_merge_sum));
@@ -844,6 +855,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CPU, m) {
   m.impl("vsa_router_scores", TORCH_FN(op_vsa_router_scores));
   m.impl("vsa_global_topk", TORCH_FN(op_vsa_global_topk));
   m.impl("vsa_csr_transpose", TORCH_FN(op_vsa_csr_transpose));
+  m.impl("vsa_dense_lists", TORCH_FN(op_vsa_dense_lists));
   m.impl("vsa_split_plan", TORCH_FN(op_vsa_split_plan));
   m.impl("vsa_split_merge_fwd", TORCH_FN(op_vsa_split_merge_fwd));
   m.impl("vsa_split_merge_sum", TORCH_FN(op_vsa_split_merge_sum));
@@ -913,6 +925,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, Meta, m) {
   m.impl("vsa_router_scores", TORCH_FN(meta_vsa_router_scores));
   m.impl("vsa_global_topk", TORCH_FN(meta_vsa_global_topk));
   m.impl("vsa_csr_transpose", TORCH_FN(meta_vsa_csr_transpose));
+  m.impl("vsa_dense_lists", TORCH_FN(meta_vsa_dense_lists));
   m.impl("vsa_split_plan", TORCH_FN(meta_vsa_split_plan));
   m.impl("vsa_split_merge_fwd", TORCH_FN(meta_vsa_split_merge_fwd));
   m.impl("vsa_split_merge_sum", TORCH_FN(meta_vsa_split_merge_sum));

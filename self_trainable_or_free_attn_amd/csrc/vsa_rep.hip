@@ -856,7 +856,7 @@ extern "C" int ES_VSA_API(vsa_rep_bwd_tables)(const void* q, const void* dout, c
   a.BH = BH;
   const int per_queue = (BH + 7) / 8 * (a.rows_pad / BK);
   Queues qs;
-  ES_REQUIRE(balanced_launch_queues(per_queue, stream, qs), ES_ERR_LAUNCH, "VSA2-rep: row-group queues unavailable");
+  ES_REQUIRE(balanced_launch_queues(per_queue, stream, qs, 256), ES_ERR_LAUNCH, "VSA2-rep: row-group queues unavailable");
   a.queues = qs.counters;
   a.fixed = qs.fixed;
   hipLaunchKernelGGL(rep_bwd_tab_kernel, dim3((unsigned)qs.grid), dim3(512), 0, stream, a);

@@ -232,10 +232,20 @@ __global__ __launch_bounds__(256) void col_count_kernel(const unsigned* __restri
   }
 }
 
-// per (b, h): column j's groups get offsets base + (earlier columns) + (earlier groups of column j); base_of[b]
-// is the absolute offset of (b, h)'s first list
+// Absolute list base of (b, h) bh0 + bhl: the first entry of a given ptr (transpose), else (bh0 + bhl) * keff with keff
+// from the top-k state or given (routers).
+struct TopkState;
+struct ListBase {
+  const TopkState* st;
+  long long keff;
+  const int* src_ptr;
+  int bh0;
+  __device__ __forceinline__ long long of(int bhl, int NB) const;
+};
+
+// per (b, h): column j's groups get offsets base + (earlier columns) + (earlier groups of column j)
 __global__ __launch_bounds__(1024) void col_scan_kernel(int* __restrict__ gcnt, int* __restrict__ k2q_ptr, int NB,
-                                                        int bh0, const long long* __restrict__ base_of) {
+                                                        ListBase lists) {
   __shared__ int red[16];
   const int bhl = blockIdx.x, NG = (NB + ROWS - 1) / ROWS;
   int* gc = gcnt + (size_t)bhl * NG * NB;
@@ -262,8 +272,8 @@ __global__ __launch_bounds__(1024) void col_scan_kernel(int* __restrict__ gcnt, 
     before += i < wv ? red[i] : 0;
     total += red[i];
   }
-  const long long base = base_of[bhl];
-  int* ptr = k2q_ptr + (size_t)(bh0 + bhl) * (NB + 1);
+  const long long base = lists.of(bhl, NB);
+  int* ptr = k2q_ptr + (size_t)(lists.bh0 + bhl) * (NB + 1);
   int run = before + inc - mine;
   for (int j = c0; j < c1; ++j) {
     ptr[j] = (int)(base + run);
@@ -307,6 +317,77 @@ struct TopkState {
   long long keff;   // min(budget, NB^2)
   int pad[2];
 };
+
+__device__ __forceinline__ long long ListBase::of(int bhl, int NB) const {
+  if (src_ptr != nullptr) return src_ptr[(size_t)(bh0 + bhl) * (NB + 1)];
+  return (long long)(bh0 + bhl) * (st ? st[bhl].keff : keff);
+}
+
+// The whole inversion of one (b, h) with NB <= INV_NB in one workgroup: the bits in LDS, thread (row segment, column)
+// counts its column's bits over its rows, one scan over the columns, then every thread emits its rows in order. (The
+// three launches of the general form are bound by their latency here: 64 blocks, two heads, 4.4 us against 9.4 for
+// the count and the scan alone. Past 512 blocks the bits leave LDS and one workgroup a head is too few.)
+constexpr int INV_NB = 512;
+__global__ __launch_bounds__(1024) void invert_small_kernel(const unsigned* __restrict__ selbits,
+                                                            int* __restrict__ k2q_ptr, int* __restrict__ k2q_idx,
+                                                            int NB, int W, ListBase lists) {
+  __shared__ unsigned bits_s[INV_NB * (INV_NB / 32 + 1)];
+  __shared__ int cnt_s[1024];   // [segment][column]
+  __shared__ int red[16];
+  const int bhl = blockIdx.x, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
+  const int cols = (NB + 63) & ~63, nseg = 1024 / cols, per = (NB + nseg - 1) / nseg, Ws = W | 1;
+  const unsigned* src = selbits + (size_t)bhl * ((NB + 31) & ~31) * W;
+  for (int e = tid; e < NB * W; e += 1024) {
+    const int r = e / W;
+    bits_s[r * Ws + e - r * W] = src[e];
+  }
+  __syncthreads();
+  const int seg = tid / cols, j = tid - seg * cols;
+  const bool mine = seg < nseg && j < NB;
+  const int r0 = min(NB, seg * per), r1 = min(NB, r0 + per), wj = j >> 5, bj = j & 31;
+  int c = 0;
+  if (mine) {
+#pragma unroll 8
+    for (int r = r0; r < r1; ++r) c += (bits_s[r * Ws + wj] >> bj) & 1u;
+  }
+  cnt_s[tid] = c;
+  __syncthreads();
+  // column totals, their exclusive scan over the columns (threads 0 .. cols - 1), then the segments' offsets
+  int tot = 0;
+  if (tid < cols)
+    for (int g = 0; g < nseg; ++g) tot += cnt_s[g * cols + tid];
+  int inc = tot;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(inc, d, 64);
+    if (l >= d) inc += y;
+  }
+  if (l == 63) red[wv] = inc;
+  __syncthreads();
+  int before = 0, total = 0;
+  for (int i = 0; i < 16; ++i) {
+    before += i < wv ? red[i] : 0;
+    total += red[i];
+  }
+  const long long base = lists.of(bhl, NB);
+  int* ptr = k2q_ptr + (size_t)(lists.bh0 + bhl) * (NB + 1);
+  if (tid < cols) {
+    int run = (int)(base + before + inc - tot);
+    if (tid < NB) ptr[tid] = run;
+    if (tid == 0) ptr[NB] = (int)(base + total);
+    for (int g = 0; g < nseg; ++g) {
+      const int n = cnt_s[g * cols + tid];
+      cnt_s[g * cols + tid] = run;
+      run += n;
+    }
+  }
+  __syncthreads();
+  if (mine) {
+    int n = cnt_s[tid];
+    for (int r = r0; r < r1; ++r)
+      if ((bits_s[r * Ws + wj] >> bj) & 1u) k2q_idx[n++] = r;
+  }
+}
 
 __global__ void gk_init_kernel(TopkState* st, unsigned* hist, int bh_count, long long nn, long long budget) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -483,24 +564,6 @@ __global__ __launch_bounds__(256) void gk_emit_kernel(const float* __restrict__ 
   }
 }
 
-// rows of the selection-bit buffer past NB (the last group's padding) must read as empty
-__global__ void clear_pad_rows_kernel(unsigned* selbits, int NB, int W, int bh_count) {
-  const int NBr = (NB + 31) & ~31, pad = NBr - NB;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= bh_count * pad * W) return;
-  const int bhl = e / (pad * W), rem = e - bhl * pad * W;
-  selbits[((size_t)bhl * NBr + NB) * W + rem] = 0;
-}
-
-// absolute list base of each (b, h): (bh0 + b) * keff (routers) or the first entry of a given ptr (transpose)
-__global__ void fill_base_kernel(long long* base, const TopkState* st, long long keff, const int* src_ptr, int NB,
-                                 int bh0, int bh_count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= bh_count) return;
-  if (src_ptr != nullptr) base[i] = src_ptr[(size_t)(bh0 + i) * (NB + 1)];
-  else base[i] = (long long)(bh0 + i) * (st ? st[i].keff : keff);
-}
-
 // the selection bitmap rows of (b, h) bh0 + b into bits_out [BH, NB, W] (the workspace pads rows to ceil32(NB))
 __global__ void export_bits_kernel(const unsigned* __restrict__ selbits, unsigned* __restrict__ bits_out, int NB, int W,
                                    int bh0, int bh_count) {
@@ -525,6 +588,18 @@ __global__ __launch_bounds__(256) void csr_bits_kernel(const int* __restrict__ p
     const int j = idx[e];
     atomicOr(&bits[j >> 5], 1u << (j & 31));
   }
+}
+
+// dense CSR lists over the T = ceil(NB / 64) 64-row tiles of a pooled sequence of NB rows, and the rows in each tile
+__global__ __launch_bounds__(256) void dense_lists_kernel(int NB, int T, int BH, int* __restrict__ cnt,
+                                                          int* __restrict__ ptr, int* __restrict__ idx) {
+  const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (e < T) cnt[e] = min(BK, NB - BK * (int)e);
+  if (e < (long long)(T + 1) * BH) {
+    const int bh = (int)(e / (T + 1)), i = (int)(e - (long long)bh * (T + 1));
+    ptr[e] = (bh * T + i) * T;
+  }
+  if (e < (long long)T * T * BH) idx[e] = (int)(e % T);
 }
 
 // ------------------------------------------------------------------------------------ VSA2 PSP router
@@ -692,7 +767,6 @@ struct TopkCarve {
   int* rowcnt;
   TopkState* st;
   unsigned* hist;
-  long long* base;
 };
 
 static size_t carve(void* base, int bh_count, int NB, TopkCarve* c) {
@@ -708,14 +782,12 @@ static size_t carve(void* base, int bh_count, int NB, TopkCarve* c) {
   char* p2 = take((size_t)bh_count * NB * 2 * 4);
   char* p3 = take((size_t)bh_count * sizeof(TopkState));
   char* p4 = take((size_t)bh_count * 256 * 4);
-  char* p5 = take((size_t)bh_count * 8);
   if (c) {
     c->selbits = (unsigned*)p0;
     c->gcnt = (int*)p1;
     c->rowcnt = (int*)p2;
     c->st = (TopkState*)p3;
     c->hist = (unsigned*)p4;
-    c->base = (long long*)p5;
   }
   return off;
 }
@@ -727,10 +799,16 @@ extern "C" size_t vsa_topk_workspace(int bh_count, int NB) {
 }
 #endif
 
-static int invert(const TopkCarve& c, int* k2q_ptr, int* k2q_idx, int NB, int bh0, int bh_count, hipStream_t stream) {
+static int invert(const TopkCarve& c, const ListBase& lists, int* k2q_ptr, int* k2q_idx, int NB, int bh_count,
+                  hipStream_t stream) {
   const int W = (NB + 31) / 32, NG = (NB + ROWS - 1) / ROWS;
+  if (NB <= INV_NB) {
+    hipLaunchKernelGGL(invert_small_kernel, dim3(bh_count), dim3(1024), 0, stream, c.selbits, k2q_ptr, k2q_idx, NB, W,
+                       lists);
+    return ES_OK;
+  }
   hipLaunchKernelGGL(col_count_kernel, dim3(NG, bh_count), dim3(256), 0, stream, c.selbits, c.gcnt, NB, W);
-  hipLaunchKernelGGL(col_scan_kernel, dim3(bh_count), dim3(1024), 0, stream, c.gcnt, k2q_ptr, NB, bh0, c.base);
+  hipLaunchKernelGGL(col_scan_kernel, dim3(bh_count), dim3(1024), 0, stream, c.gcnt, k2q_ptr, NB, lists);
   hipLaunchKernelGGL(col_emit_kernel, dim3(NG, bh_count), dim3(256), 0, stream, c.selbits, c.gcnt, k2q_idx, NB, W);
   return ES_OK;
 }
@@ -796,17 +874,11 @@ static int rows_common(const void* qc, const void* kc, const void* scores_in, vo
   a.q2k_ptr = q2k_ptr;
   a.q2k_idx = q2k_idx;
   a.selbits = c.selbits;
-  const int W = a.W, pad = ((NB + 31) & ~31) - NB;
-  if (pad > 0)
-    hipLaunchKernelGGL(clear_pad_rows_kernel, dim3((bh_count * pad * W + 255) / 256), dim3(256), 0, stream, c.selbits,
-                       NB, W, bh_count);
-  hipLaunchKernelGGL(fill_base_kernel, dim3((bh_count + 255) / 256), dim3(256), 0, stream, c.base,
-                     (const TopkState*)nullptr, (long long)NB * K, (const int*)nullptr, NB, bh0, bh_count);
   if (scores_in != nullptr)
     rows_launch<true>(a, bh_count, stream);
   else
     rows_launch<false>(a, bh_count, stream);
-  invert(c, k2q_ptr, k2q_idx, NB, bh0, bh_count, stream);
+  invert(c, ListBase{nullptr, (long long)NB * K, nullptr, bh0}, k2q_ptr, k2q_idx, NB, bh_count, stream);
   return check_launch(what);
 }
 
@@ -855,7 +927,7 @@ extern "C" int vsa_global_topk(const float* scores, int NB, int bh0, int bh_coun
              "VSA2: total selected blocks exceed int32 CSR range");
   TopkCarve c;
   carve(workspace, bh_count, NB, &c);
-  const int W = (NB + 31) / 32, pad = ((NB + 31) & ~31) - NB;
+  const int W = (NB + 31) / 32;
   hipLaunchKernelGGL(gk_init_kernel, dim3((bh_count * 256 + 255) / 256), dim3(256), 0, stream, c.st, c.hist, bh_count,
                      nn, budget);
   const int chunks = (int)std::max<long long>(1, std::min<long long>((nn + 4095) / 4096, 1024));
@@ -866,14 +938,9 @@ extern "C" int vsa_global_topk(const float* scores, int NB, int bh0, int bh_coun
   const dim3 rgrid((NB + 3) / 4, bh_count);
   hipLaunchKernelGGL(gk_rowcount_kernel, rgrid, dim3(256), 0, stream, scores, NB, c.st, c.rowcnt);
   hipLaunchKernelGGL(gk_scan_kernel, dim3(bh_count), dim3(1024), 0, stream, c.rowcnt, q2k_ptr, NB, bh0, c.st);
-  if (pad > 0)
-    hipLaunchKernelGGL(clear_pad_rows_kernel, dim3((bh_count * pad * W + 255) / 256), dim3(256), 0, stream, c.selbits,
-                       NB, W, bh_count);
   hipLaunchKernelGGL(gk_emit_kernel, rgrid, dim3(256), 0, stream, scores, NB, bh0, W, c.st, c.rowcnt, q2k_ptr,
                      q2k_idx, c.selbits);
-  hipLaunchKernelGGL(fill_base_kernel, dim3((bh_count + 255) / 256), dim3(256), 0, stream, c.base, c.st, 0LL,
-                     (const int*)nullptr, NB, bh0, bh_count);
-  invert(c, k2q_ptr, k2q_idx, NB, bh0, bh_count, stream);
+  invert(c, ListBase{c.st, 0, nullptr, bh0}, k2q_ptr, k2q_idx, NB, bh_count, stream);
   if (bits_out != nullptr)
     hipLaunchKernelGGL(export_bits_kernel, dim3((bh_count * NB * W + 255) / 256), dim3(256), 0, stream, c.selbits,
                        bits_out, NB, W, bh0, bh_count);
@@ -943,15 +1010,21 @@ extern "C" int vsa_csr_transpose(const int* ptr, const int* idx, int NB, int bh0
   ES_REQUIRE(workspace_bytes >= vsa_topk_workspace(bh_count, NB), ES_ERR_INVALID, "VSA: workspace too small");
   TopkCarve c;
   carve(workspace, bh_count, NB, &c);
-  const int W = (NB + 31) / 32, pad = ((NB + 31) & ~31) - NB;
-  if (pad > 0)
-    hipLaunchKernelGGL(clear_pad_rows_kernel, dim3((bh_count * pad * W + 255) / 256), dim3(256), 0, stream, c.selbits,
-                       NB, W, bh_count);
+  const int W = (NB + 31) / 32;
   hipLaunchKernelGGL(csr_bits_kernel, dim3((NB + 3) / 4, bh_count), dim3(256), 0, stream, ptr, idx, c.selbits, NB, W,
                      bh0);
-  hipLaunchKernelGGL(fill_base_kernel, dim3((bh_count + 255) / 256), dim3(256), 0, stream, c.base,
-                     (const TopkState*)nullptr, 0LL, ptr, NB, bh0, bh_count);
-  invert(c, out_ptr, out_idx, NB, bh0, bh_count, stream);
+  invert(c, ListBase{nullptr, 0, ptr, bh0}, out_ptr, out_idx, NB, bh_count, stream);
   return check_launch("vsa_csr_transpose");
+}
+
+extern "C" int vsa_dense_lists(int NB, int BH, int* cnt, int* ptr, int* idx, hipStream_t stream) {
+  ES_REQUIRE(cnt && ptr && idx, ES_ERR_INVALID, "VSA: null tensor pointer");
+  ES_REQUIRE(NB >= 1 && BH >= 1, ES_ERR_INVALID, "VSA: NB and BH must be positive");
+  const long long T = (NB + BK - 1) / BK, n = T * T * BH;
+  ES_REQUIRE(n < (1LL << 31), ES_ERR_UNSUPPORTED, "VSA: total listed tiles exceed int32 CSR range");
+  const long long all = std::max(n, (T + 1) * BH);
+  hipLaunchKernelGGL(dense_lists_kernel, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, stream, NB, (int)T, BH, cnt,
+                     ptr, idx);
+  return check_launch("vsa_dense_lists");
 }
 #endif

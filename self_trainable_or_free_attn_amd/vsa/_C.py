@@ -333,6 +333,15 @@ def csr_transpose(ptr, idx):
     return out_ptr, out_idx
 
 
+def dense_lists(B, H, nb, device):
+    """(tile counts [T], ptr [B, H, T + 1], idx): every 64-row tile of a pooled sequence of nb rows lists all T tiles."""
+    T = (nb + 63) // 64
+    i32 = dict(device=device, dtype=torch.int32)
+    cnt, ptr, idx = torch.empty(T, **i32), torch.empty(B, H, T + 1, **i32), torch.empty(B * H * T * T, **i32)
+    _call("vsa_dense_lists", int(nb), B * H, cnt, ptr, idx)
+    return cnt, ptr, idx
+
+
 # ------------------------------------------------------------------ attention
 def _attn_args(q, k, v, blk_cnt):
     for t, n in ((q, "q"), (k, "k"), (v, "v")):

@@ -322,12 +322,7 @@ def _fine_backward(C, q, k, v, dout, lse, delta, sel, blk_cnt, add_q, add_k, add
 
 def _coarse_lists(B, H, nb, nbc_pad, device):
     """Dense CSR over the 64-row tiles of the pooled sequence: (tile counts, ptr, idx)."""
-    T = nbc_pad // 64
-    cnt = (nb - 64 * torch.arange(T, device=device)).clamp(max=64).to(torch.int32)
-    heads = torch.arange(B * H, device=device, dtype=torch.int64)[:, None]
-    ptr = (heads * T * T + torch.arange(T + 1, device=device)[None, :] * T).to(torch.int32).reshape(B, H, T + 1)
-    idx = torch.arange(T, device=device, dtype=torch.int32).repeat(B * H * T)
-    return cnt.contiguous(), ptr.contiguous(), idx.contiguous()
+    return ext().dense_lists(B, H, nb, device)
 
 
 class _VsaFunction(torch.autograd.Function):
