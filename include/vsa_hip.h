@@ -17,7 +17,7 @@
  *                                    and computes on the first 64 columns only. D | VSA_PACKED_ROWS: every row
  *                                    (tokens, pooled rows, fp32 gradients and partials) is D columns wide instead;
  *                                    taken by the pooling, fusion, fine attention, router and split-KV entry
- *                                    points, not by the three-tier ones (vsa_rep_*, vsa_row_dot)
+ *                                    points and vsa_row_dot, not by the three-tier ones (vsa_rep_*)
  *   blk_cnt                          [NB] int32, valid tokens per block (1..64)
  *   router pools qr, kr, vr          [BH, Lr_pad, 128] bf16, Lr_pad = ceil64(NB * 64 / R)
  *   block means qc, kc, vc           [BH, NBc_pad, 128] bf16, NBc_pad = ceil64(NB)

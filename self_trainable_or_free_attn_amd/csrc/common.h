@@ -189,6 +189,15 @@ __device__ __forceinline__ float dpp_f(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWMASK, 0xF, true));
 }
 
+// sum over the 16 lanes of a DPP row (no LDS traffic), valid in the row's lane 15
+__device__ __forceinline__ float row16_sum(float x) {
+  x += dpp_f<0x111>(x);
+  x += dpp_f<0x112>(x);
+  x += dpp_f<0x114>(x);
+  x += dpp_f<0x118>(x);
+  return x;
+}
+
 // sum over the 64 lanes with DPP row shifts / broadcasts (no LDS traffic); the result is wave-uniform
 __device__ __forceinline__ float wave_sum_dpp(float x) {
   x += dpp_f<0x111>(x);        // row_shr:1

@@ -654,30 +654,30 @@ __global__ __launch_bounds__(256) void rep_unpool_kernel(const float* __restrict
   }
 }
 
-// delta[row] = <dO, O> on valid rows, 0 on padding; one wave per block, 16 lanes per token row
+// delta[row] = <dO, O> on valid rows, 0 on padding; one workgroup per block, 16 lanes per token row, four rows a lane
+// with their loads in flight together
 __global__ __launch_bounds__(256) void row_dot_kernel(const e16_t* __restrict__ x, const e16_t* __restrict__ y,
                                                       float* __restrict__ out, const int* __restrict__ blk_cnt, int L,
-                                                      int NB) {
-  const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (blk >= NB) return;
-  const int l = threadIdx.x & 63, s = l >> 4, c8 = (l & 15) * 8;
-  const size_t bh = blockIdx.y;
+                                                      int ld) {
+  const int blk = blockIdx.x, s = threadIdx.x >> 4, c8 = (threadIdx.x & 15) * 8;
   const int cnt = blk_cnt[blk];
-  for (int r = s; r < BK; r += 4) {
-    const size_t t = bh * L + (size_t)blk * BK + r;
+  const size_t t0 = (size_t)blockIdx.y * L + (size_t)blk * BK;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int r = s + 16 * k;
+    const size_t t = t0 + r;
     float acc = 0.0f;
-    if (r < cnt) {
-      const uint4 ux = *reinterpret_cast<const uint4*>(x + t * HD + c8);
-      const uint4 uy = *reinterpret_cast<const uint4*>(y + t * HD + c8);
+    if (r < cnt && c8 < ld) {
+      const uint4 ux = *reinterpret_cast<const uint4*>(x + t * ld + c8);
+      const uint4 uy = *reinterpret_cast<const uint4*>(y + t * ld + c8);
       const unsigned wx[4] = {ux.x, ux.y, ux.z, ux.w}, wy[4] = {uy.x, uy.y, uy.z, uy.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         acc += e2f((e16_t)(wx[i] & 0xffffu)) * e2f((e16_t)(wy[i] & 0xffffu)) +
                e2f((e16_t)(wx[i] >> 16)) * e2f((e16_t)(wy[i] >> 16));
     }
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) acc += __shfl_xor(acc, m, 16);
-    if ((l & 15) == 0) out[t] = acc;
+    acc = row16_sum(acc);
+    if ((threadIdx.x & 15) == 15) out[t] = acc;
   }
 }
 
@@ -883,10 +883,10 @@ extern "C" int ES_VSA_API(vsa_row_dot)(const void* x, const void* y, const int* 
                            hipStream_t stream) {
   ES_REQUIRE(x && y && blk_cnt && out, ES_ERR_INVALID, "VSA: null tensor pointer");
   ES_REQUIRE(BH > 0 && BH <= 65535 && L > 0 && L % BK == 0, ES_ERR_INVALID, "VSA: tokens must be [BH, L = NB * 64, D]");
-  ES_REQUIRE(D == 64 || D == HD, ES_ERR_UNSUPPORTED, "VSA: head dim must be 64 or 128 (rows stored with 128 columns)");
-  const int NB = L / BK;
-  hipLaunchKernelGGL(row_dot_kernel, dim3((NB + 3) / 4, BH), dim3(256), 0, stream, (const e16_t*)x, (const e16_t*)y,
-                     out, blk_cnt, L, NB);
+  HeadDim h;
+  VSA_REQUIRE_DIM(D, h);
+  hipLaunchKernelGGL(row_dot_kernel, dim3(L / BK, BH), dim3(256), 0, stream, (const e16_t*)x, (const e16_t*)y, out,
+                     blk_cnt, L, h.ld);
   return check_launch("vsa_row_dot");
 }
 

@@ -686,5 +686,5 @@ def row_dot(a, b, blk_cnt):
     """[B, H, L] fp32 rowsum(a * b) on valid rows, 0 on padding (reference rep_api.cpp row_dot)."""
     B, H, L, D = a.shape
     out = torch.empty(B, H, L, device=a.device, dtype=torch.float32)
-    _call("vsa_row_dot", _wide(a), _wide(b), blk_cnt, out, B * H, L, D)
+    _call("vsa_row_dot", _rows(a, D), _rows(b, D), blk_cnt, out, B * H, L, _dim(D))
     return out

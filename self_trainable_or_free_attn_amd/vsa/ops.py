@@ -434,10 +434,8 @@ class _FineFunction(torch.autograd.Function):
     def backward(ctx, dout, dlse):
         C = ext()
         q, k, v, blk_cnt, of, lse, *sel = ctx.saved_tensors
-        B, H, L, D = q.shape
-        zeros_c = torch.zeros(B, H, (L // 64 + 63) // 64 * 64, D, device=q.device, dtype=q.dtype)
         dout = dout.contiguous()
-        _, delta, _, _, _ = C.fuse_bwd(dout, of, zeros_c, None, blk_cnt, 0, False)
+        delta = C.row_dot(dout, of, blk_cnt)
         dq, dk, dv = _fine_backward(C, q, k, v, dout, lse, delta, tuple(sel), blk_cnt, None, None, None, ctx.split)
         return dq, dk, dv, None, None, None, None
 

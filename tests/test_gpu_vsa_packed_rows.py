@@ -69,7 +69,10 @@ def test_packed_rows_equal_padded_rows(case):
         delta, dof, doc, dc, dg = stat(BH, L), rows(BH, L, dtype=bf), rows(BH, 64, dtype=bf), stat(BH, 64), \
             rows(BH, L, dtype=bf)
         _lib.call("vsa_fuse_bwd", do, o, w(oc), gate, dof, delta, doc, dc, dg, cnt, BH, L, D, 64, 2, 0)
-        out = [o, lse, fused, delta, dof, doc, dc, dg]
+        dot = stat(BH, L)
+        _lib.call("vsa_row_dot", do, o, cnt, dot, BH, L, D)
+        assert torch.allclose(dot, delta, rtol=0, atol=1e-4)     # 64 products of about 1 in float32, two orders
+        out = [o, lse, fused, delta, dof, doc, dc, dg, dot]
         add = w(torch.linspace(-1, 1, BH * 64 * 64, device="cuda").view(BH, 64, 64))
         for dt, flag in ((bf, 0), (f32, 1)):
             dk, dv = rows(BH, L, dtype=dt), rows(BH, L, dtype=dt)
@@ -115,7 +118,7 @@ def test_wrong_head_dims_stay_refused(case):
             _lib.call("vsa_attn_fwd", x["q"], x["k"], x["v"], c["sel"].q2k_ptr, c["sel"].q2k_idx, c["cnt"], o, lse,
                       c["BH"], c["L"], D)
     with pytest.raises(RuntimeError):
-        _lib.call("vsa_row_dot", x["q"], x["k"], c["cnt"], lse, c["BH"], c["L"], PACKED)
+        _lib.call("vsa_row_dot", x["q"], x["k"], c["cnt"], lse, c["BH"], c["L"], 32 | 0x10000)
 
 
 def test_unaligned_and_strided_d64_arguments(case):
