@@ -326,8 +326,8 @@ __device__ __forceinline__ long long ListBase::of(int bhl, int NB) const {
 // The whole inversion of one (b, h) with NB <= INV_NB in one workgroup: the bits in LDS, thread (row segment, column)
 // counts its column's bits over its rows, one scan over the columns, then every thread emits its rows in order. (The
 // three launches of the general form are bound by their latency here: 64 blocks, two heads, 4.4 us against 9.4 for
-// the count and the scan alone. Past 512 blocks the bits leave LDS and one workgroup a head is too few.)
-constexpr int INV_NB = 512;
+// the count and the scan alone; 480 blocks, 24 heads, 32 us against 22, so the line lies between.)
+constexpr int INV_NB = 256;
 __global__ __launch_bounds__(1024) void invert_small_kernel(const unsigned* __restrict__ selbits,
                                                             int* __restrict__ k2q_ptr, int* __restrict__ k2q_idx,
                                                             int NB, int W, ListBase lists) {

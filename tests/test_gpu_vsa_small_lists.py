@@ -1,4 +1,4 @@
-"""The one-workgroup kv->q inversion (NB <= 512) at its edges against numpy, through the CSR transpose and the global
+"""The one-workgroup kv->q inversion (NB <= 256) at its edges against numpy, through the CSR transpose and the global
 top-k, and the dense lists of the coarse branch."""
 import numpy as np
 import pytest
@@ -7,7 +7,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("NB", [1, 31, 32, 33, 64, 65, 128, 129, 320, 321, 511, 512, 513])
+@pytest.mark.parametrize("NB", [1, 31, 32, 33, 64, 65, 128, 129, 192, 193, 255, 256, 257, 512])
 @pytest.mark.parametrize("density", [0.0, 0.2, 1.0])
 def test_csr_transpose_small(dev, NB, density):
     from self_trainable_or_free_attn_amd.vsa import _C, mask_to_selection
