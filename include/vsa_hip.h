@@ -239,6 +239,15 @@ int vsa_rep_bwd_tables(const void* q, const void* dout, const void* k_tab, const
                        int lc_stride, const float* lse, const float* delta, const unsigned* bits_a, const unsigned* bits_ab,
                        float* dk_tab, float* dv_tab, int BH, int L, int D, int RM, int tier, hipStream_t stream);
 
+/* vsa_rep_bwd_tables of both tiers in one launch (the tier-C rows alone leave most of the GPU idle): the mid table's
+ * gradients over the tier-B pairs and the tail table's over the tier-C pairs, each added into its fp32 tensors.
+ * Replaces the same reference function. */
+int vsa_rep_bwd_both_tables(const void* q, const void* dout, const void* k_mid, const void* v_mid, const float* lc_mid,
+                            int lc_mid_stride, const void* k_tail, const void* v_tail, const float* lc_tail,
+                            const float* lse, const float* delta, const unsigned* bits_a, const unsigned* bits_ab,
+                            float* dk_mid, float* dv_mid, float* dk_tail, float* dv_tail, int BH, int L, int D, int RM,
+                            hipStream_t stream);
+
 /* dK, dV (bf16) = acc (fp32 tier-A token gradients, optional) + dk_mid[group] / c_group + dk_tail[blk] / c_blk on
  * valid rows, 0 on padding; group = the token's contiguous group, or with labels / mid_counts (k-means tables,
  * both or neither) its cluster and that cluster's size. Replaces rep_api.cpp rep_unpool (rep_pool.cu:59-88). */
@@ -326,6 +335,11 @@ int vsa_rep_attn_bwd_q_f16(const void* q, const void* k, const void* v, const vo
 int vsa_rep_bwd_tables_f16(const void* q, const void* dout, const void* k_tab, const void* v_tab, const float* lc,
                            int lc_stride, const float* lse, const float* delta, const unsigned* bits_a, const unsigned* bits_ab,
                            float* dk_tab, float* dv_tab, int BH, int L, int D, int RM, int tier, hipStream_t stream);
+int vsa_rep_bwd_both_tables_f16(const void* q, const void* dout, const void* k_mid, const void* v_mid,
+                                const float* lc_mid, int lc_mid_stride, const void* k_tail, const void* v_tail,
+                                const float* lc_tail, const float* lse, const float* delta, const unsigned* bits_a,
+                                const unsigned* bits_ab, float* dk_mid, float* dv_mid, float* dk_tail, float* dv_tail,
+                                int BH, int L, int D, int RM, hipStream_t stream);
 int vsa_rep_build_kmeans_f16(const void* k, const void* v, const int* blk_cnt, void* k_mid, void* v_mid,
                              float* lc_mid, int* counts, uint8_t* labels, int BH, int L, int D, int RM, int iters,
                              unsigned seed, hipStream_t stream);

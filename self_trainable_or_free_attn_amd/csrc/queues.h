@@ -164,9 +164,11 @@ struct Queues {
 // and nothing is cleared, waited for or recorded. (The counters' kernel takes 1.4 us and its gap on the stream, and
 // the wait and record two more host calls. A forward + backward of 4096 tokens and two heads, with the launches saved
 // in its router and lists: 564 -> 368 us.)
-static bool balanced_launch_queues(int per_queue, hipStream_t stream, Queues& out, int resident = 512) {
+// claim_all: every item is claimed (few, long items that a fixed binding to XCDs would leave uneven).
+static bool balanced_launch_queues(int per_queue, hipStream_t stream, Queues& out, int resident = 512,
+                                   bool claim_all = false) {
   out.release();
-  if (8LL * per_queue <= resident) {
+  if (!claim_all && 8LL * per_queue <= resident) {
     out.counters = nullptr;
     out.fixed = per_queue;
     out.grid = 8LL * per_queue;
@@ -192,7 +194,7 @@ static bool balanced_launch_queues(int per_queue, hipStream_t stream, Queues& ou
   out.captured = captured;
   out.stream = stream;
   out.counters = r->base + slot * 8;
-  const int claimable = (per_queue + 7) / 8;
+  const int claimable = claim_all ? per_queue : (per_queue + 7) / 8;
   out.fixed = per_queue - claimable;
   out.grid = 8LL * (out.fixed + 2LL * claimable);
   hipLaunchKernelGGL(zero_queues_kernel, dim3(1), dim3(64), 0, stream, out.counters);

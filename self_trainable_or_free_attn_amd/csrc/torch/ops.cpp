@@ -440,6 +440,15 @@ static void op_vsa_rep_bwd_tables(const c10::optional<at::Tensor>& q, const c10:
 }
 static void meta_vsa_rep_bwd_tables(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_tab, const c10::optional<at::Tensor>& v_tab, const c10::optional<at::Tensor>& lc, int64_t lc_stride, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_tab, const c10::optional<at::Tensor>& dv_tab, int64_t BH, int64_t L, int64_t D, int64_t RM, int64_t tier) {}
 
+static void op_vsa_rep_bwd_both_tables(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_mid, const c10::optional<at::Tensor>& v_mid, const c10::optional<at::Tensor>& lc_mid, int64_t lc_mid_stride, const c10::optional<at::Tensor>& k_tail, const c10::optional<at::Tensor>& v_tail, const c10::optional<at::Tensor>& lc_tail, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_mid, const c10::optional<at::Tensor>& dv_mid, const c10::optional<at::Tensor>& dk_tail, const c10::optional<at::Tensor>& dv_tail, int64_t BH, int64_t L, int64_t D, int64_t RM) {
+  const Call es_op_call("vsa_rep_bwd_both_tables", {&q, &dout, &k_mid, &v_mid, &lc_mid, &k_tail, &v_tail, &lc_tail, &lse, &delta, &bits_a, &bits_ab, &dk_mid, &dv_mid, &dk_tail, &dv_tail});
+  c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
+  const hipStream_t es_op_stream =
+      es_op_call.dev ? c10::hip::getCurrentHIPStream(es_op_call.dev->index()).stream() : nullptr;
+  es_op_check("vsa_rep_bwd_both_tables", vsa_rep_bwd_both_tables(static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "q", q, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "dout", dout, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "k_mid", k_mid, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "v_mid", v_mid, ES_HALF)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables", "lc_mid", lc_mid, ES_F32)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables", "lc_mid_stride", lc_mid_stride, ES_INT)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "k_tail", k_tail, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables", "v_tail", v_tail, ES_HALF)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables", "lc_tail", lc_tail, ES_F32)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables", "lse", lse, ES_F32)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables", "delta", delta, ES_F32)), static_cast<const unsigned*>(es_op_data("vsa_rep_bwd_both_tables", "bits_a", bits_a, ES_I32)), static_cast<const unsigned*>(es_op_data("vsa_rep_bwd_both_tables", "bits_ab", bits_ab, ES_I32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables", "dk_mid", dk_mid, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables", "dv_mid", dv_mid, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables", "dk_tail", dk_tail, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables", "dv_tail", dv_tail, ES_F32)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables", "BH", BH, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables", "L", L, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables", "D", D, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables", "RM", RM, ES_INT)), es_op_stream));
+}
+static void meta_vsa_rep_bwd_both_tables(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_mid, const c10::optional<at::Tensor>& v_mid, const c10::optional<at::Tensor>& lc_mid, int64_t lc_mid_stride, const c10::optional<at::Tensor>& k_tail, const c10::optional<at::Tensor>& v_tail, const c10::optional<at::Tensor>& lc_tail, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_mid, const c10::optional<at::Tensor>& dv_mid, const c10::optional<at::Tensor>& dk_tail, const c10::optional<at::Tensor>& dv_tail, int64_t BH, int64_t L, int64_t D, int64_t RM) {}
+
 static void op_vsa_rep_unpool(const c10::optional<at::Tensor>& acc_k, const c10::optional<at::Tensor>& acc_v, const c10::optional<at::Tensor>& dk_mid, const c10::optional<at::Tensor>& dv_mid, const c10::optional<at::Tensor>& dk_tail, const c10::optional<at::Tensor>& dv_tail, const c10::optional<at::Tensor>& blk_cnt, const c10::optional<at::Tensor>& labels, const c10::optional<at::Tensor>& mid_counts, const c10::optional<at::Tensor>& dk, const c10::optional<at::Tensor>& dv, int64_t BH, int64_t L, int64_t D, int64_t RM) {
   const Call es_op_call("vsa_rep_unpool", {&acc_k, &acc_v, &dk_mid, &dv_mid, &dk_tail, &dv_tail, &blk_cnt, &labels, &mid_counts, &dk, &dv});
   c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
@@ -656,6 +665,15 @@ static void op_vsa_rep_bwd_tables_f16(const c10::optional<at::Tensor>& q, const 
 }
 static void meta_vsa_rep_bwd_tables_f16(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_tab, const c10::optional<at::Tensor>& v_tab, const c10::optional<at::Tensor>& lc, int64_t lc_stride, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_tab, const c10::optional<at::Tensor>& dv_tab, int64_t BH, int64_t L, int64_t D, int64_t RM, int64_t tier) {}
 
+static void op_vsa_rep_bwd_both_tables_f16(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_mid, const c10::optional<at::Tensor>& v_mid, const c10::optional<at::Tensor>& lc_mid, int64_t lc_mid_stride, const c10::optional<at::Tensor>& k_tail, const c10::optional<at::Tensor>& v_tail, const c10::optional<at::Tensor>& lc_tail, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_mid, const c10::optional<at::Tensor>& dv_mid, const c10::optional<at::Tensor>& dk_tail, const c10::optional<at::Tensor>& dv_tail, int64_t BH, int64_t L, int64_t D, int64_t RM) {
+  const Call es_op_call("vsa_rep_bwd_both_tables_f16", {&q, &dout, &k_mid, &v_mid, &lc_mid, &k_tail, &v_tail, &lc_tail, &lse, &delta, &bits_a, &bits_ab, &dk_mid, &dv_mid, &dk_tail, &dv_tail});
+  c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
+  const hipStream_t es_op_stream =
+      es_op_call.dev ? c10::hip::getCurrentHIPStream(es_op_call.dev->index()).stream() : nullptr;
+  es_op_check("vsa_rep_bwd_both_tables_f16", vsa_rep_bwd_both_tables_f16(static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "q", q, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "dout", dout, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "k_mid", k_mid, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "v_mid", v_mid, ES_HALF)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "lc_mid", lc_mid, ES_F32)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables_f16", "lc_mid_stride", lc_mid_stride, ES_INT)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "k_tail", k_tail, ES_HALF)), static_cast<const void*>(es_op_data("vsa_rep_bwd_both_tables_f16", "v_tail", v_tail, ES_HALF)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "lc_tail", lc_tail, ES_F32)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "lse", lse, ES_F32)), static_cast<const float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "delta", delta, ES_F32)), static_cast<const unsigned*>(es_op_data("vsa_rep_bwd_both_tables_f16", "bits_a", bits_a, ES_I32)), static_cast<const unsigned*>(es_op_data("vsa_rep_bwd_both_tables_f16", "bits_ab", bits_ab, ES_I32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "dk_mid", dk_mid, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "dv_mid", dv_mid, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "dk_tail", dk_tail, ES_F32)), static_cast<float*>(es_op_data("vsa_rep_bwd_both_tables_f16", "dv_tail", dv_tail, ES_F32)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables_f16", "BH", BH, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables_f16", "L", L, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables_f16", "D", D, ES_INT)), static_cast<int>(es_op_int("vsa_rep_bwd_both_tables_f16", "RM", RM, ES_INT)), es_op_stream));
+}
+static void meta_vsa_rep_bwd_both_tables_f16(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& dout, const c10::optional<at::Tensor>& k_mid, const c10::optional<at::Tensor>& v_mid, const c10::optional<at::Tensor>& lc_mid, int64_t lc_mid_stride, const c10::optional<at::Tensor>& k_tail, const c10::optional<at::Tensor>& v_tail, const c10::optional<at::Tensor>& lc_tail, const c10::optional<at::Tensor>& lse, const c10::optional<at::Tensor>& delta, const c10::optional<at::Tensor>& bits_a, const c10::optional<at::Tensor>& bits_ab, const c10::optional<at::Tensor>& dk_mid, const c10::optional<at::Tensor>& dv_mid, const c10::optional<at::Tensor>& dk_tail, const c10::optional<at::Tensor>& dv_tail, int64_t BH, int64_t L, int64_t D, int64_t RM) {}
+
 static void op_vsa_rep_build_kmeans_f16(const c10::optional<at::Tensor>& k, const c10::optional<at::Tensor>& v, const c10::optional<at::Tensor>& blk_cnt, const c10::optional<at::Tensor>& k_mid, const c10::optional<at::Tensor>& v_mid, const c10::optional<at::Tensor>& lc_mid, const c10::optional<at::Tensor>& counts, const c10::optional<at::Tensor>& labels, int64_t BH, int64_t L, int64_t D, int64_t RM, int64_t iters, int64_t seed) {
   const Call es_op_call("vsa_rep_build_kmeans_f16", {&k, &v, &blk_cnt, &k_mid, &v_mid, &lc_mid, &counts, &labels});
   c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
@@ -725,6 +743,7 @@ TORCH_LIBRARY(echosparse_gfx950, m) {
   m.def("vsa_rep_attn_fwd(Tensor? q, Tensor? k, Tensor? v, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? q2k_ptr, Tensor? q2k_idx, Tensor? bits_a, Tensor? bits_ab, Tensor? blk_cnt, Tensor(a!)? out, Tensor(b!)? lse, int BH, int L, int D, int RM, int phases) -> ()");
   m.def("vsa_rep_attn_bwd_q(Tensor? q, Tensor? k, Tensor? v, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? dout, Tensor? lse, Tensor? delta, Tensor? q2k_ptr, Tensor? q2k_idx, Tensor? bits_a, Tensor? bits_ab, Tensor? blk_cnt, Tensor? add_dq, int add_nb, Tensor? dq_acc, Tensor(a!)? dq, int BH, int L, int D, int RM, int phases) -> ()");
   m.def("vsa_rep_bwd_tables(Tensor? q, Tensor? dout, Tensor? k_tab, Tensor? v_tab, Tensor? lc, int lc_stride, Tensor? lse, Tensor? delta, Tensor? bits_a, Tensor? bits_ab, Tensor(a!)? dk_tab, Tensor(b!)? dv_tab, int BH, int L, int D, int RM, int tier) -> ()");
+  m.def("vsa_rep_bwd_both_tables(Tensor? q, Tensor? dout, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? lse, Tensor? delta, Tensor? bits_a, Tensor? bits_ab, Tensor(a!)? dk_mid, Tensor(b!)? dv_mid, Tensor(c!)? dk_tail, Tensor(d!)? dv_tail, int BH, int L, int D, int RM) -> ()");
   m.def("vsa_rep_unpool(Tensor? acc_k, Tensor? acc_v, Tensor? dk_mid, Tensor? dv_mid, Tensor? dk_tail, Tensor? dv_tail, Tensor? blk_cnt, Tensor? labels, Tensor? mid_counts, Tensor(a!)? dk, Tensor(b!)? dv, int BH, int L, int D, int RM) -> ()");
   m.def("vsa_row_dot(Tensor? x, Tensor? y, Tensor? blk_cnt, Tensor(a!)? out, int BH, int L, int D) -> ()");
   m.def("vsa_tier_b_lists(Tensor? ab_ptr, Tensor? ab_idx, Tensor? a_ptr, Tensor? bits_a, Tensor(a!)? b_ptr, Tensor(b!)? b_idx, int BH, int NB) -> ()");
@@ -749,6 +768,7 @@ TORCH_LIBRARY(echosparse_gfx950, m) {
   m.def("vsa_rep_attn_fwd_f16(Tensor? q, Tensor? k, Tensor? v, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? q2k_ptr, Tensor? q2k_idx, Tensor? bits_a, Tensor? bits_ab, Tensor? blk_cnt, Tensor(a!)? out, Tensor(b!)? lse, int BH, int L, int D, int RM, int phases) -> ()");
   m.def("vsa_rep_attn_bwd_q_f16(Tensor? q, Tensor? k, Tensor? v, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? dout, Tensor? lse, Tensor? delta, Tensor? q2k_ptr, Tensor? q2k_idx, Tensor? bits_a, Tensor? bits_ab, Tensor? blk_cnt, Tensor? add_dq, int add_nb, Tensor? dq_acc, Tensor(a!)? dq, int BH, int L, int D, int RM, int phases) -> ()");
   m.def("vsa_rep_bwd_tables_f16(Tensor? q, Tensor? dout, Tensor? k_tab, Tensor? v_tab, Tensor? lc, int lc_stride, Tensor? lse, Tensor? delta, Tensor? bits_a, Tensor? bits_ab, Tensor(a!)? dk_tab, Tensor(b!)? dv_tab, int BH, int L, int D, int RM, int tier) -> ()");
+  m.def("vsa_rep_bwd_both_tables_f16(Tensor? q, Tensor? dout, Tensor? k_mid, Tensor? v_mid, Tensor? lc_mid, int lc_mid_stride, Tensor? k_tail, Tensor? v_tail, Tensor? lc_tail, Tensor? lse, Tensor? delta, Tensor? bits_a, Tensor? bits_ab, Tensor(a!)? dk_mid, Tensor(b!)? dv_mid, Tensor(c!)? dk_tail, Tensor(d!)? dv_tail, int BH, int L, int D, int RM) -> ()");
   m.def("vsa_rep_build_kmeans_f16(Tensor? k, Tensor? v, Tensor? blk_cnt, Tensor(a!)? k_mid, Tensor(b!)? v_mid, Tensor(c!)? lc_mid, Tensor(d!)? counts, Tensor(e!)? labels, int BH, int L, int D, int RM, int iters, int seed) -> ()");
   m.def("vsa_rep_unpool_f16(Tensor? acc_k, Tensor? acc_v, Tensor? dk_mid, Tensor? dv_mid, Tensor? dk_tail, Tensor? dv_tail, Tensor? blk_cnt, Tensor? labels, Tensor? mid_counts, Tensor(a!)? dk, Tensor(b!)? dv, int BH, int L, int D, int RM) -> ()");
   m.def("vsa_row_dot_f16(Tensor? x, Tensor? y, Tensor? blk_cnt, Tensor(a!)? out, int BH, int L, int D) -> ()");
@@ -795,6 +815,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CUDA, m) {
   m.impl("vsa_rep_attn_fwd", TORCH_FN(op_vsa_rep_attn_fwd));
   m.impl("vsa_rep_attn_bwd_q", TORCH_FN(op_vsa_rep_attn_bwd_q));
   m.impl("vsa_rep_bwd_tables", TORCH_FN(op_vsa_rep_bwd_tables));
+  m.impl("vsa_rep_bwd_both_tables", TORCH_FN(op_vsa_rep_bwd_both_tables));
   m.impl("vsa_rep_unpool", TORCH_FN(op_vsa_rep_unpool));
   m.impl("vsa_row_dot", TORCH_FN(op_vsa_row_dot));
   m.impl("vsa_tier_b_lists", TORCH_FN(op_vsa_tier_b_lists));
@@ -819,6 +840,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CUDA, m) {
   m.impl("vsa_rep_attn_fwd_f16", TORCH_FN(op_vsa_rep_attn_fwd_f16));
   m.impl("vsa_rep_attn_bwd_q_f16", TORCH_FN(op_vsa_rep_attn_bwd_q_f16));
   m.impl("vsa_rep_bwd_tables_f16", TORCH_FN(op_vsa_rep_bwd_tables_f16));
+  m.impl("vsa_rep_bwd_both_tables_f16", TORCH_FN(op_vsa_rep_bwd_both_tables_f16));
   m.impl("vsa_rep_build_kmeans_f16", TORCH_FN(op_vsa_rep_build_kmeans_f16));
   m.impl("vsa_rep_unpool_f16", TORCH_FN(op_vsa_rep_unpool_f16));
   m.impl("vsa_row_dot_f16", TORCH_FN(op_vsa_row_dot_f16));
@@ -865,6 +887,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CPU, m) {
   m.impl("vsa_rep_attn_fwd", TORCH_FN(op_vsa_rep_attn_fwd));
   m.impl("vsa_rep_attn_bwd_q", TORCH_FN(op_vsa_rep_attn_bwd_q));
   m.impl("vsa_rep_bwd_tables", TORCH_FN(op_vsa_rep_bwd_tables));
+  m.impl("vsa_rep_bwd_both_tables", TORCH_FN(op_vsa_rep_bwd_both_tables));
   m.impl("vsa_rep_unpool", TORCH_FN(op_vsa_rep_unpool));
   m.impl("vsa_row_dot", TORCH_FN(op_vsa_row_dot));
   m.impl("vsa_tier_b_lists", TORCH_FN(op_vsa_tier_b_lists));
@@ -889,6 +912,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CPU, m) {
   m.impl("vsa_rep_attn_fwd_f16", TORCH_FN(op_vsa_rep_attn_fwd_f16));
   m.impl("vsa_rep_attn_bwd_q_f16", TORCH_FN(op_vsa_rep_attn_bwd_q_f16));
   m.impl("vsa_rep_bwd_tables_f16", TORCH_FN(op_vsa_rep_bwd_tables_f16));
+  m.impl("vsa_rep_bwd_both_tables_f16", TORCH_FN(op_vsa_rep_bwd_both_tables_f16));
   m.impl("vsa_rep_build_kmeans_f16", TORCH_FN(op_vsa_rep_build_kmeans_f16));
   m.impl("vsa_rep_unpool_f16", TORCH_FN(op_vsa_rep_unpool_f16));
   m.impl("vsa_row_dot_f16", TORCH_FN(op_vsa_row_dot_f16));
@@ -935,6 +959,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, Meta, m) {
   m.impl("vsa_rep_attn_fwd", TORCH_FN(meta_vsa_rep_attn_fwd));
   m.impl("vsa_rep_attn_bwd_q", TORCH_FN(meta_vsa_rep_attn_bwd_q));
   m.impl("vsa_rep_bwd_tables", TORCH_FN(meta_vsa_rep_bwd_tables));
+  m.impl("vsa_rep_bwd_both_tables", TORCH_FN(meta_vsa_rep_bwd_both_tables));
   m.impl("vsa_rep_unpool", TORCH_FN(meta_vsa_rep_unpool));
   m.impl("vsa_row_dot", TORCH_FN(meta_vsa_row_dot));
   m.impl("vsa_tier_b_lists", TORCH_FN(meta_vsa_tier_b_lists));
@@ -959,6 +984,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, Meta, m) {
   m.impl("vsa_rep_attn_fwd_f16", TORCH_FN(meta_vsa_rep_attn_fwd_f16));
   m.impl("vsa_rep_attn_bwd_q_f16", TORCH_FN(meta_vsa_rep_attn_bwd_q_f16));
   m.impl("vsa_rep_bwd_tables_f16", TORCH_FN(meta_vsa_rep_bwd_tables_f16));
+  m.impl("vsa_rep_bwd_both_tables_f16", TORCH_FN(meta_vsa_rep_bwd_both_tables_f16));
   m.impl("vsa_rep_build_kmeans_f16", TORCH_FN(meta_vsa_rep_build_kmeans_f16));
   m.impl("vsa_rep_unpool_f16", TORCH_FN(meta_vsa_rep_unpool_f16));
   m.impl("vsa_row_dot_f16", TORCH_FN(meta_vsa_row_dot_f16));

@@ -368,27 +368,34 @@ __global__ __launch_bounds__(256, 2) void rep_q_kernel(RepArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ table dK / dV
+// one tier's table and its gradients
+struct Table {
+  const e16_t *k, *v;  // [BH, rows_pad, D]
+  const float* lc;     // [rows], or [BH, lc_stride] per head
+  int lc_stride;
+  float *dk, *dv;      // [BH, rows_pad, D] fp32, accumulated
+  int rows, rows_pad;
+};
+
 struct TabArgs {
   const e16_t *q, *dout;
-  const e16_t *k_tab, *v_tab;  // [BH, rows_pad, D]
-  const float* lc;              // [rows], or [BH, lc_stride] per head
-  int lc_stride;
+  Table mid, tail;              // tiers B and C
   const float *lse, *delta;
   const unsigned *bits_a, *bits_ab;
-  float *dk_tab, *dv_tab;       // [BH, rows_pad, D] fp32, accumulated
   int* queues;                  // the eight row-group queue counters of this launch (queues.h)
-  int L, NB, RM, W, rows, rows_pad, tier, BH, fixed;  // tier: PH_B or PH_C
+  int L, NB, RM, W, BH, fixed;
+  int tail_groups, groups;      // 64-row groups of a head: tier C's first, then tier B's (0: a tier left out)
   float scale_log2, scale;
 };
 
 // 64-bit mask of the tier blocks of query-block row `row` among the workgroup's blocks fb .. fb + nblk - 1 (plain
 // per-thread loads: each thread of a refill looks at its own query block)
-__device__ __forceinline__ unsigned long long tier_mask(const TabArgs& a, size_t row, int fb, int nblk) {
+__device__ __forceinline__ unsigned long long tier_mask(const TabArgs& a, bool tier_b, size_t row, int fb, int nblk) {
   const int w0 = fb >> 5;
   auto word = [&](int w) -> unsigned long long {
     if (w >= a.W) return 0ull;
     const unsigned abv = a.bits_ab[row * a.W + w];
-    unsigned m = a.tier == PH_B ? (abv & ~a.bits_a[row * a.W + w]) : ~abv;
+    unsigned m = tier_b ? (abv & ~a.bits_a[row * a.W + w]) : ~abv;
     const int lo = w * 32;
     if (a.NB - lo < 32) m &= (1u << (a.NB - lo)) - 1u;
     return m;
@@ -398,7 +405,11 @@ __device__ __forceinline__ unsigned long long tier_mask(const TabArgs& a, size_t
   return nblk >= 64 ? m : (m & ((1ull << nblk) - 1ull));
 }
 
-// one 512-thread workgroup per (64 table rows, head) in head-major balanced order (queues.h), one per CU, in the
+// Both tiers' row groups run in one launch, all claimed at run time: a tier-C group walks every query block and a head
+// has few of them (15 at 957 blocks), so on its own that tier left most CUs idle, and with the groups bound to the XCDs
+// of their heads a head count that eight does not divide left XCDs idle. 957 blocks, 6 heads, both tiers: 1475 + 1265
+// us in two launches of bound groups, 2310 in one. What bounds it then is the delivery of Q / dO to every row group.
+// One 512-thread workgroup per (64 table rows, head) in head-major balanced order (queues.h), one per CU, in the
 // fine KV-owner layout (2 key halves x 2 query halves) twice: a dV group of four waves (S, P, dV) and a dK group
 // (dP with the table's V rows in registers, dS from the dV group's P handed over through LDS, dK), one accumulator
 // set per wave so that two waves share a SIMD; each query block's Q / dO is staged once for both groups.
@@ -414,17 +425,20 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
   __shared__ unsigned long long am_s[RING];
   __shared__ int wcnt_s[8];
   int grp, bh;
-  if (!balanced_head_item(a.queues, a.fixed, a.rows_pad / BK, a.BH, bh, grp)) return;
+  if (!balanced_head_item(a.queues, a.fixed, a.groups, a.BH, bh, grp)) return;
+  const bool tier_b = grp >= a.tail_groups;
+  if (tier_b) grp -= a.tail_groups;
+  const Table t = tier_b ? a.mid : a.tail;
   const int tid = threadIdx.x, l = tid & 63, hi = l >> 5, lq = l & 31;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wl = wv & 3, part = wv >> 2;  // wave within its group; 0: dV, 1: dK (wave-uniform)
   const int kh = wl & 1, qh = wl >> 1;
   const int key = 32 * kh + lq;
   const int trow = grp * BK + key;  // table row of this lane's key
-  const int per_blk = a.tier == PH_B ? a.RM : 1;
+  const int per_blk = tier_b ? a.RM : 1;
   const int fb = grp * BK / per_blk, nblk = BK / per_blk;
   const int lblk = key / per_blk;   // block of this key within the workgroup's blocks
-  const float kbias = trow < a.rows ? a.lc[(size_t)bh * a.lc_stride + trow] : -INFINITY;
+  const float kbias = trow < t.rows ? t.lc[(size_t)bh * t.lc_stride + trow] : -INFINITY;
   const size_t head = (size_t)bh * a.L;
 
   const unsigned head_bytes = (unsigned)((size_t)a.L * HD * 2);
@@ -438,11 +452,11 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
   }
   ev8 kreg[8], vreg[8];
   {
-    const size_t off = ((size_t)bh * a.rows_pad + trow) * HD + 8 * hi;
+    const size_t off = ((size_t)bh * t.rows_pad + trow) * HD + 8 * hi;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      if (part == 0) kreg[ks] = *reinterpret_cast<const ev8*>(a.k_tab + off + 16 * ks);
-      else vreg[ks] = *reinterpret_cast<const ev8*>(a.v_tab + off + 16 * ks);
+      if (part == 0) kreg[ks] = *reinterpret_cast<const ev8*>(t.k + off + 16 * ks);
+      else vreg[ks] = *reinterpret_cast<const ev8*>(t.v + off + 16 * ks);
     }
   }
   // (wave 0 also loads the block's raw LSE and delta; `stats` turns them into what st_s holds once the transfers
@@ -453,9 +467,9 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) dma16(part ? rd : rq, qd_s[sb][part] + wl * 4096 + r * 1024, ld_off[r], soff);
     if (wv == 0) {
-      const size_t t = head + (size_t)i * BK + l;
-      lv = a.lse[t];
-      dl = a.delta[t];
+      const size_t r = head + (size_t)i * BK + l;
+      lv = a.lse[r];
+      dl = a.delta[r];
     }
   };
   auto stats = [&](int sb, float lv, float dl) {  // wave 0, after dma_wait()
@@ -466,7 +480,7 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
   int produced = 0, chunk = 0;  // ring entries written so far, query-block chunks (of 256) scanned so far
   auto refill = [&]() {         // every thread (the masks from the first 256); ends with a barrier
     const int i = chunk * 256 + tid;
-    const unsigned long long m = (tid < 256 && i < a.NB) ? tier_mask(a, (size_t)bh * a.NB + i, fb, nblk) : 0ull;
+    const unsigned long long m = (tid < 256 && i < a.NB) ? tier_mask(a, tier_b, (size_t)bh * a.NB + i, fb, nblk) : 0ull;
     const unsigned long long bal = __builtin_amdgcn_ballot_w64(m != 0ull);
     if (l == 0) wcnt_s[wv] = __popcll(bal);
     __syncthreads();
@@ -584,7 +598,7 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
   }
   __syncthreads();
   if (qh == 1) return;
-  float* g = (part == 0 ? a.dv_tab : a.dk_tab) + ((size_t)bh * a.rows_pad + trow) * HD;
+  float* g = (part == 0 ? t.dv : t.dk) + ((size_t)bh * t.rows_pad + trow) * HD;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -821,6 +835,41 @@ extern "C" int ES_VSA_API(vsa_rep_attn_bwd_q)(const void* q, const void* k, cons
   return check_launch("vsa_rep_attn_bwd_q");
 }
 
+static TabArgs tab_args(const void* q, const void* dout, const float* lse, const float* delta, const unsigned* bits_a,
+                        const unsigned* bits_ab, int BH, int L, int D, int RM) {
+  TabArgs a = {};
+  a.q = (const e16_t*)q;
+  a.dout = (const e16_t*)dout;
+  a.lse = lse;
+  a.delta = delta;
+  a.bits_a = bits_a;
+  a.bits_ab = bits_ab;
+  a.L = L;
+  a.NB = L / BK;
+  a.RM = RM;
+  a.W = (a.NB + 31) / 32;
+  a.BH = BH;
+  a.scale_log2 = LOG2E / sqrtf((float)D);
+  a.scale = 1.0f / sqrtf((float)D);
+  return a;
+}
+
+static Table table(const void* k, const void* v, const float* lc, int lc_stride, float* dk, float* dv, int rows) {
+  return Table{(const e16_t*)k, (const e16_t*)v, lc, lc_stride, dk, dv, rows, (rows + 63) / 64 * 64};
+}
+
+static int launch_tables(TabArgs& a, hipStream_t stream) {
+  a.tail_groups = a.tail.rows_pad / BK;
+  a.groups = a.tail_groups + a.mid.rows_pad / BK;
+  Queues qs;
+  ES_REQUIRE(balanced_launch_queues((a.BH + 7) / 8 * a.groups, stream, qs, 0, true), ES_ERR_LAUNCH,
+             "VSA2-rep: row-group queues unavailable");
+  a.queues = qs.counters;
+  a.fixed = qs.fixed;
+  hipLaunchKernelGGL(rep_bwd_tab_kernel, dim3((unsigned)qs.grid), dim3(512), 0, stream, a);
+  return check_launch("vsa_rep_bwd_tables");
+}
+
 extern "C" int ES_VSA_API(vsa_rep_bwd_tables)(const void* q, const void* dout, const void* k_tab, const void* v_tab,
                                   const float* lc, int lc_stride, const float* lse, const float* delta,
                                   const unsigned* bits_a, const unsigned* bits_ab, float* dk_tab, float* dv_tab,
@@ -831,36 +880,26 @@ extern "C" int ES_VSA_API(vsa_rep_bwd_tables)(const void* q, const void* dout, c
   ES_REQUIRE(tier == 2 || tier == 4, ES_ERR_INVALID, "VSA2-rep: tier must be 2 (B, mid table) or 4 (C, tail table)");
   ES_REQUIRE(lc_stride == 0 || lc_stride >= (L / BK) * (tier == 2 ? RM : 1), ES_ERR_INVALID,
              "VSA2-rep: lc_stride must be 0 (shared) or >= the table's rows (NB * RM for tier 2, NB for tier 4)");
-  TabArgs a = {};
-  a.q = (const e16_t*)q;
-  a.dout = (const e16_t*)dout;
-  a.k_tab = (const e16_t*)k_tab;
-  a.v_tab = (const e16_t*)v_tab;
-  a.lc = lc;
-  a.lc_stride = lc_stride;
-  a.lse = lse;
-  a.delta = delta;
-  a.bits_a = bits_a;
-  a.bits_ab = bits_ab;
-  a.dk_tab = dk_tab;
-  a.dv_tab = dv_tab;
-  a.L = L;
-  a.NB = L / BK;
-  a.RM = RM;
-  a.W = (a.NB + 31) / 32;
-  a.tier = tier;
-  a.rows = tier == 2 ? a.NB * RM : a.NB;
-  a.rows_pad = (a.rows + 63) / 64 * 64;
-  a.scale_log2 = LOG2E / sqrtf((float)D);
-  a.scale = 1.0f / sqrtf((float)D);
-  a.BH = BH;
-  const int per_queue = (BH + 7) / 8 * (a.rows_pad / BK);
-  Queues qs;
-  ES_REQUIRE(balanced_launch_queues(per_queue, stream, qs, 256), ES_ERR_LAUNCH, "VSA2-rep: row-group queues unavailable");
-  a.queues = qs.counters;
-  a.fixed = qs.fixed;
-  hipLaunchKernelGGL(rep_bwd_tab_kernel, dim3((unsigned)qs.grid), dim3(512), 0, stream, a);
-  return check_launch("vsa_rep_bwd_tables");
+  TabArgs a = tab_args(q, dout, lse, delta, bits_a, bits_ab, BH, L, D, RM);
+  (tier == 2 ? a.mid : a.tail) = table(k_tab, v_tab, lc, lc_stride, dk_tab, dv_tab, (L / BK) * (tier == 2 ? RM : 1));
+  return launch_tables(a, stream);
+}
+
+extern "C" int ES_VSA_API(vsa_rep_bwd_both_tables)(const void* q, const void* dout, const void* k_mid, const void* v_mid,
+                                  const float* lc_mid, int lc_mid_stride, const void* k_tail, const void* v_tail,
+                                  const float* lc_tail, const float* lse, const float* delta, const unsigned* bits_a,
+                                  const unsigned* bits_ab, float* dk_mid, float* dv_mid, float* dk_tail,
+                                  float* dv_tail, int BH, int L, int D, int RM, hipStream_t stream) {
+  if (int st = rep_check(BH, L, D, RM)) return st;
+  ES_REQUIRE(q && dout && k_mid && v_mid && lc_mid && k_tail && v_tail && lc_tail && lse && delta && bits_a && bits_ab &&
+                 dk_mid && dv_mid && dk_tail && dv_tail,
+             ES_ERR_INVALID, "VSA2-rep: null tensor pointer");
+  ES_REQUIRE(lc_mid_stride == 0 || lc_mid_stride >= (L / BK) * RM, ES_ERR_INVALID,
+             "VSA2-rep: lc_mid_stride must be 0 (shared) or >= NB * RM (per head)");
+  TabArgs a = tab_args(q, dout, lse, delta, bits_a, bits_ab, BH, L, D, RM);
+  a.mid = table(k_mid, v_mid, lc_mid, lc_mid_stride, dk_mid, dv_mid, (L / BK) * RM);
+  a.tail = table(k_tail, v_tail, lc_tail, 0, dk_tail, dv_tail, L / BK);
+  return launch_tables(a, stream);
 }
 
 extern "C" int ES_VSA_API(vsa_rep_unpool)(const float* acc_k, const float* acc_v, const float* dk_mid, const float* dv_mid,

@@ -648,19 +648,19 @@ def rep_attn_bwd_q(q, k, v, k_mid, v_mid, lc_mid, k_tail, v_tail, lc_tail, dout,
               q2k_idx, bits_a, bits_ab, blk_cnt, _wide(add_dq), add_dq.shape[2] if add_dq is not None else 0, acc.w,
               dq, B * H, L, D, int(mid_reps), int(phases))
     acc.put()
-    if phases & 2:
-        dkm, dvm = _InPlace(dk_mid), _InPlace(dv_mid)
-        _call("vsa_rep_bwd_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), lse, delta, bits_a, bits_ab,
-                  dkm.w, dvm.w,
-                  B * H, L, D, int(mid_reps), 2)
-        dkm.put()
-        dvm.put()
-    if phases & 4:
-        dkt, dvt = _InPlace(dk_tail), _InPlace(dv_tail)
-        _call("vsa_rep_bwd_tables", q, dout, k_tail, v_tail, lc_tail, 0, lse, delta, bits_a, bits_ab, dkt.w, dvt.w,
-                  B * H, L, D, int(mid_reps), 4)
-        dkt.put()
-        dvt.put()
+    stats = (lse, delta, bits_a, bits_ab)
+    mids, tails = [_InPlace(dk_mid), _InPlace(dv_mid)], [_InPlace(dk_tail), _InPlace(dv_tail)]
+    if phases & 2 and phases & 4:
+        _call("vsa_rep_bwd_both_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), k_tail, v_tail, lc_tail,
+              *stats, mids[0].w, mids[1].w, tails[0].w, tails[1].w, B * H, L, D, int(mid_reps))
+    elif phases & 2:
+        _call("vsa_rep_bwd_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), *stats, mids[0].w, mids[1].w,
+              B * H, L, D, int(mid_reps), 2)
+    elif phases & 4:
+        _call("vsa_rep_bwd_tables", q, dout, k_tail, v_tail, lc_tail, 0, *stats, tails[0].w, tails[1].w, B * H, L, D,
+              int(mid_reps), 4)
+    for t in (mids if phases & 2 else []) + (tails if phases & 4 else []):
+        t.put()
     return _narrow(dq, D)
 
 
