@@ -89,6 +89,13 @@ int es_dense_attention(const void* q, const void* k, const void* v, void* out, f
 int es_dense_attention_kv(const void* q, const void* k, const void* v, void* out, float* lse2, int Lq, int Lk,
                           int H, int D, hipStream_t stream);
 
+/* Dense attention as es_dense_attention_kv for callers that can hand over device workspace: with few query tiles and
+ * heads the keys are cut into ranges that run side by side and are merged in order. es_dense_attention_workspace gives
+ * the bytes it needs (0: it runs unsplit and needs none). */
+size_t es_dense_attention_workspace(int Lq, int Lk, int H);
+int es_dense_attention_ws(const void* q, const void* k, const void* v, void* out, float* lse2, void* workspace,
+                          size_t workspace_bytes, int Lq, int Lk, int H, int D, hipStream_t stream);
+
 /* ---------------------------------------------------------------- EchoSparse map, scales and plans */
 
 /* Mean key and value of every 64-token block (tail divided by its token count), bf16.

@@ -10,6 +10,7 @@ stream (workspace sizes, limits, the error string) and tests that drive the C AB
 There is no fallback: if either library is missing or fails to load, every kernel call raises.
 """
 import ctypes
+import functools
 import numbers
 import os
 
@@ -34,6 +35,7 @@ SIGNATURES = {
     "es_compensate_fallback": [P, P, P, P, P, P, P, I, I, I],
     "es_dense_attention": [P, P, P, P, P, I, I, I],
     "es_dense_attention_kv": [P, P, P, P, P, I, I, I, I],
+    "es_dense_attention_ws": [P, P, P, P, P, P, Z, I, I, I, I],
     "es_block_means": [P, P, P, P, I, I, I],
     "es_estimate_skipped": [P, P, P, P, P, P, P, P, I, I, I],
     "es_full_step_scales": [P, P, P, P, I, I],
@@ -82,7 +84,8 @@ F16_TWINS = ("vsa_pool", "vsa_fuse_fwd", "vsa_fuse_bwd", "vsa_finalize", "vsa_at
              "vsa_split_merge_sum", "vsa_rep_build", "vsa_rep_build_kmeans", "vsa_rep_attn_fwd", "vsa_rep_attn_bwd_q", "vsa_rep_bwd_tables",
              "vsa_rep_bwd_both_tables", "vsa_rep_unpool", "vsa_row_dot")
 SIGNATURES.update({n + "_f16": SIGNATURES[n] for n in F16_TWINS})
-NO_STREAM = {"es_representatives_workspace": ([I, I, I], Z), "es_representatives_noalloc_limit": ([], Z), "es_last_error_string": ([], ctypes.c_char_p),
+NO_STREAM = {"es_representatives_workspace": ([I, I, I], Z), "es_dense_attention_workspace": ([I, I, I], Z),
+             "es_representatives_noalloc_limit": ([], Z), "es_last_error_string": ([], ctypes.c_char_p),
              "es_abi_version": ([], I), "vsa_topk_workspace": ([I, I], Z)}
 
 _lib = None
@@ -151,3 +154,8 @@ def workspace_bytes(L, H, D):
 
 def topk_workspace_bytes(bh_count, NB):
     return int(lib().vsa_topk_workspace(bh_count, NB))
+
+
+@functools.lru_cache(maxsize=1024)
+def dense_workspace_bytes(Lq, Lk, H):
+    return int(lib().es_dense_attention_workspace(Lq, Lk, H))

@@ -46,7 +46,8 @@ def dense_attention(q, k, v, return_lse=False):
         else:
             out, lse2 = gfx950.dense_attention_kv(q[b], k[b], v[b])
         outs.append(out)
-        lses.append(lse2[:Lq].t() / LOG2E)
+        if return_lse:
+            lses.append(lse2[:Lq].t() / LOG2E)
     out = outs[0][None] if B == 1 else torch.stack(outs)
     if not return_lse:
         return out

@@ -18,6 +18,7 @@
 #include "common.h"
 #include "queues.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace es {
@@ -51,6 +52,8 @@ struct AttnArgs {
   float* mass;
   int* queues;  // FIXED: the eight tile-queue counters of this launch (queues.h)
   int fixed;    // items per queue bound to dispatch slots; FIXED launches claim the rest
+  float* part;  // split dense launches: per (key range, tile, head) the tile's O [128][128], then m and l [128] each
+  int splits;   // key ranges of a split dense launch
   int L, Lk, H, nq, nb, NK, RW, tiles, per_xcd;  // L query rows, Lk key rows (Lk == L but in dense_kv)
   float threshold, tail_log2, scale;
 };
@@ -62,9 +65,11 @@ struct ChunkIds {
 };
 
 
-// one (query tile t, head h)
-template <int MODE, bool COMP, bool MASS>
-__device__ __forceinline__ void attn_tile(const AttnArgs& a, const int h, const int t) {
+constexpr int PART = BM * HD + 2 * BM;  // floats of one partial: O, m, l
+
+// one (query tile t, head h); PARTIAL: its unnormalised O, running maximum and row sum go to `part`
+template <int MODE, bool COMP, bool MASS, bool PARTIAL = false>
+__device__ __forceinline__ void attn_tile(const AttnArgs& a, const int h, const int t, float* part = nullptr) {
   __shared__ __attribute__((aligned(16))) char kv_s[2][2][BK * 256];
   __shared__ __attribute__((aligned(16))) float bias_s[2][BK];
   __shared__ float mass_s[16][129];  // [wave * 4 + row of 16 lanes][chunk % 128], rows padded against bank conflicts
@@ -588,6 +593,20 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, const int h, const 
 
   // ---------------------------------------------------------------- epilogue
   const float tot = sum_xor32(lsum);
+  if (PARTIAL) {
+    const int r = wv * 32 + lq;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(part + r * HD + 32 * db + 8 * i + 4 * hi) =
+            f32x4{o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]};
+    if (hi == 0) {
+      part[BM * HD + r] = mrun;
+      part[BM * HD + BM + r] = tot;
+    }
+    return;
+  }
   bf16_t* orow = a.out + ((size_t)(rvalid ? row : 0) * H + h) * HD;
   float* lrow = a.lse + (size_t)row * H + h;
   auto store_rows = [&](float inv) {
@@ -658,6 +677,79 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnArgs a) {
   const int t = ((x + h) & 7) * a.per_xcd + k % a.per_xcd;
   if (h >= a.H || t >= a.tiles) return;
   attn_tile<MODE, COMP, MASS>(a, h, t);
+}
+
+// Dense attention with few (tile, head) items: each item's keys are cut into `splits` ranges of whole blocks, one
+// workgroup each, and merge_parts_kernel combines the partials. A workgroup walks its keys one 64-key chunk after the
+// other (1.4 us each), so with fewer items than CUs the time is the chunk count, whatever the GPU could do beside it.
+__global__ __launch_bounds__(256, 2) void attn_split_kernel(AttnArgs a) {
+  const int items = a.tiles * a.H, w = blockIdx.x;
+  const int s = w / items, it = w - s * items, h = it / a.tiles, t = it - h * a.tiles;
+  const int c0 = (int)((long long)s * a.nb / a.splits), c1 = (int)((long long)(s + 1) * a.nb / a.splits);
+  AttnArgs b = a;  // the same problem over the key blocks c0 .. c1 - 1
+  b.k = a.k + (size_t)c0 * BK * a.H * HD;
+  b.v = a.v + (size_t)c0 * BK * a.H * HD;
+  b.Lk = min(a.Lk, c1 * BK) - c0 * BK;
+  b.nb = c1 - c0;
+  attn_tile<ONLINE, false, false, true>(b, h, t, a.part + (size_t)w * PART);
+}
+
+// O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s and the log2 LSE, the ranges in order; grid (items, 16): eight rows
+// a workgroup, 32 lanes a row, so that a row's loads are all in flight at once however few items there are
+constexpr int MAX_SPLITS = 16;
+__global__ __launch_bounds__(256) void merge_parts_kernel(AttnArgs a) {
+  const int items = a.tiles * a.H, it = blockIdx.x, h = it / a.tiles, t = it - h * a.tiles;
+  const int r = blockIdx.y * 8 + (threadIdx.x >> 5), c4 = (threadIdx.x & 31) * 4, row = t * BM + r;
+  float* lrow = a.lse + (size_t)row * a.H + h;
+  if (row >= a.L) {
+    if (c4 == 0) *lrow = 1e30f;
+    return;
+  }
+  const float* part = a.part + (size_t)it * PART;
+  const size_t step = (size_t)items * PART;
+  float m[MAX_SPLITS], l[MAX_SPLITS];
+  f32x4 x[MAX_SPLITS];
+#pragma unroll
+  for (int s = 0; s < MAX_SPLITS; ++s) {
+    const float* p = part + s * step;
+    const bool in = s < a.splits;
+    m[s] = in ? p[BM * HD + r] : -INFINITY;
+    l[s] = in ? p[BM * HD + BM + r] : 0.0f;
+    x[s] = in ? *reinterpret_cast<const f32x4*>(p + r * HD + c4) : f32x4{};
+  }
+  float M = m[0];
+#pragma unroll
+  for (int s = 1; s < MAX_SPLITS; ++s) M = fmaxf(M, m[s]);
+  const float msub = M == -INFINITY ? 0.0f : M;
+  f32x4 acc = {};
+  float sum = 0.0f;
+#pragma unroll
+  for (int s = 0; s < MAX_SPLITS; ++s) {
+    const float w = exp2f_fast(m[s] - msub);
+    sum = fmaf(w, l[s], sum);
+    acc += w * x[s];
+  }
+  const float inv = 1.0f / sum;
+  ushort4 v4;
+  v4.x = f2bf(acc[0] * inv);
+  v4.y = f2bf(acc[1] * inv);
+  v4.z = f2bf(acc[2] * inv);
+  v4.w = f2bf(acc[3] * inv);
+  *reinterpret_cast<ushort4*>(a.out + ((size_t)row * a.H + h) * HD + c4) = v4;
+  if (c4 == 0) *lrow = M + log2f(sum);
+}
+
+// Key ranges of a dense launch: as many as fill the 512 workgroups the GPU holds, each of at least four key blocks, two
+// ranges only from sixteen blocks on (the partials cost 64 KB a range and the merge a launch of 6 to 10 us); 1 (no
+// split) from 257 items on, where every CU has one. Queries x keys x heads, unsplit -> split: 3925 x 3925 x 1 90 -> 29
+// us, 256 x 33000 x 24 700 -> 164, 1537 x 1537 x 12 48 -> 39, 287 x 808 x 24 31 -> 20, 3329 x 3329 x 5 83 -> 57; in two
+// ranges of four blocks nothing (1280 x 512 x 24 31 -> 32).
+static int dense_splits(int Lq, int Lk, int H) {
+  const long long items = (long long)((Lq + BM - 1) / BM) * H;
+  const int nb = (Lk + BK - 1) / BK;
+  if (items > 256 || nb < 8) return 1;
+  const int S = (int)std::min<long long>(std::min<long long>(512 / items, MAX_SPLITS), nb / 4);
+  return S == 2 && nb < 16 ? 1 : std::max(S, 1);
 }
 
 template <int MODE, bool COMP, bool MASS>
@@ -824,4 +916,31 @@ extern "C" int es_dense_attention_kv(const void* q, const void* k, const void* v
   a.out = (bf16_t*)out;
   a.lse = lse2;
   return launch<ONLINE, false, false>(a, stream, "es_dense_attention_kv");
+}
+
+extern "C" size_t es_dense_attention_workspace(int Lq, int Lk, int H) {
+  if (Lq <= 0 || Lk <= 0 || H <= 0) return 0;
+  const int S = dense_splits(Lq, Lk, H);
+  return S <= 1 ? 0 : (size_t)S * ((Lq + BM - 1) / BM) * H * PART * sizeof(float);
+}
+
+extern "C" int es_dense_attention_ws(const void* q, const void* k, const void* v, void* out, float* lse2, void* workspace,
+                                     size_t workspace_bytes, int Lq, int Lk, int H, int D, hipStream_t stream) {
+  const size_t need = es_dense_attention_workspace(Lq, Lk, H);
+  if (need == 0) return es_dense_attention_kv(q, k, v, out, lse2, Lq, Lk, H, D, stream);
+  int st = check_common(q, k, v, Lq, H, D);
+  if (st) return st;
+  ES_REQUIRE(out && lse2 && workspace, ES_ERR_INVALID, "null tensor pointer");
+  ES_REQUIRE(workspace_bytes >= need, ES_ERR_INVALID, "workspace too small");
+  AttnArgs a = base_args(q, k, v, Lq, H);
+  a.Lk = Lk;
+  a.nb = (Lk + BK - 1) / BK;
+  a.out = (bf16_t*)out;
+  a.lse = lse2;
+  a.part = (float*)workspace;
+  a.splits = dense_splits(Lq, Lk, H);
+  const int items = a.tiles * H;
+  hipLaunchKernelGGL(attn_split_kernel, dim3(items * a.splits), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(merge_parts_kernel, dim3(items, BM / 8), dim3(256), 0, stream, a);
+  return check_launch("es_dense_attention_ws");
 }

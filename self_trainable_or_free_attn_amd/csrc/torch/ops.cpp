@@ -125,6 +125,15 @@ static void op_es_dense_attention_kv(const c10::optional<at::Tensor>& q, const c
 }
 static void meta_es_dense_attention_kv(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& k, const c10::optional<at::Tensor>& v, const c10::optional<at::Tensor>& out, const c10::optional<at::Tensor>& lse2, int64_t Lq, int64_t Lk, int64_t H, int64_t D) {}
 
+static void op_es_dense_attention_ws(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& k, const c10::optional<at::Tensor>& v, const c10::optional<at::Tensor>& out, const c10::optional<at::Tensor>& lse2, const c10::optional<at::Tensor>& workspace, int64_t workspace_bytes, int64_t Lq, int64_t Lk, int64_t H, int64_t D) {
+  const Call es_op_call("es_dense_attention_ws", {&q, &k, &v, &out, &lse2, &workspace});
+  c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
+  const hipStream_t es_op_stream =
+      es_op_call.dev ? c10::hip::getCurrentHIPStream(es_op_call.dev->index()).stream() : nullptr;
+  es_op_check("es_dense_attention_ws", es_dense_attention_ws(static_cast<const void*>(es_op_data("es_dense_attention_ws", "q", q, ES_HALF)), static_cast<const void*>(es_op_data("es_dense_attention_ws", "k", k, ES_HALF)), static_cast<const void*>(es_op_data("es_dense_attention_ws", "v", v, ES_HALF)), static_cast<void*>(es_op_data("es_dense_attention_ws", "out", out, ES_OUT)), static_cast<float*>(es_op_data("es_dense_attention_ws", "lse2", lse2, ES_F32)), static_cast<void*>(es_op_data("es_dense_attention_ws", "workspace", workspace, ES_ANY)), static_cast<size_t>(es_op_int("es_dense_attention_ws", "workspace_bytes", workspace_bytes, ES_SIZE)), static_cast<int>(es_op_int("es_dense_attention_ws", "Lq", Lq, ES_INT)), static_cast<int>(es_op_int("es_dense_attention_ws", "Lk", Lk, ES_INT)), static_cast<int>(es_op_int("es_dense_attention_ws", "H", H, ES_INT)), static_cast<int>(es_op_int("es_dense_attention_ws", "D", D, ES_INT)), es_op_stream));
+}
+static void meta_es_dense_attention_ws(const c10::optional<at::Tensor>& q, const c10::optional<at::Tensor>& k, const c10::optional<at::Tensor>& v, const c10::optional<at::Tensor>& out, const c10::optional<at::Tensor>& lse2, const c10::optional<at::Tensor>& workspace, int64_t workspace_bytes, int64_t Lq, int64_t Lk, int64_t H, int64_t D) {}
+
 static void op_es_block_means(const c10::optional<at::Tensor>& k, const c10::optional<at::Tensor>& v, const c10::optional<at::Tensor>& k_mean, const c10::optional<at::Tensor>& v_mean, int64_t L, int64_t H, int64_t D) {
   const Call es_op_call("es_block_means", {&k, &v, &k_mean, &v_mean});
   c10::OptionalDeviceGuard es_op_guard(es_op_call.dev);
@@ -708,6 +717,7 @@ TORCH_LIBRARY(echosparse_gfx950, m) {
   m.def("es_compensate_fallback(Tensor? q, Tensor? k_mean, Tensor? v_mean, Tensor? keep, Tensor(a!)? lse, Tensor(b!)? out, Tensor? flags, int L, int H, int D) -> ()");
   m.def("es_dense_attention(Tensor? q, Tensor? k, Tensor? v, Tensor(a!)? out, Tensor(b!)? lse2, int L, int H, int D) -> ()");
   m.def("es_dense_attention_kv(Tensor? q, Tensor? k, Tensor? v, Tensor(a!)? out, Tensor(b!)? lse2, int Lq, int Lk, int H, int D) -> ()");
+  m.def("es_dense_attention_ws(Tensor? q, Tensor? k, Tensor? v, Tensor(a!)? out, Tensor(b!)? lse2, Tensor(c!)? workspace, int workspace_bytes, int Lq, int Lk, int H, int D) -> ()");
   m.def("es_block_means(Tensor? k, Tensor? v, Tensor(a!)? k_mean, Tensor(b!)? v_mean, int L, int H, int D) -> ()");
   m.def("es_estimate_skipped(Tensor? q, Tensor? k_mean, Tensor? keep, Tensor? offset, Tensor? lse, Tensor(a!)? mass, Tensor(b!)? scale_exact, Tensor(c!)? scale_skip, int L, int H, int D) -> ()");
   m.def("es_full_step_scales(Tensor? offset, Tensor(a!)? lse, Tensor(b!)? scale_exact, Tensor(c!)? scale_skip, int L, int H) -> ()");
@@ -780,6 +790,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CUDA, m) {
   m.impl("es_compensate_fallback", TORCH_FN(op_es_compensate_fallback));
   m.impl("es_dense_attention", TORCH_FN(op_es_dense_attention));
   m.impl("es_dense_attention_kv", TORCH_FN(op_es_dense_attention_kv));
+  m.impl("es_dense_attention_ws", TORCH_FN(op_es_dense_attention_ws));
   m.impl("es_block_means", TORCH_FN(op_es_block_means));
   m.impl("es_estimate_skipped", TORCH_FN(op_es_estimate_skipped));
   m.impl("es_full_step_scales", TORCH_FN(op_es_full_step_scales));
@@ -852,6 +863,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, CPU, m) {
   m.impl("es_compensate_fallback", TORCH_FN(op_es_compensate_fallback));
   m.impl("es_dense_attention", TORCH_FN(op_es_dense_attention));
   m.impl("es_dense_attention_kv", TORCH_FN(op_es_dense_attention_kv));
+  m.impl("es_dense_attention_ws", TORCH_FN(op_es_dense_attention_ws));
   m.impl("es_block_means", TORCH_FN(op_es_block_means));
   m.impl("es_estimate_skipped", TORCH_FN(op_es_estimate_skipped));
   m.impl("es_full_step_scales", TORCH_FN(op_es_full_step_scales));
@@ -924,6 +936,7 @@ TORCH_LIBRARY_IMPL(echosparse_gfx950, Meta, m) {
   m.impl("es_compensate_fallback", TORCH_FN(meta_es_compensate_fallback));
   m.impl("es_dense_attention", TORCH_FN(meta_es_dense_attention));
   m.impl("es_dense_attention_kv", TORCH_FN(meta_es_dense_attention_kv));
+  m.impl("es_dense_attention_ws", TORCH_FN(meta_es_dense_attention_ws));
   m.impl("es_block_means", TORCH_FN(meta_es_block_means));
   m.impl("es_estimate_skipped", TORCH_FN(meta_es_estimate_skipped));
   m.impl("es_full_step_scales", TORCH_FN(meta_es_full_step_scales));

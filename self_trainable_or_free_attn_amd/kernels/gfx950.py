@@ -128,13 +128,23 @@ def rebuild_plan(exact_bits, skip_bits, keep, counts, blocks, refine, refine_cou
               refine_counts, refine.shape[-1], means, mean_counts, H, nq, nb)
 
 
+def _dense(q, k, v, out, lse, Lq, Lk, H, D):
+    """Dense attention into out / lse; few query tiles and heads run over key ranges side by side, in a workspace."""
+    n = _lib.dense_workspace_bytes(Lq, Lk, H)
+    if n == 0:
+        _lib.call("es_dense_attention_kv", q, k, v, out, lse, Lq, Lk, H, D)
+    else:
+        ws = torch.empty(n, device=q.device, dtype=torch.uint8)
+        _lib.call("es_dense_attention_ws", q, k, v, out, lse, ws, n, Lq, Lk, H, D)
+
+
 def dense_attention(q, k, v):
     """Dense attention over all keys: returns (out (L, H, D) bf16, lse (nq * 128, H) float32 in log2 units with
     1e30 past L) -- the replacement of the FlashAttention-4 call that seeds the offsets."""
     L, H, D = _check_qkv(q, k, v)
     out = torch.empty_like(q)
     lse = torch.empty(_cdiv(L, BM) * BM, H, device=q.device, dtype=torch.float32)
-    _lib.call("es_dense_attention", q, k, v, out, lse, L, H, D)
+    _dense(q, k, v, out, lse, L, L, H, D)
     return out, lse
 
 
@@ -146,7 +156,7 @@ def dense_attention_kv(q, k, v):
     assert k.shape == v.shape == (Lk, H, D), "k and v must be (Lk, H, 128) with q's heads"
     out = torch.empty_like(q)
     lse = torch.empty(_cdiv(Lq, BM) * BM, H, device=q.device, dtype=torch.float32)
-    _lib.call("es_dense_attention_kv", q, k, v, out, lse, Lq, Lk, H, D)
+    _dense(q, k, v, out, lse, Lq, Lk, H, D)
     return out, lse
 
 
