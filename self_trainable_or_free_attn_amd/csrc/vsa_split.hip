@@ -11,8 +11,11 @@
 //            of cnt) + j; then one direct task (slot -1) per other row, in row order
 //   merges : one {r, first slot, c, 0} per split row; info = {tasks, split rows, split slots, NR, E, E <= budget,
 //            thr without the per-(b, h) term, W}
-// One workgroup of 1024 threads plans the whole list: each thread owns a contiguous run of rows, and three
-// workgroup scans give every thread its slot, task and merge bases. Nothing is read back to the host.
+// One workgroup of 1024 threads plans the whole list: each thread owns a contiguous run of rows, and two workgroup
+// scans give every thread its slot, task and merge bases. Nothing is read back to the host. What bounds it is one
+// CU's instructions and the latency of a thread's list pointers: a row costs no division (its head and the head's
+// threshold move along) and PLAN_ROWS rows' pointers are loaded together (with a division, a double-precision
+// threshold and a wait per row: 67 us for 9 456 rows, 53 now, most of it the task stores of one CU).
 //
 // Merges (one workgroup per split row, in chunk order: deterministic):
 //   forward : o = sum_i 2^(lse_i - M) o_i / sum_i 2^(lse_i - M), lse = (M + log2 sum) ln 2 (reference
@@ -29,6 +32,7 @@ namespace es {
 namespace {
 
 constexpr int PLAN_THREADS = 1024;
+constexpr int PLAN_ROWS = 8;  // rows of a thread whose list pointers are loaded together
 
 struct PlanArgs {
   const int* ptr;
@@ -68,61 +72,84 @@ __global__ __launch_bounds__(PLAN_THREADS) void plan_kernel(PlanArgs a) {
   const long long W = (long long)a.ptr[(size_t)a.BH * (a.NB + 1) - 1] - a.ptr[0];
   int gthr = max(a.chunk + 1, a.min_len);
   if (a.tail_frac > 0.0) gthr = max(gthr, (int)ceil(a.tail_frac * (double)W / (double)a.resident));
-  auto row = [&](int r, int& beg, int& n, int& c) {
-    const int bh = r / a.NB, i = r - bh * a.NB;
+  auto head_thr = [&](int bh) {
+    if (!(a.rel_mean > 0.0) || bh >= a.BH) return gthr;
     const int* hp = a.ptr + (size_t)bh * (a.NB + 1);
-    beg = hp[i];
-    n = hp[i + 1] - beg;
-    int thr = gthr;
-    if (a.rel_mean > 0.0) thr = max(thr, (int)ceil(a.rel_mean * (double)(hp[a.NB] - hp[0]) / (double)a.NB));
-    c = n >= thr ? (n + a.chunk - 1) / a.chunk : 0;
+    return max(gthr, (int)ceil(a.rel_mean * (double)(hp[a.NB] - hp[0]) / (double)a.NB));
   };
-  // 1: chunk counts and eligible rows
-  long long cnt_mine = 0, elig_mine = 0;
-  for (int r = r0; r < r1; ++r) {
-    int beg, n, c;
-    row(r, beg, n, c);
-    cnt_mine += c;
-    elig_mine += c > 0;
-  }
-  long long cnt_tot, E;
-  const long long cnt_before = plan_scan(cnt_mine, red, &cnt_tot);
-  plan_scan(elig_mine, red, &E);
-  const bool ok = E <= (long long)a.budget;
-  // 2: split rows, split chunks, direct rows of this thread
-  long long split_mine = 0, chunks_mine = 0, direct_mine = 0;
-  {
-    long long incl = cnt_before;
-    for (int r = r0; r < r1; ++r) {
-      int beg, n, c;
-      row(r, beg, n, c);
-      incl += c;
-      const bool split = ok && c > 0 && incl <= a.max_slots;
-      split_mine += split;
-      chunks_mine += split ? c : 0;
-      direct_mine += split ? 0 : 1;
+  const int bh0 = r0 / a.NB, i0 = r0 - bh0 * a.NB, thr0 = head_thr(bh0);
+  // f(row, list begin, list length, chunks) for this thread's rows in order; row r of head bh starts at ptr[r + bh]
+  auto each_row = [&](auto&& f) {
+    int bl = bh0, il = i0, bh = bh0, i = i0, thr = thr0;
+    for (int rb = r0; rb < r1; rb += PLAN_ROWS) {
+      int beg[PLAN_ROWS], end[PLAN_ROWS];
+#pragma unroll
+      for (int k = 0; k < PLAN_ROWS; ++k) {
+        const size_t at = rb + k < r1 ? (size_t)(rb + k) + bl : 0;
+        beg[k] = a.ptr[at];
+        end[k] = a.ptr[at + 1];
+        if (++il == a.NB) {
+          il = 0;
+          ++bl;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < PLAN_ROWS; ++k) asm volatile("" : "+v"(beg[k]), "+v"(end[k]));  // (loads not sunk to uses)
+#pragma unroll
+      for (int k = 0; k < PLAN_ROWS; ++k) {
+        if (rb + k >= r1) break;
+        const int n = end[k] - beg[k];
+        f(rb + k, beg[k], n, n >= thr ? (n + a.chunk - 1) / a.chunk : 0);
+        if (++i == a.NB) {
+          i = 0;
+          thr = head_thr(++bh);
+        }
+      }
     }
-  }
-  long long nsplit, t_split, ndirect;
-  const long long split_before = plan_scan(split_mine, red, &nsplit);
-  plan_scan(chunks_mine, red, &t_split);
-  const long long direct_before = plan_scan(direct_mine, red, &ndirect);
+  };
+  // Two counts share a 64-bit scan (each is below 2^32: at most the edges plus the rows of an int32 CSR)
+  auto pair = [](unsigned lo, unsigned up) { return (long long)(((unsigned long long)up << 32) | lo); };
+  auto lo32 = [](long long x) { return (long long)(unsigned)x; };
+  auto up32 = [](long long x) { return (long long)(unsigned)((unsigned long long)x >> 32); };
+  // 1: chunk counts and eligible rows
+  unsigned cnt_mine = 0, elig_mine = 0;
+  each_row([&](int, int, int, int c) {
+    cnt_mine += (unsigned)c;
+    elig_mine += c > 0;
+  });
+  long long tot;
+  const long long cnt_before = lo32(plan_scan(pair(cnt_mine, elig_mine), red, &tot));
+  const long long E = up32(tot);
+  const bool ok = E <= (long long)a.budget;
+  // 2: split rows and their chunks before this thread (every other row is direct)
+  unsigned split_mine = 0, chunks_mine = 0;
+  long long incl = cnt_before;
+  each_row([&](int, int, int, int c) {
+    incl += c;
+    const bool split = ok && c > 0 && incl <= a.max_slots;
+    split_mine += split;
+    chunks_mine += split ? (unsigned)c : 0u;
+  });
+  const long long split_before = lo32(plan_scan(pair(split_mine, chunks_mine), red, &tot));
+  const long long nsplit = lo32(tot), t_split = up32(tot), ndirect = NR - nsplit, direct_before = r0 - split_before;
   // 3: write
-  long long incl = cnt_before, ms = split_before, dt = direct_before;
-  for (int r = r0; r < r1; ++r) {
-    int beg, n, c;
-    row(r, beg, n, c);
+  long long ms = split_before, dt = direct_before;
+  incl = cnt_before;
+  each_row([&](int r, int beg, int n, int c) {
     const long long slot0 = incl;
     incl += c;
     if (ok && c > 0 && incl <= a.max_slots) {
+      // j n / c, in 32 bits where j n fits them
+      auto cut = [&](int j) {
+        return n < 65536 ? (int)((unsigned)j * (unsigned)n / (unsigned)c) : (int)((long long)j * n / c);
+      };
       for (int j = 0; j < c; ++j)
-        a.tasks[slot0 + j] = make_int4(r, beg + (int)((long long)j * n / c), beg + (int)((long long)(j + 1) * n / c),
-                                       (int)(slot0 + j));
+        a.tasks[slot0 + j] = make_int4(r, beg + cut(j), beg + cut(j + 1), (int)(slot0 + j));
       a.merges[ms++] = make_int4(r, (int)slot0, c, 0);
     } else {
       a.tasks[t_split + dt++] = make_int4(r, beg, beg + n, -1);
     }
-  }
+  });
   if (threadIdx.x == 0) {
     a.info[0] = (int)(t_split + ndirect);
     a.info[1] = (int)nsplit;
@@ -135,7 +162,20 @@ __global__ __launch_bounds__(PLAN_THREADS) void plan_kernel(PlanArgs a) {
   }
 }
 
-// thread -> (row = tid / 4, 32 columns (tid % 4) * 32 ..)
+// Merges: grid (max_merges, 4), 16 rows of a split row block per workgroup, thread -> (row, 8 columns). The partials of
+// a row are summed in chunk order, MERGE_AHEAD of them loaded together (a thread of 32 columns with one partial in
+// flight waited for each in turn: 128 rows of 19 partials, forward 45 us, sum 34; 27, 3.4 TB/s, and 24 now).
+constexpr int MERGE_AHEAD = 8;
+
+__device__ __forceinline__ uint4 pack8e(const f32x4& x0, const f32x4& x1) {
+  uint4 u;
+  u.x = (unsigned)f2e(x0[0]) | ((unsigned)f2e(x0[1]) << 16);
+  u.y = (unsigned)f2e(x0[2]) | ((unsigned)f2e(x0[3]) << 16);
+  u.z = (unsigned)f2e(x1[0]) | ((unsigned)f2e(x1[1]) << 16);
+  u.w = (unsigned)f2e(x1[2]) | ((unsigned)f2e(x1[3]) << 16);
+  return u;
+}
+
 __global__ __launch_bounds__(256) void merge_fwd_kernel(const float* __restrict__ part_o,
                                                         const float* __restrict__ part_lse,
                                                         const int4* __restrict__ merges, const int* __restrict__ info,
@@ -144,46 +184,48 @@ __global__ __launch_bounds__(256) void merge_fwd_kernel(const float* __restrict_
   if ((int)blockIdx.x >= info[1]) return;
   const int4 mg = merges[blockIdx.x];
   const int bh = mg.x / NB, qb = mg.x - bh * NB, slot0 = mg.y, c = mg.z;
-  const int row = threadIdx.x >> 2, c0 = (threadIdx.x & 3) * 32;
+  const int row = blockIdx.y * 16 + (threadIdx.x >> 4), c0 = (threadIdx.x & 15) * 8;
   if (c0 >= ld) return;  // (rows of ld columns)
   const size_t tok = (size_t)bh * L + (size_t)qb * BK + row;
-  float acc[32];
-#pragma unroll
-  for (int e = 0; e < 32; ++e) acc[e] = 0.0f;
+  f32x4 acc[2] = {f32x4{}, f32x4{}};
   float out_lse = -INFINITY;
   if (row < blk_cnt[qb] || !mask_rows) {
+    const float* pl = part_lse + (size_t)slot0 * BK + row;
     float mx = -INFINITY;
-    for (int j = 0; j < c; ++j) mx = fmaxf(mx, part_lse[(size_t)(slot0 + j) * BK + row]);
+#pragma unroll 8
+    for (int j = 0; j < c; ++j) mx = fmaxf(mx, pl[(size_t)j * BK]);
     if (mx != -INFINITY) {
       float sum = 0.0f;
-      for (int j = 0; j < c; ++j) {
-        const float w = exp2f(part_lse[(size_t)(slot0 + j) * BK + row] - mx);
-        const f32x4* src = reinterpret_cast<const f32x4*>(part_o + ((size_t)(slot0 + j) * BK + row) * ld + c0);
-        sum += w;
+      for (int j0 = 0; j0 < c; j0 += MERGE_AHEAD) {
+        f32x4 x[MERGE_AHEAD][2];
+        float w[MERGE_AHEAD];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const f32x4 x = src[q];
+        for (int k = 0; k < MERGE_AHEAD; ++k) {
+          const int j = min(j0 + k, c - 1);
+          const f32x4* src = reinterpret_cast<const f32x4*>(part_o + ((size_t)(slot0 + j) * BK + row) * ld + c0);
+          x[k][0] = src[0];
+          x[k][1] = src[1];
+          w[k] = pl[(size_t)j * BK];
+        }
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[4 * q + e] += w * x[e];
+        for (int k = 0; k < MERGE_AHEAD; ++k) asm volatile("" : "+v"(x[k][0]), "+v"(x[k][1]), "+v"(w[k]));  // (not sunk)
+#pragma unroll
+        for (int k = 0; k < MERGE_AHEAD; ++k) {
+          if (j0 + k >= c) break;
+          const float wk = exp2f(w[k] - mx);
+          sum += wk;
+          acc[0] += wk * x[k][0];
+          acc[1] += wk * x[k][1];
         }
       }
       const float inv = 1.0f / sum;
-#pragma unroll
-      for (int e = 0; e < 32; ++e) acc[e] *= inv;
+      acc[0] *= inv;
+      acc[1] *= inv;
       out_lse = (mx + log2f(sum)) * 0.6931471805599453f;
     }
   }
-  uint4* dst = reinterpret_cast<uint4*>(o + tok * ld + c0);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    uint4 u;
-    u.x = (unsigned)f2e(acc[8 * q + 0]) | ((unsigned)f2e(acc[8 * q + 1]) << 16);
-    u.y = (unsigned)f2e(acc[8 * q + 2]) | ((unsigned)f2e(acc[8 * q + 3]) << 16);
-    u.z = (unsigned)f2e(acc[8 * q + 4]) | ((unsigned)f2e(acc[8 * q + 5]) << 16);
-    u.w = (unsigned)f2e(acc[8 * q + 6]) | ((unsigned)f2e(acc[8 * q + 7]) << 16);
-    dst[q] = u;
-  }
-  if ((threadIdx.x & 3) == 0) lse[tok] = out_lse;
+  *reinterpret_cast<uint4*>(o + tok * ld + c0) = pack8e(acc[0], acc[1]);
+  if (c0 == 0) lse[tok] = out_lse;
 }
 
 __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict__ part, const int4* __restrict__ merges,
@@ -194,49 +236,43 @@ __global__ __launch_bounds__(256) void merge_sum_kernel(const float* __restrict_
   if ((int)blockIdx.x >= info[1]) return;
   const int4 mg = merges[blockIdx.x];
   const int bh = mg.x / NB, blk = mg.x - bh * NB, slot0 = mg.y, c = mg.z;
-  const int row = threadIdx.x >> 2, c0 = (threadIdx.x & 3) * 32;
+  const int row = blockIdx.y * 16 + (threadIdx.x >> 4), c0 = (threadIdx.x & 15) * 8;
   if (c0 >= ld) return;  // (rows of ld columns)
   const size_t tok = (size_t)bh * L + (size_t)blk * BK + row;
   const int cnt = blk_cnt[blk];
-  float acc[32];
-#pragma unroll
-  for (int e = 0; e < 32; ++e) acc[e] = 0.0f;
+  f32x4 acc[2] = {f32x4{}, f32x4{}};
   if (row < cnt) {
-    for (int j = 0; j < c; ++j) {
-      const f32x4* src = reinterpret_cast<const f32x4*>(part + ((size_t)(slot0 + j) * BK + row) * ld + c0);
+    for (int j0 = 0; j0 < c; j0 += MERGE_AHEAD) {
+      f32x4 x[MERGE_AHEAD][2];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const f32x4 x = src[q];
+      for (int k = 0; k < MERGE_AHEAD; ++k) {
+        const int j = min(j0 + k, c - 1);
+        const f32x4* src = reinterpret_cast<const f32x4*>(part + ((size_t)(slot0 + j) * BK + row) * ld + c0);
+        x[k][0] = src[0];
+        x[k][1] = src[1];
+      }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * q + e] += x[e];
+      for (int k = 0; k < MERGE_AHEAD; ++k) asm volatile("" : "+v"(x[k][0]), "+v"(x[k][1]));  // (not sunk to their uses)
+#pragma unroll
+      for (int k = 0; k < MERGE_AHEAD; ++k) {
+        if (j0 + k >= c) break;
+        acc[0] += x[k][0];
+        acc[1] += x[k][1];
       }
     }
     if (add != nullptr) {
       const float inv = 1.0f / (float)cnt;
       const f32x4* ad = reinterpret_cast<const f32x4*>(add + ((size_t)bh * add_nb + blk) * ld + c0);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const f32x4 x = ad[q];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * q + e] += x[e] * inv;
-      }
+      acc[0] += ad[0] * inv;
+      acc[1] += ad[1] * inv;
     }
   }
   if (out_f32 != nullptr) {
     f32x4* dst = reinterpret_cast<f32x4*>(out_f32 + tok * ld + c0);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) dst[q] = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    dst[0] = acc[0];
+    dst[1] = acc[1];
   } else {
-    uint4* dst = reinterpret_cast<uint4*>(out + tok * ld + c0);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint4 u;
-      u.x = (unsigned)f2e(acc[8 * q + 0]) | ((unsigned)f2e(acc[8 * q + 1]) << 16);
-      u.y = (unsigned)f2e(acc[8 * q + 2]) | ((unsigned)f2e(acc[8 * q + 3]) << 16);
-      u.z = (unsigned)f2e(acc[8 * q + 4]) | ((unsigned)f2e(acc[8 * q + 5]) << 16);
-      u.w = (unsigned)f2e(acc[8 * q + 6]) | ((unsigned)f2e(acc[8 * q + 7]) << 16);
-      dst[q] = u;
-    }
+    *reinterpret_cast<uint4*>(out + tok * ld + c0) = pack8e(acc[0], acc[1]);
   }
 }
 
@@ -282,7 +318,7 @@ extern "C" int ES_VSA_API(vsa_split_merge_fwd)(const float* part_o, const float*
   ES_REQUIRE(BH >= 1 && L > 0 && L % BK == 0, ES_ERR_INVALID, "o must be [B,H,L,D]");
   if (max_merges <= 0) return ES_OK;
   ES_REQUIRE(part_o && part_lse && merges && info && blk_cnt && o && lse, ES_ERR_INVALID, "VSA2: null tensor pointer");
-  hipLaunchKernelGGL(merge_fwd_kernel, dim3(max_merges), dim3(256), 0, stream, part_o, part_lse, (const int4*)merges,
+  hipLaunchKernelGGL(merge_fwd_kernel, dim3(max_merges, 4), dim3(256), 0, stream, part_o, part_lse, (const int4*)merges,
                      info, blk_cnt, (e16_t*)o, lse, L, L / BK, h.ld, mask_rows);
   return check_launch("vsa_split_merge_fwd");
 }
@@ -295,7 +331,7 @@ extern "C" int ES_VSA_API(vsa_split_merge_sum)(const float* part, const int* mer
   ES_REQUIRE(BH >= 1 && L > 0 && L % BK == 0, ES_ERR_INVALID, "out must be [B,H,L,D]");
   if (max_merges <= 0) return ES_OK;
   ES_REQUIRE(part && merges && info && blk_cnt && (out || out_f32), ES_ERR_INVALID, "VSA2: null tensor pointer");
-  hipLaunchKernelGGL(merge_sum_kernel, dim3(max_merges), dim3(256), 0, stream, part, (const int4*)merges, info, add,
+  hipLaunchKernelGGL(merge_sum_kernel, dim3(max_merges, 4), dim3(256), 0, stream, part, (const int4*)merges, info, add,
                      add_nb, blk_cnt, (e16_t*)out, out_f32, L, L / BK, h.ld);
   return check_launch("vsa_split_merge_sum");
 }
