@@ -352,6 +352,7 @@ class _VsaFunction(torch.autograd.Function):
         ctx.gate_act, ctx.has_gate, ctx.split = gate_act, gate is not None, split
         ctx.bwd_variant, ctx.bwd_source = bwd
         ctx.mark_non_differentiable(*sel)
+        ctx.set_materialize_grads(False)      # (no zero-filled gradients for the selection's lists)
         return (o, *sel)
 
     @staticmethod
@@ -363,7 +364,7 @@ class _VsaFunction(torch.autograd.Function):
             raise RuntimeError("VSA backward frees its intermediates after the first backward; "
                                "re-run the forward instead of backward(retain_graph=True) twice")
         ctx.held = None
-        dout = dout.contiguous()
+        dout = torch.zeros_like(held["of"]) if dout is None else dout.contiguous()
         _, delta_f, dout_c, delta_c, dgate = C.fuse_bwd(dout, held["of"], held["oc"], gate if ctx.has_gate else None,
                                                         blk_cnt, ctx.gate_act, False)
         held["of"] = None
@@ -428,13 +429,14 @@ class _FineFunction(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, blk_cnt, of, lse, *sel)
         ctx.split = split
         ctx.bwd_variant, ctx.bwd_source = bwd
+        ctx.set_materialize_grads(False)      # (lse has no gradient: no zero-filled dlse)
         return of, lse
 
     @staticmethod
     def backward(ctx, dout, dlse):
         C = ext()
         q, k, v, blk_cnt, of, lse, *sel = ctx.saved_tensors
-        dout = dout.contiguous()
+        dout = torch.zeros_like(of) if dout is None else dout.contiguous()
         delta = C.row_dot(dout, of, blk_cnt)
         dq, dk, dv = _fine_backward(C, q, k, v, dout, lse, delta, tuple(sel), blk_cnt, None, None, None, ctx.split)
         return dq, dk, dv, None, None, None, None

@@ -224,13 +224,14 @@ class _RepFineFunction(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, blk_cnt, o, lse)
         ctx.tab, ctx.sel, ctx.mid_reps, ctx.phases = tab, sel, spec.mid_reps, phases
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)      # (no zero-filled dlse)
         return o, lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
         C = ext()
         q, k, v, blk_cnt, o, lse = ctx.saved_tensors
-        dout = dout.contiguous()
+        dout = torch.zeros_like(o) if dout is None else dout.contiguous()
         delta = C.row_dot(dout, o, blk_cnt)
         dq, dk, dv = _fine_backward(C, q, k, v, ctx.tab, dout, lse, delta, blk_cnt, ctx.sel, ctx.mid_reps, ctx.phases)
         ctx.tab = ctx.sel = None
@@ -275,6 +276,7 @@ class _RepAttentionFunction(torch.autograd.Function):
         ctx.has_gate, ctx.gate_act, ctx.mid_reps, ctx.phases = gate is not None, gate_act, tiers.mid_reps, phases
         outs = (sel.q2k_ptr, sel.q2k_idx, sel.k2q_ptr, sel.k2q_idx, sel.bits_a, sel.bits_ab)
         ctx.mark_non_differentiable(*outs)
+        ctx.set_materialize_grads(False)      # (no zero-filled gradients for the selection)
         return (o,) + outs
 
     @staticmethod
@@ -285,7 +287,7 @@ class _RepAttentionFunction(torch.autograd.Function):
         if h is None:
             raise RuntimeError("rep_attention backward frees its intermediates after the first backward")
         ctx.held = None
-        dout = dout.contiguous()
+        dout = torch.zeros_like(h["of"]) if dout is None else dout.contiguous()
         _, delta_f, dout_c, delta_c, dgate = C.fuse_bwd(dout, h["of"], h["oc"], gate if ctx.has_gate else None,
                                                         blk_cnt, ctx.gate_act, False)
         c_cnt, c_ptr, c_idx = h["coarse"]
