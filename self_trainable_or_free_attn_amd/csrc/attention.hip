@@ -924,8 +924,8 @@ extern "C" size_t es_dense_attention_workspace(int Lq, int Lk, int H) {
   return S <= 1 ? 0 : (size_t)S * ((Lq + BM - 1) / BM) * H * PART * sizeof(float);
 }
 
-extern "C" int es_dense_attention_ws(const void* q, const void* k, const void* v, void* out, float* lse2, void* workspace,
-                                     size_t workspace_bytes, int Lq, int Lk, int H, int D, hipStream_t stream) {
+extern "C" int es_dense_attention_ws(const void* q, const void* k, const void* v, void* out, float* lse2,
+                                     void* workspace, size_t workspace_bytes, int Lq, int Lk, int H, int D, hipStream_t stream) {
   const size_t need = es_dense_attention_workspace(Lq, Lk, H);
   if (need == 0) return es_dense_attention_kv(q, k, v, out, lse2, Lq, Lk, H, D, stream);
   int st = check_common(q, k, v, Lq, H, D);

@@ -58,8 +58,8 @@ constexpr int POOL_BLOCKS = 4;  // 64-token blocks per workgroup
 // grid (cdiv(ceil64(NB), 4), BH), 192 threads: 48 per block = 3 tensors x 16 chunks of 8 columns. Each column sums its
 // group's rows in order, then the group sums in order, so the float result is that of a sequential loop. The rows are
 // read sixteen at a time, all in flight before the first is added (one row after the other, the sums waited for each
-// load in turn: 24 us for three 4096-token, 2-head tensors against 8 now, 36 against 24 for 240 blocks and 12 heads). The pooled tensors' padding rows are written as zeros here, so callers need not clear
-// them first.
+// load in turn: 24 us for three 4096-token, 2-head tensors against 8 now, 36 against 24 for 240 blocks and 12 heads). The
+// pooled tensors' padding rows are written as zeros here, so callers need not clear them first.
 template <int R>
 __global__ __launch_bounds__(192) void pool_kernel(PoolArgs a) {
   constexpr int G = BK / R, BATCH = 16;

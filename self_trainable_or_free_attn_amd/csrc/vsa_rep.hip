@@ -16,8 +16,8 @@
 //   rep_bwd_q_kernel    dQ over the same stream (S^T, dP^T, dQ^T += K^T dS^T), deterministic.
 //   rep_bwd_tab_kernel  dK / dV of the representative tables, KV-owner: a workgroup owns 64 table rows and walks
 //                       every query block that has one of its pairs in the tier (pairs outside get P = 0), so the
-//                       shared rows need no atomics; a dV pass and a dK pass (two waves per SIMD, 119.8 -> 118.0 ms
-//                       per C4 step at B = 1). Tier-A token dK / dV come from the fine KV-owner kernel.
+//                       shared rows need no atomics; a dV and a dK wave group share each staged Q / dO, both tiers in
+//                       one launch. Tier-A token dK / dV come from the fine KV-owner kernel.
 //   rep_unpool_kernel   dX = acc + dk_mid[group] / c_group + dk_tail[blk] / c_blk on valid rows (the adjoint of the
 //                       means), tier_b_lists_kernel (A|B lists minus tier A), row_dot_kernel (delta).
 #include "../../include/vsa_hip.h"
@@ -408,7 +408,8 @@ __device__ __forceinline__ unsigned long long tier_mask(const TabArgs& a, bool t
 // Both tiers' row groups run in one launch, all claimed at run time: a tier-C group walks every query block and a head
 // has few of them (15 at 957 blocks), so on its own that tier left most CUs idle, and with the groups bound to the XCDs
 // of their heads a head count that eight does not divide left XCDs idle. 957 blocks, 6 heads, both tiers: 1475 + 1265
-// us in two launches of bound groups, 2310 in one. What bounds it then is the delivery of Q / dO to every row group.
+// us in two launches of bound groups, 2310 in one; 1857 blocks, 48 heads, which eight divides: 39.5 and 39.7 ms. What
+// bounds it then is the delivery of Q / dO to every row group.
 // One 512-thread workgroup per (64 table rows, head) in head-major balanced order (queues.h), one per CU, in the
 // fine KV-owner layout (2 key halves x 2 query halves) twice: a dV group of four waves (S, P, dV) and a dK group
 // (dP with the table's V rows in registers, dS from the dV group's P handed over through LDS, dK), one accumulator
