@@ -77,12 +77,15 @@ def _dim(D):
 
 def _rows(x, D):
     """x as rows stored D columns wide (None stays None). At D = 64 a tensor in any layout is taken: one that is not
-    contiguous or not 16-byte aligned is copied first. A width other than D is narrowed, or zero-padded at D = 128."""
+    contiguous or not 16-byte aligned is copied first. A narrower tensor is zero-padded to D columns (the kernels read
+    D of every row), a wider one narrowed."""
     if x is None:
         return None
     if D == HD:
         return _wide(x)
-    if x.shape[-1] != D:
+    if x.shape[-1] < D:
+        return F.pad(x, (0, D - x.shape[-1])).contiguous()
+    if x.shape[-1] > D:
         x = x[..., :D]
     plain = type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling()
     at = x.data_ptr() if plain else x.storage_offset() * x.element_size()

@@ -1,0 +1,43 @@
+"""How the VSA operators hand D = 64 rows to the entry points, which read D columns of every row whatever the tensor's
+width: fake GPU tensors, nothing is launched."""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from self_trainable_or_free_attn_amd import _lib
+from self_trainable_or_free_attn_amd.vsa import _C
+
+BF = torch.bfloat16
+
+
+def test_rows_pad_and_narrow():
+    x = torch.arange(1, 97.0).view(3, 32)
+    assert torch.equal(_C._rows(x, 64), torch.cat([x, torch.zeros(3, 32)], 1))
+    y = torch.arange(1, 301.0).view(3, 100)
+    assert torch.equal(_C._rows(y, 64), y[:, :64]) and _C._rows(y, 64).is_contiguous()
+    assert torch.equal(_C._rows(x, 128), torch.cat([x, torch.zeros(3, 96)], 1))
+
+
+@pytest.mark.parametrize("width", [16, 32, 63, 64, 100, 128])
+def test_secondary_tensors_reach_the_kernels_with_full_rows(monkeypatch, width):
+    """A coarse output, a gradient to add and a partial of another width than the tokens' 64."""
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: calls.append((name, args)))
+    with FakeTensorMode():
+        tok = lambda w=64: torch.empty(1, 2, 320, w, device="cuda", dtype=BF)
+        f32 = lambda *s: torch.empty(*s, device="cuda")
+        cnt = torch.empty(5, device="cuda", dtype=torch.int32)
+        oc, add = torch.empty(1, 2, 64, width, device="cuda", dtype=BF), f32(1, 2, 64, width)
+        _C.fuse_fwd(tok(), oc, None, cnt, 0)
+        _C.fuse_bwd(tok(), tok(width), oc, None, cnt, 0)
+        _C.finalize(f32(1, 2, 320, width), add, cnt, tok())
+        _C.row_dot(tok(), tok(width), cnt)
+        i32 = lambda *s: torch.empty(*s, device="cuda", dtype=torch.int32)
+        _C.split_merge_sum(f32(4, 64, width), i32(2, 4), i32(8), add, cnt, tok())
+        _C.router_lse(torch.empty(1, 2, 64, 64, device="cuda", dtype=BF), oc, cnt, 16)
+        _C.attn_bwd_q(tok(), tok(), tok(), tok(width), f32(1, 2, 320), f32(1, 2, 320), i32(1, 2, 6), i32(20), cnt, add)
+    assert len(calls) == 7
+    for name, args in calls:
+        for a in args:                     # (the float tensors that are not per-token statistics, [1, 2, 320])
+            if isinstance(a, torch.Tensor) and a.is_floating_point() and a.shape[-1] != 320:
+                assert a.shape[-1] == 64 and a.is_contiguous(), (name, tuple(a.shape))
