@@ -75,6 +75,17 @@ def _dim(D):
     return D if D == HD else D | VSA_PACKED_ROWS
 
 
+def _aligned(x):
+    """x has an address and it is a multiple of 16. A tensor that is being traced or transformed (torch.compile, fake
+    tensors, torch.func wrappers) has none to look at: the graph copies its rows, wherever they will lie."""
+    if torch.compiler.is_compiling() or type(x) not in (torch.Tensor, torch.nn.Parameter):
+        return False
+    try:
+        return x.data_ptr() % 16 == 0
+    except RuntimeError:                  # a torch.func wrapper (their Python type is torch.Tensor)
+        return False
+
+
 def _rows(x, D):
     """x as rows stored D columns wide (None stays None). At D = 64 a tensor in any layout is taken: one that is not
     contiguous or not 16-byte aligned is copied first. A narrower tensor is zero-padded to D columns (the kernels read
@@ -87,9 +98,7 @@ def _rows(x, D):
         return F.pad(x, (0, D - x.shape[-1])).contiguous()
     if x.shape[-1] > D:
         x = x[..., :D]
-    plain = type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling()
-    at = x.data_ptr() if plain else x.storage_offset() * x.element_size()
-    return x if x.is_contiguous() and at % 16 == 0 else x.clone(memory_format=torch.contiguous_format)
+    return x if x.is_contiguous() and _aligned(x) else x.clone(memory_format=torch.contiguous_format)
 
 
 class _InRows:

@@ -41,3 +41,57 @@ def test_secondary_tensors_reach_the_kernels_with_full_rows(monkeypatch, width):
         for a in args:                     # (the float tensors that are not per-token statistics, [1, 2, 320])
             if isinstance(a, torch.Tensor) and a.is_floating_point() and a.shape[-1] != 320:
                 assert a.shape[-1] == 64 and a.is_contiguous(), (name, tuple(a.shape))
+
+
+def _fine(q, k, v, cnt, a, b, c, d):
+    from self_trainable_or_free_attn_amd.vsa import Selection, fine_block_sparse_attention
+    return fine_block_sparse_attention(q, k, v, cnt, Selection(a, b, c, d), backend="generic")
+
+
+def _fine_args(D):
+    i32 = lambda *s: torch.empty(*s, device="cuda", dtype=torch.int32)
+    qkv = [torch.empty(1, 2, 320, D, device="cuda", dtype=BF) for _ in range(3)]
+    return (*qkv, i32(5), i32(1, 2, 6), i32(20), i32(1, 2, 6), i32(20))
+
+
+TRACED = {
+    "fine_block_sparse_attention": (_fine, _fine_args),
+    "attn_fwd": (lambda q, k, v, cnt, a, b, c, d: _C.attn_fwd(q, k, v, a, b, cnt), _fine_args),
+    "attn_bwd_q_acc": (lambda q, k, v, cnt, a, b, c, d: _C.attn_bwd_q_acc(
+        q, k, v, q, q[..., 0].float(), q[..., 0].float(), a, b, cnt, q.float()), _fine_args),
+    "pool_fwd": (lambda q, k, v, cnt, a, b, c, d: _C.pool_fwd(q, k, v, cnt, 16), _fine_args),
+    "row_dot": (lambda q, k, v, cnt, a, b, c, d: _C.row_dot(q, k, cnt), _fine_args),
+}
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("name", sorted(TRACED))
+def test_operators_trace_into_one_graph(name, dynamic, D):
+    """Under torch.compile(fullgraph=True) a tensor has no address to look at."""
+    f, args = TRACED[name]
+    _lib.ops()
+    torch._dynamo.reset()
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        out = torch.compile(f, fullgraph=True, backend="eager", dynamic=dynamic)(*args(D))
+    first = out[0] if isinstance(out, (list, tuple)) else out
+    assert first.is_cuda and first.shape[:2] == (1, 2)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_operators_under_forward_mode(D):
+    """A torch.func wrapper is a torch.Tensor without storage; the operators have no derivative, and take it."""
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        q, k, v, cnt, *lists = _fine_args(D)
+        (o, lse), _ = torch.func.jvp(lambda x: _C.attn_fwd(x, k, v, *lists[:2], cnt), (q,), (torch.ones_like(q),))
+        assert o.shape == q.shape and lse.shape == q.shape[:3]
+        dot, _ = torch.func.jvp(lambda x: _C.row_dot(x, k, cnt), (q,), (torch.ones_like(q),))
+        assert dot.shape == q.shape[:3]
+
+
+def test_unaligned_rows_are_copied():
+    x = torch.zeros(3 * 64 + 1, dtype=BF)
+    aligned, shifted = x[:-1].view(3, 64), x[1:].view(3, 64)
+    assert _C._rows(aligned, 64) is aligned
+    copy = _C._rows(shifted, 64)
+    assert copy is not shifted and copy.data_ptr() % 16 == 0 and torch.equal(copy, shifted)
