@@ -10,7 +10,6 @@ stream (workspace sizes, limits, the error string) and tests that drive the C AB
 There is no fallback: if either library is missing or fails to load, every kernel call raises.
 """
 import ctypes
-import functools
 import numbers
 import os
 
@@ -156,6 +155,16 @@ def topk_workspace_bytes(bh_count, NB):
     return int(lib().vsa_topk_workspace(bh_count, NB))
 
 
-@functools.lru_cache(maxsize=1024)
 def dense_workspace_bytes(Lq, Lk, H):
-    return int(lib().es_dense_attention_workspace(Lq, Lk, H))
+    """es_dense_attention_workspace in Python arithmetic, which Dynamo can trace (also over symbolic sizes) and a ctypes
+    call cannot be. The rule and its reasons stand at dense_splits in csrc/attention.hip; es_dense_attention_ws refuses a
+    workspace smaller than its own rule asks for."""
+    if Lq <= 0 or Lk <= 0 or H <= 0:
+        return 0
+    items, nb = (Lq + 127) // 128 * H, (Lk + 63) // 64
+    if items > 256 or nb < 8:
+        return 0
+    ranges = min(512 // items, 16, nb // 4)
+    if ranges < 2 or (ranges == 2 and nb < 16):
+        return 0
+    return ranges * items * (128 * 128 + 2 * 128) * 4
