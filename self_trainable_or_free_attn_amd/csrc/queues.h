@@ -77,22 +77,18 @@ __device__ __forceinline__ bool balanced_item(int* queues, int fixed, int per_xc
 
 // Head-major variant for kernels whose workgroups each stream a whole head's rows (the three-tier table
 // gradients): queue x holds every row group of heads x, x + 8, ..., so that one XCD's L2 serves all workgroups of
-// a head. Same claiming as above; `groups` row groups per head.
-__device__ __forceinline__ bool balanced_head_item(int* queues, int fixed, int groups, int heads, int& hd, int& grp) {
-  const int w = blockIdx.x, per_queue = (heads + 7) / 8 * groups;
-  int x = w & 7, k = w >> 3;
-  if (k >= fixed) {
-    __shared__ int item_s;
-    if (threadIdx.x < 64) {
-      const int it = claim_item(queues, x, fixed, per_queue);
-      if (threadIdx.x == 0) item_s = it;
-    }
-    __syncthreads();
-    const int it = __builtin_amdgcn_readfirstlane(item_s);
-    if (it < 0) return false;
-    x = it / per_queue;
-    k = it - x * per_queue;
+// a head; `groups` row groups per head. Every item is claimed (a launch with claim_all).
+__device__ __forceinline__ bool balanced_head_item(int* queues, int groups, int heads, int& hd, int& grp) {
+  const int per_queue = (heads + 7) / 8 * groups;
+  __shared__ int item_s;
+  if (threadIdx.x < 64) {
+    const int it = claim_item(queues, blockIdx.x & 7, 0, per_queue);
+    if (threadIdx.x == 0) item_s = it;
   }
+  __syncthreads();
+  const int it = __builtin_amdgcn_readfirstlane(item_s);
+  if (it < 0) return false;
+  const int x = it / per_queue, k = it - x * per_queue;
   hd = x + 8 * (k / groups);
   grp = k % groups;
   return hd < heads;
@@ -159,16 +155,15 @@ struct Queues {
 
 // Sets up one balanced launch of eight queues of per_queue items each: takes a counter slot, orders the stream
 // after the slot's previous launch, clears the slot on `stream` and gives the grid size. false if the device's
-// counter ring is unavailable. A launch of at most `resident` items (the workgroups that the 256 CUs hold at once:
-// two each, or one of the kernels that fill a CU) has no tail to balance: every item is bound to its dispatch slot
-// and nothing is cleared, waited for or recorded. (The counters' kernel takes 1.4 us and its gap on the stream, and
-// the wait and record two more host calls. A forward + backward of 4096 tokens and two heads, with the launches saved
-// in its router and lists: 564 -> 368 us.)
-// claim_all: every item is claimed (few, long items that a fixed binding to XCDs would leave uneven).
-static bool balanced_launch_queues(int per_queue, hipStream_t stream, Queues& out, int resident = 512,
-                                   bool claim_all = false) {
+// counter ring is unavailable. A launch of at most RESIDENT items, padding included (the 256 CUs hold two of its
+// workgroups each), has no tail to balance: every item is bound to its dispatch slot and nothing is cleared, waited for
+// or recorded. (The counters' kernel takes 1.4 us and its gap on the stream, and the wait and record two more host
+// calls.) claim_all: every item is claimed and a slot taken at any size (few, long items that a fixed binding to XCDs
+// would leave uneven).
+constexpr int RESIDENT = 512;
+static bool balanced_launch_queues(int per_queue, hipStream_t stream, Queues& out, bool claim_all = false) {
   out.release();
-  if (!claim_all && 8LL * per_queue <= resident) {
+  if (!claim_all && 8LL * per_queue <= RESIDENT) {
     out.counters = nullptr;
     out.fixed = per_queue;
     out.grid = 8LL * per_queue;

@@ -383,7 +383,7 @@ struct TabArgs {
   const float *lse, *delta;
   const unsigned *bits_a, *bits_ab;
   int* queues;                  // the eight row-group queue counters of this launch (queues.h)
-  int L, NB, RM, W, BH, fixed;
+  int L, NB, RM, W, BH;
   int tail_groups, groups;      // 64-row groups of a head: tier C's first, then tier B's (0: a tier left out)
   float scale_log2, scale;
 };
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(512, 1) void rep_bwd_tab_kernel(TabArgs a) {
   __shared__ unsigned long long am_s[RING];
   __shared__ int wcnt_s[8];
   int grp, bh;
-  if (!balanced_head_item(a.queues, a.fixed, a.groups, a.BH, bh, grp)) return;
+  if (!balanced_head_item(a.queues, a.groups, a.BH, bh, grp)) return;
   const bool tier_b = grp >= a.tail_groups;
   if (tier_b) grp -= a.tail_groups;
   const Table t = tier_b ? a.mid : a.tail;
@@ -863,10 +863,9 @@ static int launch_tables(TabArgs& a, hipStream_t stream) {
   a.tail_groups = a.tail.rows_pad / BK;
   a.groups = a.tail_groups + a.mid.rows_pad / BK;
   Queues qs;
-  ES_REQUIRE(balanced_launch_queues((a.BH + 7) / 8 * a.groups, stream, qs, 0, true), ES_ERR_LAUNCH,
+  ES_REQUIRE(balanced_launch_queues((a.BH + 7) / 8 * a.groups, stream, qs, true), ES_ERR_LAUNCH,
              "VSA2-rep: row-group queues unavailable");
   a.queues = qs.counters;
-  a.fixed = qs.fixed;
   hipLaunchKernelGGL(rep_bwd_tab_kernel, dim3((unsigned)qs.grid), dim3(512), 0, stream, a);
   return check_launch("vsa_rep_bwd_tables");
 }

@@ -320,7 +320,7 @@ def _fine_backward(C, q, k, v, dout, lse, delta, sel, blk_cnt, add_q, add_k, add
     return dq, dk, dv
 
 
-def _coarse_lists(B, H, nb, nbc_pad, device):
+def _coarse_lists(B, H, nb, device):
     """Dense CSR over the 64-row tiles of the pooled sequence: (tile counts, ptr, idx)."""
     return ext().dense_lists(B, H, nb, device)
 
@@ -335,7 +335,7 @@ class _VsaFunction(torch.autograd.Function):
         B, H, L, D = q.shape
         nb = L // 64
         qr, kr, qc, kc, vc = C.pool_fwd(q, k, v, blk_cnt, R)
-        c_cnt, c_ptr, c_idx = _coarse_lists(B, H, nb, qc.shape[2], q.device)
+        c_cnt, c_ptr, c_idx = _coarse_lists(B, H, nb, q.device)
         oc, lse_c = C.attn_fwd(qc, kc, vc, c_ptr, c_idx, c_cnt)
         if given is not None:
             sel = (given.q2k_ptr, given.q2k_idx, given.k2q_ptr, given.k2q_idx)

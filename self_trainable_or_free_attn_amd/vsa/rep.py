@@ -264,7 +264,7 @@ class _RepAttentionFunction(torch.autograd.Function):
         B, H, L, D = q.shape
         nb = L // 64
         qr, kr, qc, kc, vc = C.pool_fwd(q, k, v, blk_cnt, R)
-        c_cnt, c_ptr, c_idx = _coarse_lists(B, H, nb, qc.shape[2], q.device)
+        c_cnt, c_ptr, c_idx = _coarse_lists(B, H, nb, q.device)
         oc, lse_c = C.attn_fwd(qc, kc, vc, c_ptr, c_idx, c_cnt)
         sel = given if given is not None else _select_tiers(C, qr, kr, blk_cnt, R, tiers, row_norm, max_score_bytes)
         del qr, kr
