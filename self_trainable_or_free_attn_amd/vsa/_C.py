@@ -661,17 +661,18 @@ def rep_attn_bwd_q(q, k, v, k_mid, v_mid, lc_mid, k_tail, v_tail, lc_tail, dout,
               dq, B * H, L, D, int(mid_reps), int(phases))
     acc.put()
     stats = (lse, delta, bits_a, bits_ab)
-    mids, tails = [_InPlace(dk_mid), _InPlace(dv_mid)], [_InPlace(dk_tail), _InPlace(dv_tail)]
-    if phases & 2 and phases & 4:
+    mids = [_InPlace(dk_mid), _InPlace(dv_mid)] if phases & 2 else []
+    tails = [_InPlace(dk_tail), _InPlace(dv_tail)] if phases & 4 else []
+    if mids and tails:
         _call("vsa_rep_bwd_both_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), k_tail, v_tail, lc_tail,
-              *stats, mids[0].w, mids[1].w, tails[0].w, tails[1].w, B * H, L, D, int(mid_reps))
-    elif phases & 2:
-        _call("vsa_rep_bwd_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), *stats, mids[0].w, mids[1].w,
+              *stats, *(t.w for t in mids + tails), B * H, L, D, int(mid_reps))
+    elif mids:
+        _call("vsa_rep_bwd_tables", q, dout, k_mid, v_mid, lc_mid, _lc_stride(lc_mid), *stats, *(t.w for t in mids),
               B * H, L, D, int(mid_reps), 2)
-    elif phases & 4:
-        _call("vsa_rep_bwd_tables", q, dout, k_tail, v_tail, lc_tail, 0, *stats, tails[0].w, tails[1].w, B * H, L, D,
+    elif tails:
+        _call("vsa_rep_bwd_tables", q, dout, k_tail, v_tail, lc_tail, 0, *stats, *(t.w for t in tails), B * H, L, D,
               int(mid_reps), 4)
-    for t in (mids if phases & 2 else []) + (tails if phases & 4 else []):
+    for t in mids + tails:
         t.put()
     return _narrow(dq, D)
 

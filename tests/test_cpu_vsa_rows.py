@@ -95,3 +95,24 @@ def test_unaligned_rows_are_copied():
     assert _C._rows(aligned, 64) is aligned
     copy = _C._rows(shifted, 64)
     assert copy is not shifted and copy.data_ptr() % 16 == 0 and torch.equal(copy, shifted)
+
+
+@pytest.mark.parametrize("phases", range(8))
+def test_table_gradients_pad_only_the_tables_in_use(monkeypatch, phases):
+    """At D = 64 a table's gradients are padded to 128 columns and written back: only those of the tiers that run."""
+    calls, wide = [], []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: calls.append(name))
+    pad = _C._wide
+    monkeypatch.setattr(_C, "_wide", lambda x: wide.append(x) or pad(x))
+    with FakeTensorMode():
+        bf = lambda n, w=64: torch.empty(1, 2, n, w, device="cuda", dtype=BF)
+        f32, i32 = (lambda *s, t=t: torch.empty(*s, device="cuda", dtype=t) for t in (torch.float32, torch.int32))
+        grads = [f32(1, 2, n, 64) for n in (64, 64, 64, 64)]
+        _C.rep_attn_bwd_q(bf(320), bf(320), bf(320), bf(64), bf(64), f32(20), bf(64), bf(64), f32(5), bf(320),
+                          f32(1, 2, 320), f32(1, 2, 320), i32(1, 2, 6), i32(20), i32(1, 2, 5, 1), i32(1, 2, 5, 1),
+                          i32(5), *grads, 4, phases)
+    used = (grads[:2] if phases & 2 else []) + (grads[2:] if phases & 4 else [])
+    seen = [x for x in wide if any(x is g for g in grads)]
+    assert len(seen) == len(used) and all(any(x is g for x in seen) for g in used)
+    want = {0: [], 2: ["vsa_rep_bwd_tables"], 4: ["vsa_rep_bwd_tables"], 6: ["vsa_rep_bwd_both_tables"]}[phases & 6]
+    assert calls[1:] == want
