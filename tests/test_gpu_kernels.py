@@ -77,9 +77,9 @@ def test_torch_operators_refuse_views_wrong_dtypes_and_wrapping_ints(data):
 
 
 def test_balanced_launch_replays_in_a_graph(data):
-    """A balanced launch (dense attention) captured in a HIP graph takes its counter slot from the captured ring:
-    three replays, with uncaptured launches of the same kernel and host synchronisations between them, each write
-    the eager bytes."""
+    """A small dense attention launch (80 items with padding: all bound to their dispatch slots, no queue counters)
+    captured in a HIP graph: three replays, with uncaptured launches of the same kernel and host synchronisations
+    between them, each write the eager bytes. Launches that take counters: test_gpu_balanced_rings.py."""
     qd, kd, vd = data["qd"], data["kd"], data["vd"]
     ops = torch.ops.echosparse_gfx950
     out_e = torch.empty_like(qd)
@@ -482,9 +482,9 @@ def test_sparse_attention_stream_edges(data, plan, reps, dev):
 
 
 def test_sparse_attention_balanced_launches_concurrent_and_repeated(data, plan, reps, dev):
-    """The sparse step hands the last tiles of each XCD queue out at run time through a 64-slot ring of counters:
-    launches on three streams at once and 70 launches in a row (the ring wraps) give bytes-identical outputs,
-    which also pins that every tile runs exactly once whichever workgroup takes it."""
+    """Small sparse launches (80 items with padding: all bound to their dispatch slots, no queue counters) on three
+    streams at once and 70 in a row give bytes-identical outputs, which also pins that every tile runs exactly once.
+    Launches that take counters: test_gpu_balanced_rings.py."""
     p = plan
     R, km, vm = reps
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)
@@ -520,10 +520,9 @@ def test_sparse_attention_balanced_launches_concurrent_and_repeated(data, plan, 
 
 
 def test_balanced_ring_waits_for_a_live_slot(data, plan, reps, dev):
-    """A long balanced launch (dense attention, L = 32768, H = 8) on one stream while 70 short sparse launches run
-    on another: the short ones wrap the 64-slot counter ring and reach the slot the long launch still uses; the
-    launch that takes it must wait for the long one instead of clearing its counters, so every output is
-    bytes-identical to the same launches run one after another."""
+    """A long balanced launch (dense attention, L = 32768, H = 8), which holds a counter slot, on one stream while 70
+    short sparse launches, which take none, run on another: every output is bytes-identical to the same launches run
+    one after another. Short launches that wrap the ring onto a live slot: test_gpu_balanced_rings.py."""
     p = plan
     R, km, vm = reps
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(dev)

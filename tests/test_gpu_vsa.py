@@ -460,9 +460,9 @@ def test_vsa_attention_forward_backward(qkv):
 
 
 def test_balanced_launches_concurrent_and_repeated(qkv):
-    """The fine forward, KV-owner backward and dQ kernels hand the last query / key blocks of each XCD queue out at
-    run time through a 64-slot counter ring: calls on two streams at once and 40 calls in a row (wrapping the ring)
-    give bytes-identical outputs."""
+    """Small launches of the fine forward, KV-owner backward and dQ kernels (32 items with padding: all bound to their
+    dispatch slots, no queue counters) on two streams at once and 40 in a row give bytes-identical outputs. Launches
+    that take counters: test_gpu_balanced_rings.py."""
     log("balanced launches")
     q, k, v = qkv["gpu"]
     m = random_mask(5)
