@@ -1,6 +1,6 @@
-"""Dense attention over key ranges side by side (few query tiles and heads) against float64, at the edges of its rule:
-the fewest key blocks, ranges of unequal length, a last block of one key, ragged query tiles, and the item counts around
-256 where it stops splitting. Outputs are bf16 (half a step, 2^-8 of the value, and the probabilities' rounding to
+"""Dense attention over key ranges side by side (few query tiles and heads) against float64, at the edges of its rule,
+each size with the number of ranges it takes: the fewest key blocks that split (12 in three ranges, 16 in two), ranges
+of unequal length, a last block of one key, ragged query tiles, and the item counts around 256 where it stops splitting. Outputs are bf16 (half a step, 2^-8 of the value, and the probabilities' rounding to
 bf16, which averages over the keys): 2e-2 and relative 1e-2 as everywhere."""
 import math
 
@@ -12,13 +12,18 @@ from helpers import check_close, f32
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("Lq,Lk,H", [(1, 449, 1), (128, 512, 1), (129, 513, 2), (300, 1537, 3), (1537, 1537, 12),
-                                     (256, 33000, 24), (77, 40001, 1), (1280, 700, 24), (2600, 2600, 12),
-                                     (2816, 575, 12), (4000, 4001, 8), (4100, 1000, 8)])
-def test_split_dense_matches_float64(dev, Lq, Lk, H):
+@pytest.mark.parametrize("Lq,Lk,H,ranges", [(1, 449, 1, 1), (128, 512, 1, 1), (129, 513, 2, 1), (100, 705, 2, 3),
+                                            (128, 768, 1, 3), (129, 769, 1, 3), (60, 1000, 3, 4), (1400, 960, 20, 1),
+                                            (1400, 961, 20, 2), (300, 1537, 3, 6), (1537, 1537, 12, 3),
+                                            (256, 33000, 24, 10), (77, 40001, 1, 16), (1280, 700, 24, 1),
+                                            (2600, 2600, 12, 2), (2816, 575, 12, 1), (4000, 4001, 8, 2),
+                                            (4100, 1000, 8, 1)])
+def test_split_dense_matches_float64(dev, Lq, Lk, H, ranges):
     from self_trainable_or_free_attn_amd import _lib
     from self_trainable_or_free_attn_amd.kernels import gfx950 as K
-    print("dense", Lq, Lk, H, "workspace", _lib.dense_workspace_bytes(Lq, Lk, H), flush=True)
+    print("dense", Lq, Lk, H, "ranges", ranges, flush=True)
+    partial = (128 * 128 + 2 * 128) * 4   # a range's float32 O, maximum and row sum of one 128-row query tile
+    assert _lib.dense_workspace_bytes(Lq, Lk, H) == (ranges > 1) * ranges * -(-Lq // 128) * H * partial
     g = torch.Generator(device=dev).manual_seed(Lq + Lk)
     q = 2.0 * torch.randn(Lq, H, 128, device=dev, generator=g)
     k, v = (torch.randn(Lk, H, 128, device=dev, generator=g) for _ in range(2))
@@ -64,3 +69,16 @@ def test_split_replays_in_a_graph(dev):
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(lse, wlse)
         K.dense_attention_kv(q, k, v)
+
+
+def test_split_and_unsplit_calls_compile(dev):
+    """Traced into one graph, with fake tensors through the Meta kernels: the eager bytes."""
+    from self_trainable_or_free_attn_amd.attention import dense_attention
+    for Lq, Lk in ((300, 3000), (1537, 1537), (5000, 200)):
+        print("compiled dense", Lq, Lk, flush=True)
+        qkv = [torch.randn(1, n, 3, 128, device=dev).bfloat16() for n in (Lq, Lk, Lk)]
+        want = dense_attention(*qkv, return_lse=True)
+        torch._dynamo.reset()
+        f = torch.compile(lambda q, k, v: dense_attention(q, k, v, return_lse=True), backend="aot_eager", fullgraph=True)
+        got = f(*qkv)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
