@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("NB,heads,K", [(1, 2, 1), (63, 2, 5), (64, 2, 64), (65, 2, 16), (128, 3, 0), (129, 2, 40),
                                         (256, 2, 17), (257, 2, 100), (512, 1, 60), (513, 1, 60), (1024, 1, 200),
                                         (1025, 1, 1), (2048, 1, 333),
-                                        (33, 1025, 7), (130, 411, 20), (200, 300, 50), (300, 205, 31)])
+                                        (33, 1025, 7), (130, 411, 20), (200, 300, 50), (300, 205, 31), (600, 108, 40),
+                                        (1025, 63, 9), (2048, 32, 17)])
 @pytest.mark.parametrize("given", [False, True])
 def test_row_selection_widths(dev, NB, heads, K, given):
     from self_trainable_or_free_attn_amd.vsa import _C
