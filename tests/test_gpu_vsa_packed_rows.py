@@ -143,3 +143,22 @@ def test_unaligned_and_strided_d64_arguments(case):
     acc = torch.zeros(1, 3, c["L"], 128, device="cuda")[..., :64]
     with pytest.raises(RuntimeError):     # (an accumulator must be contiguous, as before)
         _C.attn_bwd_q_acc(q, k, v, x["do"], lse, delta, sel.q2k_ptr, sel.q2k_idx, cnt, acc)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_compiled_fine_attention_trains_as_eager(case, D):
+    from self_trainable_or_free_attn_amd.vsa import Selection, fine_block_sparse_attention
+    c, sel = case, case["sel"]
+    x = {n: F.pad(t, (0, D - 64)) for n, t in c["x"].items()}
+    qkv = [x[n].clone().requires_grad_(True) for n in "qkv"]
+    lists = (sel.q2k_ptr, sel.q2k_idx, sel.k2q_ptr, sel.k2q_idx)
+
+    def f(q, k, v, cnt, *lists):
+        return fine_block_sparse_attention(q, k, v, cnt, Selection(*lists))
+
+    want = f(*qkv, c["cnt"], *lists)
+    grads = torch.autograd.grad(want[0], qkv, x["do"])
+    torch._dynamo.reset()
+    got = torch.compile(f, backend="aot_eager", fullgraph=True)(*qkv, c["cnt"], *lists)
+    for a, b in zip((*got, *torch.autograd.grad(got[0], qkv, x["do"])), (*want, *grads)):
+        assert torch.equal(a, b)
