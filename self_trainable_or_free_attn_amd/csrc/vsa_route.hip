@@ -325,8 +325,10 @@ __device__ __forceinline__ long long ListBase::of(int bhl, int NB) const {
 
 // The whole inversion of one (b, h) with NB <= INV_NB in one workgroup: the bits in LDS, thread (row segment, column)
 // counts its column's bits over its rows, one scan over the columns, then every thread emits its rows in order. (The
-// three launches of the general form are bound by their latency here: 64 blocks, two heads, 4.4 us against 9.4 for
-// the count and the scan alone; 480 blocks, 24 heads, 32 us against 22, so the line lies between.)
+// three launches of the general form are bound by their latency here. A CSR transpose, one workgroup against three
+// launches, us: NB 64, 2 heads 9.3 and 14.1; NB 256: 1 head 13.3 and 14.0, 24 16.5 and 18.3, 256 54 and 67; NB 320: 1
+// head 18.5 and 18.3, 24 22.5 and 24.2; NB 384: 1 head 27 and 20, 24 31 and 25, 256 76 and 88. Past 256 columns a thread
+// has a column's rows in two or three segments only, so the line lies there at every head count.)
 constexpr int INV_NB = 256;
 __global__ __launch_bounds__(1024) void invert_small_kernel(const unsigned* __restrict__ selbits,
                                                             int* __restrict__ k2q_ptr, int* __restrict__ k2q_idx,
@@ -824,14 +826,26 @@ static void rows_launch_n(const RowsArgs& a, int bh_count, bool narrow, hipStrea
     hipLaunchKernelGGL((rows_select_kernel<FROM_SCORES, NCH, ROWS>), grid, dim3(256), lds, stream, a);
 }
 
-// The search keeps the smallest power of two of chunk registers that holds a row. Strips of 8 rows (a wave searches
-// two rows instead of eight, the S tile is computed four times) while the grid of 32-row strips is under eight
-// workgroups per CU: below that a strip's serial searches are what the launch waits for, above it the repeated
-// products are (routing NB = 480, 24 heads: 98 us in 360 strips of 32 rows, 52 in strips of 8; NB = 64, 2 heads: 51 -> 8 us).
+// Strips of 8 rows (a wave searches two rows instead of eight, the S tile is computed four times) instead of 32? While
+// there are few strips: what the launch waits for then is a strip's serial searches, with more the repeated products.
+// Past 1024 blocks the keys of 32 rows leave room for two workgroups per CU, and a grid that starts another round of 512
+// without filling it is faster in short strips; past 1280 they leave room for one, and every grid is. route_rows, us, 8
+// rows / 32 rows: NB 64: 4 strips of 32 rows 11.4 / 17.3, 256 19.5 / 17.7, 512 31.6 / 21.0; NB 240: 192 29 / 33, 256 34 /
+// 33, 384 43 / 38, 1024 81 / 62; NB 420: 294 64 / 66, 378 70 / 68; NB 600: 380 96 / 100, 456 118 / 101; NB 1000: 288 118 /
+// 126, 384 130 / 128, 512 158 / 129; NB 1025: 264 156 / 176, 396 193 / 182, 693 267 / 292, 1023 363 / 325; NB 1200: 380
+// 179 / 191, 1026 387 / 437, 6004 1841 / 1804; NB 1281: 287 180 / 303, 5986 1997 / 3174; NB 1857: 1003 518 / 684.
+static bool short_strips(int NB, int bh_count) {
+  const long long strips = (long long)((NB + ROWS - 1) / ROWS) * bh_count;
+  if (NB <= 512) return strips <= 300;
+  if (NB > 1280 || strips <= 384) return true;
+  return NB > 1024 && strips > 512 && 8 * strips < 7 * 512 * ((strips + 511) / 512);
+}
+
+// the search keeps the smallest power of two of chunk registers that holds a row
 template <bool FROM_SCORES>
 static void rows_launch(const RowsArgs& a, int bh_count, hipStream_t stream) {
   const int nchunk = (a.NB + 63) / 64;
-  const bool narrow = (long long)((a.NB + ROWS - 1) / ROWS) * bh_count < 2048;
+  const bool narrow = short_strips(a.NB, bh_count);
   if (nchunk <= 2) rows_launch_n<FROM_SCORES, 2>(a, bh_count, narrow, stream);
   else if (nchunk <= 4) rows_launch_n<FROM_SCORES, 4>(a, bh_count, narrow, stream);
   else if (nchunk <= 8) rows_launch_n<FROM_SCORES, 8>(a, bh_count, narrow, stream);

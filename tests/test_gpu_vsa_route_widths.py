@@ -1,6 +1,6 @@
 """The per-row block selection at the edges of its register layouts (2, 4, 8, 16, 32 chunks of 64 columns) and of its
-strip rule (8 rows per workgroup under 2048 strips of 32, else 32), bit for bit against the oracle. Pooled rows hold
-small integers, so every dot product is exact, scores tie often and the order of ties is tested too."""
+strip rule (8 or 32 rows per workgroup), bit for bit against the oracle. Pooled rows hold small integers, so every dot
+product is exact, scores tie often and the order of ties is tested too."""
 import numpy as np
 import pytest
 import torch
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
                                         (256, 2, 17), (257, 2, 100), (512, 1, 60), (513, 1, 60), (1024, 1, 200),
                                         (1025, 1, 1), (2048, 1, 333),
                                         (33, 1025, 7), (130, 411, 20), (200, 300, 50), (300, 205, 31), (600, 108, 40),
-                                        (1025, 63, 9), (2048, 32, 17)])
+                                        (64, 150, 9), (64, 151, 9), (1024, 12, 9), (1024, 13, 9), (1025, 15, 9),
+                                        (1025, 17, 9), (1280, 12, 30), (1281, 12, 30), (2048, 32, 17)])
 @pytest.mark.parametrize("given", [False, True])
 def test_row_selection_widths(dev, NB, heads, K, given):
     from self_trainable_or_free_attn_amd.vsa import _C
