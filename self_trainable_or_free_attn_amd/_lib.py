@@ -161,10 +161,13 @@ def dense_workspace_bytes(Lq, Lk, H):
     workspace smaller than its own rule asks for."""
     if Lq <= 0 or Lk <= 0 or H <= 0:
         return 0
-    items, nb = (Lq + 127) // 128 * H, (Lk + 63) // 64
+    tiles, nb = (Lq + 127) // 128, (Lk + 63) // 64
+    items = tiles * H
     if items > 256 or nb < 8:
         return 0
     ranges = min(512 // items, 16, nb // 4)
     if ranges < 2 or (ranges == 2 and nb < 16):
         return 0
-    return ranges * items * (128 * 128 + 2 * 128) * 4
+    whole = (190 if 8 * H * ((tiles + 7) // 8) > 256 else 124) * nb
+    split = (190 if ranges * items > 256 else 124) * ((nb + ranges - 1) // ranges) + 400 + 9 * ranges * items // 5
+    return ranges * items * (128 * 128 + 2 * 128) * 4 if split < whole else 0

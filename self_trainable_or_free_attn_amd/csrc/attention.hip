@@ -740,16 +740,22 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(AttnArgs a) {
 }
 
 // Key ranges of a dense launch: as many as fill the 512 workgroups the GPU holds, each of at least four key blocks, two
-// ranges only from sixteen blocks on (the partials cost 64 KB a range and the merge a launch of 6 to 10 us); 1 (no
-// split) from 257 items on, where every CU has one. Queries x keys x heads, unsplit -> split: 3925 x 3925 x 1 90 -> 29
-// us, 256 x 33000 x 24 700 -> 164, 1537 x 1537 x 12 48 -> 39, 287 x 808 x 24 31 -> 20, 3329 x 3329 x 5 83 -> 57; in two
-// ranges of four blocks nothing (1280 x 512 x 24 31 -> 32).
+// ranges only from sixteen blocks on, and only where the shorter walk outweighs the partials and the merge; 1: no split.
+// Both sides in 10 ns: a 64-key chunk takes 1.24 us in a workgroup alone on its CU and 1.9 us beside another (an unsplit
+// grid pads the tiles of each head to eight runs, and past 256 places some CUs get two); a merge launch 4 us and each
+// partial, 65 KB written and read, 18 ns. The two sides give the faster form at 195 of 198 measured sizes, the others
+// within 5 %. Queries x keys x heads, unsplit -> split, us: 3925 x 3925 x 1 90 -> 29, 256 x 33000 x 24 700 -> 164, 287 x
+// 808 x 24 31 -> 20, 640 x 1280 x 20 32 -> 30, 2048 x 4096 x 12 90 -> 79; left unsplit: 640 x 705 x 20 23 -> 26, 2048 x
+// 1024 x 12 28 -> 35, 4096 x 1024 x 8 32 -> 41, 32768 x 1024 x 1 27 -> 38, 1280 x 512 x 24 31 -> 32.
 static int dense_splits(int Lq, int Lk, int H) {
-  const long long items = (long long)((Lq + BM - 1) / BM) * H;
-  const int nb = (Lk + BK - 1) / BK;
+  const long long tiles = (Lq + BM - 1) / BM, items = tiles * H, nb = (Lk + BK - 1) / BK;
   if (items > 256 || nb < 8) return 1;
-  const int S = (int)std::min<long long>(std::min<long long>(512 / items, MAX_SPLITS), nb / 4);
-  return S == 2 && nb < 16 ? 1 : std::max(S, 1);
+  const long long S = std::min(std::min<long long>(512 / items, MAX_SPLITS), nb / 4);
+  if (S < 2 || (S == 2 && nb < 16)) return 1;
+  auto walk = [](long long places, long long chunks) { return (places > 256 ? 190 : 124) * chunks; };
+  const long long whole = walk(8 * H * ((tiles + 7) / 8), nb);
+  const long long split = walk(S * items, (nb + S - 1) / S) + 400 + 9 * S * items / 5;
+  return split < whole ? (int)S : 1;
 }
 
 template <int MODE, bool COMP, bool MASS>

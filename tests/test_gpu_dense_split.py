@@ -1,7 +1,8 @@
 """Dense attention over key ranges side by side (few query tiles and heads) against float64, at the edges of its rule,
 each size with the number of ranges it takes: the fewest key blocks that split (12 in three ranges, 16 in two), ranges
-of unequal length, a last block of one key, ragged query tiles, and the item counts around 256 where it stops splitting. Outputs are bf16 (half a step, 2^-8 of the value, and the probabilities' rounding to
-bf16, which averages over the keys): 2e-2 and relative 1e-2 as everywhere."""
+of unequal length, a last block of one key, ragged query tiles, the item counts around 256 where it stops splitting, and
+sizes on both sides of where the merge costs more than it saves. Outputs are bf16 (half a step, 2^-8 of the value, and
+the probabilities' rounding to bf16, which averages over the keys): 2e-2 and relative 1e-2 as everywhere."""
 import math
 
 import pytest
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
                                             (1400, 961, 20, 2), (300, 1537, 3, 6), (1537, 1537, 12, 3),
                                             (256, 33000, 24, 10), (77, 40001, 1, 16), (1280, 700, 24, 1),
                                             (2600, 2600, 12, 2), (2816, 575, 12, 1), (4000, 4001, 8, 2),
-                                            (4100, 1000, 8, 1)])
+                                            (4100, 1000, 8, 1), (640, 705, 20, 1), (640, 1280, 20, 5),
+                                            (2048, 1025, 12, 1), (2048, 4097, 12, 2)])
 def test_split_dense_matches_float64(dev, Lq, Lk, H, ranges):
     from self_trainable_or_free_attn_amd import _lib
     from self_trainable_or_free_attn_amd.kernels import gfx950 as K
