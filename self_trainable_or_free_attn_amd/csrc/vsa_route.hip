@@ -841,11 +841,19 @@ static bool short_strips(int NB, int bh_count) {
   return NB > 1024 && strips > 512 && 8 * strips < 7 * 512 * ((strips + 511) / 512);
 }
 
+// Scores alone have no searches to spread: short strips only while every one of them has a CU to itself. block_scores, us, 8
+// rows / 32 rows, at 64 strips of 32 rows: NB 64 4.0 / 4.4, 480 9.1 / 10.7, 1000 15.8 / 19.0, 2048 28.7 / 35.1; at 75 to
+// 80: NB 64 5.1 / 4.4, 480 13.0 / 10.7; at 255 to 260: NB 300 19.6 / 11.8, 480 29.0 / 11.8, 2048 86 / 43; at 768: NB 2048
+// 198 / 121.
+static bool short_score_strips(int NB, int bh_count) {
+  return (long long)((NB + WIDE_ROWS - 1) / WIDE_ROWS) * bh_count <= 256;
+}
+
 // the search keeps the smallest power of two of chunk registers that holds a row
 template <bool FROM_SCORES>
 static void rows_launch(const RowsArgs& a, int bh_count, hipStream_t stream) {
   const int nchunk = (a.NB + 63) / 64;
-  const bool narrow = short_strips(a.NB, bh_count);
+  const bool narrow = a.K < 0 ? short_score_strips(a.NB, bh_count) : short_strips(a.NB, bh_count);
   if (nchunk <= 2) rows_launch_n<FROM_SCORES, 2>(a, bh_count, narrow, stream);
   else if (nchunk <= 4) rows_launch_n<FROM_SCORES, 4>(a, bh_count, narrow, stream);
   else if (nchunk <= 8) rows_launch_n<FROM_SCORES, 8>(a, bh_count, narrow, stream);

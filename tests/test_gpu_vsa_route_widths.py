@@ -43,3 +43,20 @@ def test_row_selection_widths(dev, NB, heads, K, given):
         assert np.array_equal(qi[base:base + NB * K], np.nonzero(mask)[1])
         assert np.array_equal(kp[0, h], base + np.concatenate([[0], np.cumsum(mask.sum(0))]))
         assert np.array_equal(ki[base:base + NB * K], np.nonzero(mask.T)[1])
+
+
+@pytest.mark.parametrize("NB,heads", [(1, 1), (40, 51), (40, 52), (64, 32), (64, 33), (250, 9), (1000, 2), (1000, 3),
+                                      (2048, 1), (2048, 2), (2049, 1)])
+def test_block_scores_on_both_sides_of_their_strip_rule(dev, NB, heads):
+    """Scores alone: 8 rows per workgroup while a launch has at most 256 workgroups, else 32."""
+    from self_trainable_or_free_attn_amd.vsa import _C
+    print("scores", NB, heads, flush=True)
+    g = torch.Generator().manual_seed(NB + heads)
+    pad = (NB + 63) // 64 * 64
+    qc, kc = (torch.zeros(1, heads, pad, 128) for _ in range(2))
+    for x in (qc, kc):
+        x[:, :, :NB, :16] = torch.randint(-2, 3, (1, heads, NB, 16), generator=g).float()
+    got = _C.block_scores(qc.bfloat16().to(dev), kc.bfloat16().to(dev), NB).float().cpu().numpy()
+    for h in sorted({0, heads // 2, heads - 1}):
+        want = ref.block_scores(qc[:, h:h + 1, :NB].numpy(), kc[:, h:h + 1, :NB].numpy())
+        assert np.array_equal(got[h], np.asarray(want, dtype=np.float32).reshape(NB, NB))
