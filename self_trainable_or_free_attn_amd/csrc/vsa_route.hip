@@ -817,12 +817,12 @@ static int invert(const TopkCarve& c, const ListBase& lists, int* k2q_ptr, int* 
 
 template <bool FROM_SCORES, int NCH>
 static void rows_launch_n(const RowsArgs& a, int bh_count, bool narrow, hipStream_t stream) {
-  const int SR = narrow || NCH == 0 ? WIDE_ROWS : ROWS;
+  const int SR = narrow || FROM_SCORES || NCH == 0 ? WIDE_ROWS : ROWS;
   const size_t lds = (size_t)SR * ((a.NB + 63) & ~63) * 2;  // <= 128 KB
   const dim3 grid((a.NB + SR - 1) / SR, bh_count);
   if (SR == WIDE_ROWS)
     hipLaunchKernelGGL((rows_select_kernel<FROM_SCORES, NCH, WIDE_ROWS>), grid, dim3(256), lds, stream, a);
-  else if constexpr (NCH != 0)
+  else if constexpr (NCH != 0 && !FROM_SCORES)
     hipLaunchKernelGGL((rows_select_kernel<FROM_SCORES, NCH, ROWS>), grid, dim3(256), lds, stream, a);
 }
 
@@ -841,6 +841,9 @@ static bool short_strips(int NB, int bh_count) {
   return NB > 1024 && strips > 512 && 8 * strips < 7 * 512 * ((strips + 511) / 512);
 }
 
+// Given scores have no products to repeat: short strips at every size. row_topk of given scores, us, 8 rows / 32 rows: NB
+// 64: 8 strips of 32 rows 8.2 / 16.0, 1024 21.7 / 24.7, 4096 70 / 70; NB 300: 10 26.5 / 50.6, 1020 66 / 81, 4100 194 /
+// 216; NB 1025: 33 80 / 170, 1023 230 / 379, 4092 792 / 1538; NB 2048: 64 138 / 270, 1024 383 / 943.
 // Scores alone have no searches to spread: short strips only while every one of them has a CU to itself. block_scores, us, 8
 // rows / 32 rows, at 64 strips of 32 rows: NB 64 4.0 / 4.4, 480 9.1 / 10.7, 1000 15.8 / 19.0, 2048 28.7 / 35.1; at 75 to
 // 80: NB 64 5.1 / 4.4, 480 13.0 / 10.7; at 255 to 260: NB 300 19.6 / 11.8, 480 29.0 / 11.8, 2048 86 / 43; at 768: NB 2048

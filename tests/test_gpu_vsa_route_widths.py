@@ -1,6 +1,6 @@
 """The per-row block selection at the edges of its register layouts (2, 4, 8, 16, 32 chunks of 64 columns) and of its
-strip rule (8 or 32 rows per workgroup), bit for bit against the oracle. Pooled rows hold small integers, so every dot
-product is exact, scores tie often and the order of ties is tested too."""
+strip rule (8 or 32 rows per workgroup; 8 with given scores), bit for bit against the oracle. Pooled rows hold small
+integers, so every dot product is exact, scores tie often and the order of ties is tested too."""
 import numpy as np
 import pytest
 import torch
