@@ -21,6 +21,7 @@ BLOCK = 64
 HD = 128                # the widest token row; the three-tier entry points store every row this wide
 VSA_PACKED_ROWS = 0x10000   # flag of the entry points' D: rows are stored D columns wide (include/vsa_hip.h)
 _FWD_VARIANT = [0]
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _check(cond, msg):
@@ -75,30 +76,27 @@ def _dim(D):
     return D if D == HD else D | VSA_PACKED_ROWS
 
 
-def _aligned(x):
-    """x has an address and it is a multiple of 16. A tensor that is being traced or transformed (torch.compile, fake
-    tensors, torch.func wrappers) has none to look at: the graph copies its rows, wherever they will lie."""
-    if torch.compiler.is_compiling() or type(x) not in (torch.Tensor, torch.nn.Parameter):
-        return False
-    try:
-        return x.data_ptr() % 16 == 0
-    except RuntimeError:                  # a torch.func wrapper (their Python type is torch.Tensor)
-        return False
-
-
 def _rows(x, D):
     """x as rows stored D columns wide (None stays None). At D = 64 a tensor in any layout is taken: one that is not
     contiguous or not 16-byte aligned is copied first. A narrower tensor is zero-padded to D columns (the kernels read
-    D of every row), a wider one narrowed."""
+    D of every row), a wider one narrowed. A tensor that is being traced or transformed (torch.compile, fake tensors,
+    torch.func wrappers) has no address to look at: the graph copies its rows, wherever they will lie."""
     if x is None:
         return None
     if D == HD:
         return _wide(x)
-    if x.shape[-1] < D:
-        return F.pad(x, (0, D - x.shape[-1])).contiguous()
-    if x.shape[-1] > D:
+    w = x.shape[-1]
+    if w < D:
+        return F.pad(x, (0, D - w)).contiguous()
+    if w > D:
         x = x[..., :D]
-    return x if x.is_contiguous() and _aligned(x) else x.clone(memory_format=torch.contiguous_format)
+    if type(x) in _PLAIN and not torch.compiler.is_compiling():
+        try:
+            if x.data_ptr() % 16 == 0 and x.is_contiguous():
+                return x
+        except RuntimeError:              # a torch.func wrapper (their Python type is torch.Tensor)
+            pass
+    return x.clone(memory_format=torch.contiguous_format)
 
 
 class _InRows:
