@@ -815,6 +815,9 @@ static int invert(const TopkCarve& c, const ListBase& lists, int* k2q_ptr, int* 
   return ES_OK;
 }
 
+// Given scores have no products to repeat: short strips at every size. row_topk of given scores, us, 8 rows / 32 rows: NB
+// 64: 8 strips of 32 rows 8.2 / 16.0, 1024 21.7 / 24.7, 4096 70 / 70; NB 300: 10 26.5 / 50.6, 1020 66 / 81, 4100 194 /
+// 216; NB 1025: 33 80 / 170, 1023 230 / 379, 4092 792 / 1538; NB 2048: 64 138 / 270, 1024 383 / 943.
 template <bool FROM_SCORES, int NCH>
 static void rows_launch_n(const RowsArgs& a, int bh_count, bool narrow, hipStream_t stream) {
   const int SR = narrow || FROM_SCORES || NCH == 0 ? WIDE_ROWS : ROWS;
@@ -828,22 +831,22 @@ static void rows_launch_n(const RowsArgs& a, int bh_count, bool narrow, hipStrea
 
 // Strips of 8 rows (a wave searches two rows instead of eight, the S tile is computed four times) instead of 32? While
 // there are few strips: what the launch waits for then is a strip's serial searches, with more the repeated products.
-// Past 1024 blocks the keys of 32 rows leave room for two workgroups per CU, and a grid that starts another round of 512
-// without filling it is faster in short strips; past 1280 they leave room for one, and every grid is. route_rows, us, 8
-// rows / 32 rows: NB 64: 4 strips of 32 rows 11.4 / 17.3, 256 19.5 / 17.7, 512 31.6 / 21.0; NB 240: 192 29 / 33, 256 34 /
+// Past 832 blocks the keys of 32 rows leave room for two workgroups per CU, past 1280 for one. With two, a grid that starts
+// another round of 512 without filling it is faster in short strips past 1024 blocks; with one every grid is. route_rows,
+// us, 8 rows / 32 rows: NB 64: 4 strips of 32 rows 11.4 / 17.3, 256 19.5 / 17.7, 512 31.6 / 21.0; NB 240: 192 29 / 33, 256 34 /
 // 33, 384 43 / 38, 1024 81 / 62; NB 420: 294 64 / 66, 378 70 / 68; NB 600: 380 96 / 100, 456 118 / 101; NB 1000: 288 118 /
 // 126, 384 130 / 128, 512 158 / 129; NB 1025: 264 156 / 176, 396 193 / 182, 693 267 / 292, 1023 363 / 325; NB 1200: 380
 // 179 / 191, 1026 387 / 437, 6004 1841 / 1804; NB 1281: 287 180 / 303, 5986 1997 / 3174; NB 1857: 1003 518 / 684.
-static bool short_strips(int NB, int bh_count) {
+// Rows of 64 columns repeat half the products, so their lines lie further out: NB 64: 384 17.3 / 18.1, 512 21.3 / 18.1; NB
+// 240: 384 32.4 / 34.4, 512 39.5 / 34.6; NB 600: 380 79 / 91, 513 98 / 94; NB 1000: 384 104 / 117, 512 127 / 119, 768 162 /
+// 180, 1024 212 / 206; NB 1025: 759 229 / 276, 2046 539 / 566; NB 1200: 494 187 / 183, 1026 317 / 406.
+static bool short_strips(int NB, int ld, int bh_count) {
   const long long strips = (long long)((NB + ROWS - 1) / ROWS) * bh_count;
-  if (NB <= 512) return strips <= 300;
-  if (NB > 1280 || strips <= 384) return true;
-  return NB > 1024 && strips > 512 && 8 * strips < 7 * 512 * ((strips + 511) / 512);
+  const bool half = ld < HD;
+  if (NB > (half ? 1024 : 1280) || strips <= (half ? 400 : NB <= 512 ? 300 : 384)) return true;
+  return NB > (half ? 832 : 1024) && strips > 512 && 8 * strips < 7 * 512 * ((strips + 511) / 512);
 }
 
-// Given scores have no products to repeat: short strips at every size. row_topk of given scores, us, 8 rows / 32 rows: NB
-// 64: 8 strips of 32 rows 8.2 / 16.0, 1024 21.7 / 24.7, 4096 70 / 70; NB 300: 10 26.5 / 50.6, 1020 66 / 81, 4100 194 /
-// 216; NB 1025: 33 80 / 170, 1023 230 / 379, 4092 792 / 1538; NB 2048: 64 138 / 270, 1024 383 / 943.
 // Scores alone have no searches to spread: short strips only while every one of them has a CU to itself. block_scores, us, 8
 // rows / 32 rows, at 64 strips of 32 rows: NB 64 4.0 / 4.4, 480 9.1 / 10.7, 1000 15.8 / 19.0, 2048 28.7 / 35.1; at 75 to
 // 80: NB 64 5.1 / 4.4, 480 13.0 / 10.7; at 255 to 260: NB 300 19.6 / 11.8, 480 29.0 / 11.8, 2048 86 / 43; at 768: NB 2048
@@ -856,7 +859,7 @@ static bool short_score_strips(int NB, int bh_count) {
 template <bool FROM_SCORES>
 static void rows_launch(const RowsArgs& a, int bh_count, hipStream_t stream) {
   const int nchunk = (a.NB + 63) / 64;
-  const bool narrow = a.K < 0 ? short_score_strips(a.NB, bh_count) : short_strips(a.NB, bh_count);
+  const bool narrow = a.K < 0 ? short_score_strips(a.NB, bh_count) : short_strips(a.NB, a.ld, bh_count);
   if (nchunk <= 2) rows_launch_n<FROM_SCORES, 2>(a, bh_count, narrow, stream);
   else if (nchunk <= 4) rows_launch_n<FROM_SCORES, 4>(a, bh_count, narrow, stream);
   else if (nchunk <= 8) rows_launch_n<FROM_SCORES, 8>(a, bh_count, narrow, stream);

@@ -60,3 +60,26 @@ def test_block_scores_on_both_sides_of_their_strip_rule(dev, NB, heads):
     for h in sorted({0, heads // 2, heads - 1}):
         want = ref.block_scores(qc[:, h:h + 1, :NB].numpy(), kc[:, h:h + 1, :NB].numpy())
         assert np.array_equal(got[h], np.asarray(want, dtype=np.float32).reshape(NB, NB))
+
+
+@pytest.mark.parametrize("NB,heads", [(64, 200), (64, 201), (600, 21), (600, 22), (833, 19), (833, 20), (1000, 16),
+                                      (1000, 27), (1000, 28), (1024, 32), (1025, 16)])
+def test_row_selection_of_64_column_rows(dev, NB, heads):
+    """Rows of 64 columns have strip lines of their own."""
+    from self_trainable_or_free_attn_amd.vsa import _C
+    K = 11
+    print("rows of 64 columns", NB, heads, flush=True)
+    g = torch.Generator().manual_seed(NB + 3 * heads)
+    pad = (NB + 63) // 64 * 64
+    qc, kc = (torch.zeros(1, heads, pad, 64) for _ in range(2))
+    for x in (qc, kc):
+        x[:, :, :NB, :16] = torch.randint(-2, 3, (1, heads, NB, 16), generator=g).float()
+    qp, qi, kp, ki = (x.cpu().numpy() for x in _C.route_rows(qc.bfloat16().to(dev), kc.bfloat16().to(dev), NB, K))
+    for h in sorted({0, heads // 2, heads - 1}):
+        s = ref.block_scores(qc[:, h:h + 1, :NB].numpy(), kc[:, h:h + 1, :NB].numpy())
+        mask = ref.row_topk_mask(s, K).reshape(NB, NB)
+        base = h * NB * K
+        assert np.array_equal(qp[0, h], base + np.arange(NB + 1) * K)
+        assert np.array_equal(qi[base:base + NB * K], np.nonzero(mask)[1])
+        assert np.array_equal(kp[0, h], base + np.concatenate([[0], np.cumsum(mask.sum(0))]))
+        assert np.array_equal(ki[base:base + NB * K], np.nonzero(mask.T)[1])
