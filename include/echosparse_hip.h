@@ -3,10 +3,11 @@
  * Every entry point takes caller-owned device pointers (no allocation inside), plain sizes and the HIP stream to
  * enqueue on, never synchronises, and returns an es_status; on failure es_last_error_string() holds a message.
  * es_block_attention, es_sparse_attention, es_dense_attention and es_dense_attention_kv balance their tiles over
- * the XCDs through counters in a ring of 64 slots of device memory, one slot per call of more than 512 tiles (smaller
- * ones use none): any number of such calls may overlap on one GPU (a call waits on its stream for the previous user of its slot). Calls recorded in a stream
- * capture take slots from a second ring of 64 without waiting: graph replays may overlap uncaptured calls, not each
- * other.
+ * the XCDs through counters in a ring of 64 slots of device memory, one slot per call with
+ * 8 * H * ceil(tiles / 8) > 512, tiles = ceil(L / 128) or the number that es_sparse_attention is given (smaller calls,
+ * and es_dense_attention_ws calls that use their workspace, take none): any number of such calls may overlap on one GPU
+ * (a call waits on its stream for the previous user of its slot). Calls recorded in a stream capture take slots from a
+ * second ring of 64 without waiting: graph replays that take slots may overlap uncaptured calls, not each other.
  * Tensor layouts are the reference's (shapes in row-major order):
  *   q, k, v            (L, H, D) bf16, D = 128                       token-major, as echosparse passes them
  *   offset, lse        (nq * 128, H) float32, log2 units, 1e30 for rows >= L

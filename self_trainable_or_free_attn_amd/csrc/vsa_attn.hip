@@ -305,10 +305,11 @@ __device__ __forceinline__ float lse_to_log2(float lse) { return lse == -INFINIT
 // and dS, dK += dS^T Q, with K and V of its keys in registers; 32 matrix instructions per wave and chunk and one
 // barrier. The two query halves' sums are added once at the end. Both accumulator sets and both operand rows need 192 of
 // the 256 registers that two waves per SIMD leave; what else is loop-invariant (LDS and transfer offsets) is therefore
-// rebuilt from one register each by XOR, and lse and delta go to LDS without passing through registers. What bounds it
+// rebuilt from one register each by XOR, and lse and delta go to LDS without passing through registers. (At D = 128 thirteen
+// registers, sixteen in the task form, still spill: 52 bytes of scratch a lane, outside the chunk loop.) What bounds it
 // is each wave's chain of products and exponentials per chunk, as in the forward. Against a dV wave and a dK wave per
 // key half that handed P over through LDS with a second barrier: 4256 -> 3625 us at 480 blocks, 24 heads, top 60
-// (666 -> 800 TFLOP/s), 604 -> 540 at 240 blocks, 12 heads, top 24; at D = 64, 3187 -> 2400.
+// (666 -> 800 TFLOP/s; 3690 to 3730 on other cards), 604 -> 540 at 240 blocks, 12 heads, top 24; at D = 64, 3187 -> 2400.
 template <bool TASKS, int DH>
 __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   constexpr int NKS = DH / 16, NDB = DH / 32;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void vsa_bwd_kv_kernel(VsaBwdArgs a) {
   };
   // LDS offsets of this wave's query half: row reads of k-step ks at aoff ^ 32 ks, transposed reads of channel block
   // db at toff ^ 64 db (exact: the swizzle is an XOR of the 16-byte chunk), so two registers hold what would be
-  // sixteen; the kernel fits its two accumulator sets and both operand rows in 256 registers that way
+  // sixteen; the chunk loop fits its two accumulator sets and both operand rows in 256 registers that way
   int aoff = qh * 8192 + tile_off(lq, hi);
   int toff0, toff1;
   {
